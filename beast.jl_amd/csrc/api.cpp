@@ -282,6 +282,11 @@ extern "C" int bh_mesh_create(bh_ctx *ctx, const double *vertices, int64_t nv, c
         BH_REQUIRE(nn > 0, "cell %lld is degenerate (zero area)", (long long)c);
         g[12] = 0.5 * nn;
         for (int k = 0; k < 3; ++k) g[13 + k] = n[k] / nn;
+        for (int a = 0; a < 3; ++a) {
+            const double d0 = g[3 * a] - g[9], d1 = g[3 * a + 1] - g[10], d2 = g[3 * a + 2] - g[11];
+            m->rho = std::max(m->rho, std::sqrt(d0 * d0 + d1 * d1 + d2 * d2));
+        }
+        m->cmax = std::max(m->cmax, std::sqrt(g[9] * g[9] + g[10] * g[10] + g[11] * g[11]));
     }
     m->d_geo.upload(m->geo.data(), m->geo.size(), ctx->stream);
     BH_CHECK_HIP(hipStreamSynchronize(ctx->stream));

@@ -192,6 +192,34 @@ void pool_alloc(Ctx &ctx, DevBuf<T> &b, size_t count)
     if (count) b.adopt((T *)pool_alloc(ctx, count * sizeof(T)), count);
 }
 
+// A call's workspace from the context's pool.  done() gives it back once the work that uses it
+// is complete; without that (an error on the way) it is freed, which waits for the device.
+template <typename T>
+struct PoolBuf {
+    Ctx *ctx = nullptr;
+    T *p = nullptr;
+    size_t n = 0;
+    PoolBuf() = default;
+    PoolBuf(Ctx &c, size_t count) { alloc(c, count); }
+    PoolBuf(const PoolBuf &) = delete;
+    PoolBuf &operator=(const PoolBuf &) = delete;
+    ~PoolBuf() { if (p) (void)hipFree(p); }
+    void alloc(Ctx &c, size_t count) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        ctx = &c;
+        n = count;
+        if (count) p = (T *)pool_alloc(c, count * sizeof(T));
+    }
+    void upload(const T *h, size_t count, hipStream_t s) {
+        if (count) BH_CHECK_HIP(hipMemcpyAsync(p, h, count * sizeof(T), hipMemcpyHostToDevice, s));
+    }
+    void done() {
+        if (p) pool_free(*ctx, p, n * sizeof(T));
+        p = nullptr;
+    }
+};
+
 // Brackets one launch on ctx.stream when profiling is on.
 struct ProfScope {
     Ctx &ctx;
@@ -242,6 +270,8 @@ struct Mesh {
     std::vector<double> V;      // [nv][3]
     std::vector<int32_t> C;     // [nf][3]
     std::vector<double> geo;    // per cell: vertices[9], centroid[3], area, normal[3]
+    double rho = 0.0;           // largest vertex-to-centroid distance of a cell
+    double cmax = 0.0;          // largest |centroid|
     DevBuf<double> d_geo;       // same on device
     static constexpr int kGeo = 16;
     // quadrature points per triangle-rule degree: [nf][Q][4] (x - centroid, weight)

@@ -158,7 +158,7 @@ def farfield_sample(bj, ctx, X, x, k, nth=181, nph=361):
         ff = bj.potential(op, Y, x, X)
         walls.append(time.perf_counter() - t0)
     kern = {}
-    for name in ("k_ff_current", "k_ff_partial_cells", "k_ff_partial", "k_ff_finish"):
+    for name in ("k_ff_current", "k_ff_cells", "k_ff_partial_cells", "k_ff_partial", "k_ff_finish"):
         n_, s_, w_ = ctx.kernel_stats(name)
         if n_:
             kern[name] = {"launches": n_, "avg_ms": round(1e3 * s_ / n_, 3)}

@@ -57,6 +57,26 @@ def test_farfield_cell_factored_paths(bj, orc, golden, k):
         assert _relmax(got, want) < 1e-12, (k, _relmax(got, want))
 
 
+@pytest.mark.parametrize("rule", [1, 4, 7, 10])
+@pytest.mark.parametrize("gamma", [0.0, 0.4j, -2.5j, 8.0j, 17.0j, 0.05 - 0.2j, 3.0 + 1.0j, -2.0 + 14.0j, 5.0])
+def test_farfield_series_degrees(bj, orc, golden, gamma, rule):
+    """The cells' symmetric series at each of its degrees and beyond them, lossless and lossy,
+    for rules with and without negative weights, on a stretched mesh at a ragged number of
+    directions (single ones too): FP64 end to end, so 1e-12 of the largest component."""
+    m = bj.readmesh(os.path.join(golden, "sphere2.in"))
+    m = bj.Mesh(m.vertices * np.array([1.3, 0.8, 1.0]) + np.array([0.2, -0.1, 0.4]), m.cells)
+    X = bj.raviartthomas(m)
+    rng = np.random.default_rng(rule)
+    u = rng.standard_normal(X.numfunctions()) + 1j * rng.standard_normal(X.numfunctions())
+    for count in (1, 67):
+        Y = rng.standard_normal((count, 3))
+        Y /= np.linalg.norm(Y, axis=1)[:, None]
+        for op in _ops(bj, gamma, 1.0)[:3]:
+            got = bj.potential(op, Y, u, X, quadstrat=bj.SingleNumQStrat(rule))
+            want = orc.farfield(op.kind, gamma, 1.0, Y, u, X, degree=rule)
+            assert _relmax(got, want) < 1e-12, (op, count, _relmax(got, want))
+
+
 def test_farfield_shapes_and_edges(bj, orc, golden):
     """One direction, an empty point set, a grid of points keeps its shape, a zero current
     gives zeros, and two calls give the same bits (fixed-order reduction)."""
