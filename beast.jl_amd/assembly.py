@@ -206,8 +206,10 @@ def assemble(op, X, Y=None, quadstrat=defaultquadstrat, precision="fp64", ctx=No
     prec = {"fp64": nat.FP64, "fp32": nat.FP32}[precision]
     dt = np.complex128 if prec == nat.FP64 else np.complex64
     M, N = X.numfunctions(), Y.numfunctions()
+    terms = list(_terms(op))
+    fresh = out is None and len(terms) > 0   # the first term writes every entry, the others add to it
     if out is None:
-        out = np.zeros((M, N), dtype=dt, order="F")
+        out = (np.empty if fresh else np.zeros)((M, N), dtype=dt, order="F")
         row_offset = col_offset = 0
     if out.dtype != dt or not out.flags.f_contiguous or out.ndim != 2:
         raise ValueError("out must be a 2-d Fortran-ordered array of the assembly precision")
@@ -221,11 +223,12 @@ def assemble(op, X, Y=None, quadstrat=defaultquadstrat, precision="fp64", ctx=No
     lib = nat.load()
     with ctx.lock:
         xh, yh = space_handle(X, ctx), space_handle(Y, ctx)
-        for coef, term in _terms(op):
+        for i, (coef, term) in enumerate(terms):
             qs = resolve_quadstrat(quadstrat, term, X, Y)
             sc = (C.c_double * 2)(complex(coef).real, complex(coef).imag)
             nat.check(lib.bh_assemble(ctx.handle, C.byref(op_struct(term)), C.byref(qs_struct(qs)), prec, xh, yh, sc,
-                                      1, out.ctypes.data_as(C.c_void_p), out.shape[0], row_offset, col_offset))
+                                      0 if fresh and i == 0 else 1, out.ctypes.data_as(C.c_void_p), out.shape[0],
+                                      row_offset, col_offset))
     return out
 
 

@@ -2281,15 +2281,15 @@ extern "C" int bh_assemble(bh_ctx *ctx, const bh_operator *op, const bh_quadstra
                (long long)M, (long long)N);
     const bool fp32 = precision == BH_FP32;
     const size_t es = fp32 ? 8 : 16;
-    DevBuf<char> dZ((size_t)M * N * es);
+    PoolBuf<char> dZ(*ctx, (size_t)M * N * es);
     char *hz = (char *)Z + (size_t)(row_off + col_off * ld) * es;
-    if (accumulate)
-        BH_CHECK_HIP(hipMemcpy2DAsync(dZ.p, M * es, hz, ld * es, M * es, N, hipMemcpyHostToDevice, ctx->stream));
     const double sr = scale ? scale[0] : 1.0, si = scale ? scale[1] : 0.0;
-    assemble_device(*ctx, op, qs, fp32, *const_cast<bh_space *>(X), *const_cast<bh_space *>(Y), dZ.p, M, false,
-                    accumulate != 0, sr, si);
-    BH_CHECK_HIP(hipMemcpy2DAsync(hz, ld * es, dZ.p, M * es, M * es, N, hipMemcpyDeviceToHost, ctx->stream));
-    BH_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+    // the device forms the block alone; what the caller's matrix holds is added to it on the
+    // way into that memory, so it does not travel to the device and back
+    assemble_device(*ctx, op, qs, fp32, *const_cast<bh_space *>(X), *const_cast<bh_space *>(Y), dZ.p, M, false, false,
+                    sr, si);
+    download_block(*ctx, dZ.p, hz, (size_t)ld * es, (size_t)M * es, N, fp32 ? 4 : 8, accumulate != 0);
+    dZ.done();
     BH_API_END
 }
 

@@ -150,6 +150,9 @@ struct Ctx {
     // tournament buffers, the block-column stream), so that repeated
     // factorisations allocate and free nothing
     std::shared_ptr<void> lu_cache;
+    // pinned slots that results leave the device through (download_block), allocated with the
+    // first large result and freed with the context
+    std::shared_ptr<void> host_stage;
     // objects (meshes, matrices) created on this context; destruction of the
     // context is deferred until the last of them is gone
     std::atomic<int> refs{0};
@@ -191,6 +194,11 @@ void pool_alloc(Ctx &ctx, DevBuf<T> &b, size_t count)
     pool_release(ctx, b);
     if (count) b.adopt((T *)pool_alloc(ctx, count * sizeof(T)), count);
 }
+
+// Copies (add = false) or adds (add = true; complex entries of 2 es-byte reals, es 4 or 8) the
+// contiguous columns of `width` bytes at dev to host columns `pitch` bytes apart, after the work
+// queued on the context stream, and waits for it.
+void download_block(Ctx &ctx, const void *dev, void *host, size_t pitch, size_t width, int64_t cols, int es, bool add);
 
 // A call's workspace from the context's pool.  done() gives it back once the work that uses it
 // is complete; without that (an error on the way) it is freed, which waits for the device.
