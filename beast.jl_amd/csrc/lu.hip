@@ -7,10 +7,12 @@
 // (Golub & Van Loan, Matrix Computations, Alg. 3.4.x).
 //
 // FP64 factors (block depth 256) keep LAPACK's pivots exactly:
-//   k_panel         32-column panel as one cooperative kernel: each workgroup keeps
-//                   its rows in LDS; per column one grid barrier exchanges the
-//                   per-workgroup pivot candidates (value, row, row contents).
-//                   Pivot choice is LAPACK's: largest |Re|+|Im|, first row on ties.
+//   k_panel64       32-column panel, one row per thread in registers; per column the
+//                   workgroups exchange pivot candidates through tagged words in
+//                   device memory.  Pivot choice is LAPACK's: largest |Re|+|Im|,
+//                   first row on ties.
+//   k_apply64       the panel's row moves and its block row in the block's other
+//                   columns; 32-row unit-lower solves of the wide block rows.
 // FP32 factors (block depth 1024 while the trailing matrix is large, factored as
 // two 512-column halves, then 512) pivot each 32-column panel by tournament
 // (communication-avoiding LU, Grigori, Demmel & Xiang, SIAM J. Matrix Anal. Appl.
@@ -23,12 +25,12 @@
 //                   update of the block.
 //   k_tslu_apply    moves the planned rows in the block's other columns, solves the
 //                   panel's block row and turns the panel rows into L21 = A21 U11^-1.
+// Shared by both:
 //   The next block column is factored on a second stream while the trailing
 //   update of the current one runs (look-ahead by one block).
-// Shared by both:
 //   k_swap_plan, k_laswp_apply  row interchanges: the sequential swaps replayed
 //                   once on row indices, then each moved row moved once.
-//   k_trsm_unit     32-row unit-lower solve for U12, column in registers.
+//   k_trsm_unit     32-row unit-lower solve for FP32 U12, column in registers.
 //   k_cgemm         C -= A B on MFMA (v_mfma_{f32,f64}_16x16x4): FP64 updates and
 //                   the FP32 updates inside a block column.
 //   k_cgemm_bf16x3  FP32 trailing update from split-bf16 planes (hi*hi + hi*lo +
@@ -39,8 +41,6 @@
 // k_trsv_flag).  FP32 factors precondition flexible GMRES
 // inside iterative refinement in FP64 (GMRES-IR, Carson & Higham, SIAM J. Sci.
 // Comput. 40 (2018)), whose residuals use the resident FP64 matrix.
-#include <hip/hip_cooperative_groups.h>
-
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -82,166 +82,375 @@ __device__ __forceinline__ V csubv(V a, V b)
     return {a.x - b.x, a.y - b.y};
 }
 
-// ---------------------------------------------------------------- grid barrier
-// Two-level barrier by generation.  Workgroup g arrives on the counter of group
-// g % 8 (the XCD it was dispatched to, each counter on its own 128-byte line);
-// the last arrival of a group arrives on the top counter; the last group bumps
-// the generation that everyone waits on.  Counters reset themselves, so the
-// state carries over between launches.  Agent-scope release/acquire makes the
-// data written before the barrier visible to every XCD after it.
-constexpr int kBarStride = 32;   // unsigned words per cache line
-constexpr int kBarWords = kBarStride * 10;
-
-__device__ __forceinline__ void grid_barrier(unsigned *bar, unsigned nblocks, unsigned &gen)
+// Maximum over a wave of unsigned keys (DPP: quad, half-row and row mirrors, then
+// the row broadcasts of lanes 15 and 31), read from lane 63.
+__device__ __forceinline__ unsigned wave_max_u32(unsigned v)
 {
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned ngroups = nblocks < 8 ? nblocks : 8;
-        const unsigned grp = blockIdx.x & 7;
-        const unsigned gsize = (nblocks - grp + 7) / 8;
-        unsigned *gcnt = bar + kBarStride * (1 + grp);
-        unsigned *top = bar + kBarStride * 9;
-        __threadfence();
-        const unsigned a = __hip_atomic_fetch_add(gcnt, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (a == gsize - 1) {
-            __hip_atomic_store(gcnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const unsigned t = __hip_atomic_fetch_add(top, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-            if (t == ngroups - 1) {
-                __hip_atomic_store(top, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_fetch_add(&bar[0], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        while (__hip_atomic_load(&bar[0], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) == gen)
-            __builtin_amdgcn_s_sleep(1);
-        __threadfence();
-    }
-    gen += 1;
-    __syncthreads();
+    int x = (int)v;
+    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
+    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
+    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0x141, 0xF, 0xF, false));  // row_half_mirror
+    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0x140, 0xF, 0xF, false));  // row_mirror
+    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0x142, 0xA, 0xF, false));  // row_bcast:15
+    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0x143, 0xC, 0xF, false));  // row_bcast:31
+    return (unsigned)__builtin_amdgcn_readlane(x, 63);
 }
 
-// (value, row) argmax across a wave: larger value wins, smaller row on ties
-template <typename T>
-__device__ __forceinline__ void wave_argmax(T &v, int &r)
-{
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const T v2 = __shfl_xor(v, off, 64);
-        const int r2 = __shfl_xor(r, off, 64);
-        if (v2 > v || (v2 == v && r2 < r)) { v = v2; r = r2; }
-    }
-}
+// ---------------------------------------------------------------- FP64 panel
+// A 32-column panel with LAPACK's partial pivoting.  Each thread holds one row of the panel
+// in registers for the whole panel; rows do not move, each tracks the position that the
+// interchanges give it and is stored there at the end.  Per column: every wave finds its
+// best row (largest |Re|+|Im|, smallest position on ties) by DPP, puts that row into LDS,
+// and after one barrier the workgroup knows its best.  One workgroup (the last rows) goes on
+// from there.  Several exchange their candidates through slots in device memory: each
+// publishes value, position and row as 64-bit words that carry the column's tag in their
+// low bits, so a word is valid by itself and neither fences nor counters are needed; one
+// wave of each workgroup reads all slots, takes the best and reads that row.  Slots
+// alternate by column parity: a workgroup rewrites one only after every workgroup has
+// published the next column, i.e. has read this one.
+// Bound by latency: per column about one store and two dependent loads across the XCDs, and
+// the rows' way through LDS.  Measured on the MI355X per panel of 32 columns, before (rows in
+// LDS at a stride that put a wave's accesses on one bank, a grid barrier per column) and now:
+// 17,406 rows 398 us alone -> 251 us beside the trailing products; 702 rows, three
+// workgroups, 238 -> 123 us; up to 512 rows, one workgroup, 93 us.
+// The columns run in four phases of eight.  In a phase the live columns shift down by one
+// register per column and the finished multipliers enter at the end, so that the column
+// being eliminated is always the phase's first register (a full unroll does not fit the
+// instruction cache, a dynamic column index would put the row into scratch memory).
+// Finished columns meet zeros in the pivot row.
+constexpr int kPW = 32;            // panel width
+constexpr int kP64Phase = 8;
+constexpr int kP64T = 256;         // rows per workgroup beside the trailing products: the registers of half a CU,
+                                   // as their workgroups, so that neither waits for a whole CU to drain
+constexpr int kP64TOne = 512;      // rows of the panels that one workgroup takes
+constexpr long long kP64WaitTicks = 2000000000LL;   // 20 s of the 100 MHz clock, then the panel reports an error
 
-// ---------------------------------------------------------------- panel
-constexpr int kPW = 32;   // panel width
-
-template <typename T>
-struct PanelWork {
-    T *slot_val;                    // [2][G]
-    int *slot_row;                  // [2][G]
-    typename CT<T>::t *cand;        // [2][G][kPW]
-    typename CT<T>::t *diag;        // [2][kPW]
-    unsigned *bar;                  // [kBarWords]
-    int *info;                      // first zero pivot (1-based), 0 if none
+struct Panel64Slots {
+    int stride;                // slots per parity: that of the largest panel, so that a slot keeps its place
+    unsigned long long *key;   // [2][stride][2]: value bits 63..12 | tag 12; value bits 11..0, position 32, tag 20
+    unsigned long long *row;   // [2][stride][4 kPW]: for each of the row's doubles its high and low half, each | tag 32
+    int *info;                 // first zero pivot (1-based), 0 if none, -1: a wait ran out
+    int *moves;                // [2 kPW]: row that ends at c + i; position where row c + i ends below the panel (-1: none)
 };
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_panel(typename CT<T>::t *A, long long lda, int n, int k0, int pw, int rpb,
-                                               long long *ipiv, PanelWork<T> w)
+__device__ __forceinline__ void put_word(unsigned long long *p, unsigned long long v)
 {
-    using V = typename CT<T>::t;
-    extern __shared__ char smem_raw[];
-    V *L = (V *)smem_raw;   // [rpb][kPW]
-    __shared__ V prow[kPW], drow[kPW];
-    __shared__ T wv_val[4];
-    __shared__ int wv_row[4];
-    const int G = gridDim.x;
-    const int g = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int r0 = k0 + g * rpb;
-    const int r1 = min(n, r0 + rpb);
-    const int nrows = max(0, r1 - r0);
-    for (int idx = tid; idx < nrows * kPW; idx += 256) {
-        const int r = idx / kPW, c = idx % kPW;
-        L[idx] = c < pw ? A[(long long)(r0 + r) * lda + k0 + c] : V{0, 0};
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ unsigned long long get_word(const unsigned long long *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// a candidate: value bits + 1 in (hi, lo) order, hi = 0 for none; smaller position on ties
+struct Cand64 {
+    unsigned hi, lo, pos;
+};
+
+__device__ __forceinline__ bool better(const Cand64 &a, const Cand64 &b)
+{
+    return a.hi != b.hi ? a.hi > b.hi : (a.lo != b.lo ? a.lo > b.lo : a.pos < b.pos);
+}
+
+// lane of the wave's best candidate (any lane if there is none)
+__device__ __forceinline__ int best_lane(const Cand64 &k)
+{
+    const unsigned H = wave_max_u32(k.hi);
+    unsigned long long m = __ballot(k.hi == H);
+    if (m & (m - 1)) {
+        const unsigned L = wave_max_u32(k.hi == H ? k.lo : 0u);
+        m = __ballot(k.hi == H && k.lo == L);
+        if (m & (m - 1)) {
+            const unsigned Q = wave_max_u32(k.hi == H && k.lo == L ? ~k.pos : 0u);
+            m = __ballot(k.hi == H && k.lo == L && ~k.pos == Q);
+        }
     }
-    unsigned gen = __hip_atomic_load(&w.bar[0], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    for (int j = 0; j < pw; ++j) {
-        const int c = k0 + j;
-        const int par = j & 1;
-        // local candidate: largest |Re|+|Im| in column j among rows >= c, first row on ties
-        T best = (T)-1;
-        int brow = INT_MAX;
-        for (int r = tid; r < nrows; r += 256) {
-            const int grw = r0 + r;
-            if (grw < c) continue;
-            const V a = L[r * kPW + j];
-            const T v = fabs(a.x) + fabs(a.y);
-            if (v > best || (v == best && grw < brow)) { best = v; brow = grw; }
-        }
-        wave_argmax(best, brow);
-        if (lane == 0) { wv_val[wid] = best; wv_row[wid] = brow; }
-        __syncthreads();
-        best = wv_val[0];
-        brow = wv_row[0];
+    return __ffsll((long long)m) - 1;
+}
+
+template <int NT>
+struct Panel64Lds {
+    double2 row[2][NT / 64][kPW];     // the waves' best rows
+    Cand64 key[2][NT / 64];
+    double2 u[kPW];                   // the pivot row (several workgroups)
+    int pos;                          // its position
+    double2 buf[NT / 64][64 * 9];     // eight columns of a wave's rows, for whole-line loads and stores
+};
+
+template <int NT, int C0>
+__device__ __forceinline__ void panel64_phase(double2 (&v)[kPW], int &pos, bool &used, bool valid, int k0, int pw,
+                                              long long *ipiv, const Panel64Slots &w, Panel64Lds<NT> &S)
+{
+    constexpr int W = kPW - C0, NW = NT / 64;
+    constexpr bool kMany = NT == kP64T;   // several workgroups
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int G = gridDim.x, g = blockIdx.x;
+#pragma unroll 1
+    for (int t = 0; t < kP64Phase; ++t) {
+        const int j = C0 + t, c = k0 + j, par = j & 1;
+        if (j >= pw) {   // past the last column of a narrow panel: only the shift
+            const double2 v0 = v[C0];
 #pragma unroll
-        for (int q = 1; q < 4; ++q)
-            if (wv_val[q] > best || (wv_val[q] == best && wv_row[q] < brow)) { best = wv_val[q]; brow = wv_row[q]; }
-        if (tid == 0) {
-            w.slot_val[par * G + g] = best;
-            w.slot_row[par * G + g] = brow;
+            for (int q = 1; q < W; ++q) v[C0 + q - 1] = v[C0 + q];
+            v[kPW - 1] = v0;
+            continue;
         }
-        if (brow != INT_MAX && tid < kPW) w.cand[((size_t)par * G + g) * kPW + tid] = L[(brow - r0) * kPW + tid];
-        // wave 0 (lanes 32 .. 63) also writes the diagonal row: the barrier's release fence
-        // is thread 0's and orders only its own wave's stores
-        if (c >= r0 && c < r1 && tid >= 32 && tid < 32 + kPW) w.diag[par * kPW + tid - 32] = L[(c - r0) * kPW + tid - 32];
-        grid_barrier(w.bar, G, gen);
-        // global winner over the G candidates
-        best = (T)-1;
-        brow = INT_MAX;
-        for (int t = tid; t < G; t += 256) {
-            const T v = w.slot_val[par * G + t];
-            const int rw = w.slot_row[par * G + t];
-            if (rw == INT_MAX) continue;
-            if (v > best || (v == best && rw < brow)) { best = v; brow = rw; }
+        Cand64 k{0u, 0u, (unsigned)pos};
+        if (valid && !used) {
+            double mag = fabs(v[C0].x) + fabs(v[C0].y);
+            if (!(mag >= 0.0)) mag = 0.0;   // a NaN ranks last
+            const unsigned long long b = (unsigned long long)__double_as_longlong(mag);
+            k.hi = (unsigned)(b >> 32) + 1u;
+            k.lo = (unsigned)b;
         }
-        wave_argmax(best, brow);
-        if (lane == 0) { wv_val[wid] = best; wv_row[wid] = brow; }
-        __syncthreads();
-        int p = wv_row[0];
-        best = wv_val[0];
+        const int wl = best_lane(k);
+        if (lane == wl) {
+            S.key[par][wid] = k;
 #pragma unroll
-        for (int q = 1; q < 4; ++q)
-            if (wv_val[q] > best || (wv_val[q] == best && wv_row[q] < p)) { best = wv_val[q]; p = wv_row[q]; }
-        // the workgroup owning row p published it
-        const int gp = (p - k0) / rpb;
-        if (tid < kPW) prow[tid] = w.cand[((size_t)par * G + gp) * kPW + tid];
-        else if (tid >= 64 && tid < 64 + kPW) drow[tid - 64] = w.diag[par * kPW + tid - 64];
-        __syncthreads();
-        const V piv = prow[j];
-        if (g == 0 && tid == 0) {
-            ipiv[c] = p;
-            if (piv.x == (T)0 && piv.y == (T)0 && *w.info == 0) *w.info = c + 1;
-        }
-        if (p != c) {
-            if (p >= r0 && p < r1 && tid < kPW) L[(p - r0) * kPW + tid] = drow[tid];
-            if (c >= r0 && c < r1 && tid >= 64 && tid < 64 + kPW) L[(c - r0) * kPW + tid - 64] = prow[tid - 64];
-        }
-        __syncthreads();
-        if (piv.x != (T)0 || piv.y != (T)0) {
-            const T den = piv.x * piv.x + piv.y * piv.y;
-            const V inv{piv.x / den, -piv.y / den};
-            for (int r = tid; r < nrows; r += 256) {
-                if (r0 + r <= c) continue;
-                const V l = cmulv(L[r * kPW + j], inv);
-                L[r * kPW + j] = l;
-                for (int jj = j + 1; jj < pw; ++jj) L[r * kPW + jj] = csubv(L[r * kPW + jj], cmulv(l, prow[jj]));
+            for (int q = 0; q < W; ++q) {
+                double2 x = v[C0 + q];
+                if (q > W - kP64Phase && q >= W - t) x = double2{0.0, 0.0};   // finished columns
+                S.row[par][wid][q] = x;
             }
         }
         __syncthreads();
+        Cand64 best = S.key[par][0];
+        int wb = 0;
+#pragma unroll
+        for (int q = 1; q < NW; ++q) {
+            const Cand64 kq = S.key[par][q];
+            if (better(kq, best)) { best = kq; wb = q; }
+        }
+        const double2 *u = S.row[par][wb];
+        int p = best.hi ? (int)best.pos : c;
+        if constexpr (kMany) {
+            const unsigned tag = (unsigned)c + 1u;
+            if (wid == 0) {   // publish: lane l writes double l of the row
+                if (lane < 2 * W) {
+                    const unsigned long long b = (unsigned long long)__double_as_longlong(((const double *)u)[lane]);
+                    unsigned long long *o = w.row + ((size_t)par * w.stride + g) * 4 * kPW + 2 * lane;
+                    put_word(o, (b & 0xffffffff00000000ull) | tag);
+                    put_word(o + 1, (b << 32) | tag);
+                }
+                if (lane == 0) {
+                    const unsigned long long b = best.hi ? ((unsigned long long)best.hi << 32) | best.lo : 0ull;
+                    unsigned long long *o = w.key + ((size_t)par * w.stride + g) * 2;
+                    put_word(o, (b & ~0xfffull) | (tag & 0xfffu));
+                    put_word(o + 1, (b << 52) | ((unsigned long long)(unsigned)best.pos << 20) | (tag & 0xfffffu));
+                }
+            }
+            if (wid == NW - 1) {
+                Cand64 mine{0u, 0u, 0u};
+                int mg = 0;
+                const long long t0 = wall_clock64();
+                bool late = false;
+                int spins = 0;
+                for (int q0 = 0; q0 < G; q0 += 64) {
+                    const int q = q0 + lane;
+                    const unsigned long long *o = w.key + ((size_t)par * w.stride + min(q, G - 1)) * 2;
+                    unsigned long long a, b;
+                    for (;;) {
+                        a = get_word(o);
+                        b = get_word(o + 1);
+                        const bool ok = (a & 0xfffu) == (tag & 0xfffu) && (b & 0xfffffu) == (tag & 0xfffffu);
+                        if (__all(ok)) break;
+                        // a wait that has run out ends the others too
+                        if ((++spins & 1023) == 0 &&
+                            (wall_clock64() - t0 > kP64WaitTicks ||
+                             __hip_atomic_load(w.info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < 0)) {
+                            late = true;
+                            break;
+                        }
+                    }
+                    const unsigned long long b64 = (a & ~0xfffull) | (b >> 52);
+                    const Cand64 kq{(unsigned)(b64 >> 32), (unsigned)b64, (unsigned)(b >> 20)};
+                    if (q < G && better(kq, mine)) { mine = kq; mg = q; }
+                }
+                const int bl = best_lane(mine);
+                const int gb = __builtin_amdgcn_readlane(mg, bl);
+                const unsigned bhi = (unsigned)__builtin_amdgcn_readlane((int)mine.hi, bl);
+                const int bp = __builtin_amdgcn_readlane((int)mine.pos, bl);
+                const unsigned long long *o = w.row + ((size_t)par * w.stride + gb) * 4 * kPW + 2 * min(lane, 2 * W - 1);
+                unsigned long long a, b;
+                for (;;) {
+                    a = get_word(o);
+                    b = get_word(o + 1);
+                    if (late || __all((unsigned)a == tag && (unsigned)b == tag)) break;
+                    if ((++spins & 1023) == 0 && wall_clock64() - t0 > kP64WaitTicks) late = true;
+                }
+                if (late && lane == 0) __hip_atomic_store(w.info, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (lane < 2 * W)
+                    ((double *)S.u)[lane] = __longlong_as_double((long long)((a & 0xffffffff00000000ull) | (b >> 32)));
+                if (lane == 0) S.pos = bhi ? bp : c;
+            }
+            __syncthreads();
+            u = S.u;
+            p = S.pos;
+        }
+        const double2 piv = u[0];
+        const bool nz = piv.x != 0.0 || piv.y != 0.0;
+        if (g == 0 && tid == 0) {
+            ipiv[c] = p;
+            if (!nz && *w.info == 0) *w.info = c + 1;
+        }
+        if (valid && !used) {
+            if (pos == p) { used = true; pos = c; }
+            else if (pos == c) pos = p;
+        }
+        const double den = piv.x * piv.x + piv.y * piv.y;
+        const double2 inv{piv.x / den, -piv.y / den};
+        const double2 v0 = v[C0];
+        const bool elim = valid && !used && nz;
+        double2 l = cmulv(v0, inv);
+        if (!elim) l = double2{0.0, 0.0};
+#pragma unroll
+        for (int q = 1; q < W; ++q) v[C0 + q - 1] = csubv(v[C0 + q], cmulv(l, u[q]));
+        v[kPW - 1] = elim ? l : v0;
     }
-    for (int idx = tid; idx < nrows * kPW; idx += 256) {
-        const int r = idx / kPW, c = idx % kPW;
-        if (c < pw) A[(long long)(r0 + r) * lda + k0 + c] = L[idx];
+    // the live columns are now first, the finished ones last: put them in order
+    double2 f[kP64Phase];
+#pragma unroll
+    for (int q = 0; q < kP64Phase; ++q) f[q] = v[kPW - kP64Phase + q];
+#pragma unroll
+    for (int q = kPW - 1; q >= C0 + kP64Phase; --q) v[q] = v[q - kP64Phase];
+#pragma unroll
+    for (int q = 0; q < kP64Phase; ++q) v[C0 + q] = f[q];
+}
+
+template <int NT>
+__global__ __launch_bounds__(NT, 2) void k_panel64(double2 *A, long long lda, int n, int k0, int pw, long long *ipiv,
+                                                   Panel64Slots w)
+{
+    __shared__ Panel64Lds<NT> S;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int wave0 = k0 + blockIdx.x * NT + wid * 64;   // the wave's first row
+    const int row = wave0 + lane;
+    const bool valid = row < n;
+    double2 *buf = S.buf[wid];
+    double2 v[kPW];
+    // eight columns (128 bytes) of eight rows per load, turned through the wave's own LDS
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int r = i * 8 + (lane >> 3), col = ch * 8 + (lane & 7);
+            buf[r * 9 + (lane & 7)] = wave0 + r < n && col < pw ? A[(long long)(wave0 + r) * lda + k0 + col] : double2{0.0, 0.0};
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[ch * 8 + q] = buf[lane * 9 + q];
+        __builtin_amdgcn_wave_barrier();
+    }
+    int pos = valid ? row : -1;
+    bool used = false;
+    panel64_phase<NT, 0>(v, pos, used, valid, k0, pw, ipiv, w, S);
+    panel64_phase<NT, 8>(v, pos, used, valid, k0, pw, ipiv, w, S);
+    panel64_phase<NT, 16>(v, pos, used, valid, k0, pw, ipiv, w, S);
+    panel64_phase<NT, 24>(v, pos, used, valid, k0, pw, ipiv, w, S);
+    // every workgroup has read its rows before any gets here: it published columns formed from them
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) buf[lane * 9 + q] = v[ch * 8 + q];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int r = i * 8 + (lane >> 3), col = ch * 8 + (lane & 7);
+            const int to = __shfl(pos, r, 64);
+            const double2 x = buf[r * 9 + (lane & 7)];
+            if (to >= 0 && col < pw) A[(long long)to * lda + k0 + col] = x;
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (valid && pos < k0 + pw) w.moves[pos - k0] = row;
+    if (valid && row < k0 + pw) w.moves[kPW + row - k0] = pos >= k0 + pw ? pos : -1;
+}
+
+// Columns beside an FP64 panel [c, c + pw), 16 per workgroup out of [a0, a1) and [b0, b1):
+// the panel's row moves (moves; NULL: none), and in the columns of [b0, b1) the panel's
+// block row, B := L^-1 B on the rows c .. c + pw with L the unit lower triangle at (c, lc).
+// Four columns to a wave, 16 lanes to a column, each with two rows: the solved entry goes
+// to the column's lanes by a row broadcast.  (One thread per column took 23 us: a chain of
+// 528 complex multiplications; 224 columns take 7 us this way.)
+template <int K>
+__device__ __forceinline__ double row_bcast(double x)   // lane K of each 16
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x150 + K, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x150 + K, 0xF, 0xF, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+template <int I>
+__device__ __forceinline__ void unit_solve_step(double2 &x0, double2 &x1, const double2 (*L)[kPW + 1], int r)
+{
+    if constexpr (I < kPW - 1) {
+        const double2 xs = I < 16 ? x0 : x1;
+        const double2 xi{row_bcast<I & 15>(xs.x), row_bcast<I & 15>(xs.y)};
+        if constexpr (I < 15) {
+            const double2 u = csubv(x0, cmulv(L[r][I], xi));
+            if (r > I) x0 = u;
+        }
+        const double2 u = csubv(x1, cmulv(L[r + 16][I], xi));
+        if (r + 16 > I) x1 = u;
+        unit_solve_step<I + 1>(x0, x1, L, r);
+    }
+}
+
+__global__ __launch_bounds__(256) void k_apply64(double2 *A, long long lda, int c, int lc, int pw, const int *moves,
+                                                 int a0, int a1, int b0, int b1)
+{
+    __shared__ double2 s_buf[2 * kPW][17];
+    __shared__ double2 L[kPW][kPW + 1];
+    __shared__ int s_src[2 * kPW], s_dst[2 * kPW];
+    const int tid = threadIdx.x;
+    const bool solve = (int)blockIdx.x * 16 + 16 > a1 - a0;   // some of its columns are right of the panel
+    if (tid < 2 * kPW) {
+        const int i = tid & (kPW - 1);
+        int src = -1, dst = -1;
+        if (i < pw) {
+            if (tid < kPW) { src = moves ? moves[i] : c + i; dst = c + i; }
+            else if (moves) { src = c + i; dst = moves[kPW + i]; }
+        }
+        s_src[tid] = src;
+        s_dst[tid] = dst;
+    }
+    if (solve)
+        for (int e = tid; e < kPW * kPW; e += 256) {
+            const int i = e / kPW, q = e % kPW;
+            L[i][q] = i < pw && q < pw ? A[(long long)(c + i) * lda + lc + q] : double2{0.0, 0.0};
+        }
+    __syncthreads();
+    const int w1 = a1 - a0;
+    {
+        const int cl = tid & 15, t = blockIdx.x * 16 + cl;
+        const int col = t < w1 ? a0 + t : (t < w1 + (b1 - b0) ? b0 + (t - w1) : -1);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int e = (tid >> 4) + 16 * k;
+            s_buf[e][cl] = col >= 0 && s_dst[e] >= 0 ? A[(long long)s_src[e] * lda + col] : double2{0.0, 0.0};
+        }
+    }
+    __syncthreads();
+    if (solve) {
+        const int cl = tid >> 4, r = tid & 15;
+        double2 x0 = s_buf[r][cl], x1 = s_buf[r + 16][cl];
+        unit_solve_step<0>(x0, x1, L, r);
+        if ((int)blockIdx.x * 16 + cl >= w1) {
+            s_buf[r][cl] = x0;
+            s_buf[r + 16][cl] = x1;
+        }
+        __syncthreads();
+    }
+    {
+        const int cl = tid & 15, t = blockIdx.x * 16 + cl;
+        const int col = t < w1 ? a0 + t : (t < w1 + (b1 - b0) ? b0 + (t - w1) : -1);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int e = (tid >> 4) + 16 * k;
+            if (col >= 0 && s_dst[e] >= 0 && (t >= w1 || s_src[e] != s_dst[e])) A[(long long)s_dst[e] * lda + col] = s_buf[e][cl];
+        }
     }
 }
 
@@ -262,20 +471,6 @@ __global__ __launch_bounds__(256) void k_panel(typename CT<T>::t *A, long long l
 constexpr int kTsluT = 256;             // rows (threads) per tournament workgroup
 constexpr int kTsluFan = kTsluT / kPW;  // candidate sets merged per workgroup
 constexpr int kPlanMax = 2 * kPW;       // row moves of one panel
-
-// Maximum over a wave of unsigned keys (DPP: quad, half-row and row mirrors, then
-// the row broadcasts of lanes 15 and 31), read from lane 63.
-__device__ __forceinline__ unsigned wave_max_u32(unsigned v)
-{
-    int x = (int)v;
-    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, false));   // quad_perm 1,0,3,2
-    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0x4E, 0xF, 0xF, false));   // quad_perm 2,3,0,1
-    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0x141, 0xF, 0xF, false));  // row_half_mirror
-    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0x140, 0xF, 0xF, false));  // row_mirror
-    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0x142, 0xA, 0xF, false));  // row_bcast:15
-    x = (int)max((unsigned)x, (unsigned)__builtin_amdgcn_update_dpp(x, x, 0x143, 0xC, 0xF, false));  // row_bcast:31
-    return (unsigned)__builtin_amdgcn_readlane(x, 63);
-}
 
 // Partial pivoting over up to kTsluT rows held in registers, one row per thread
 // (v: the row's first kPW entries; rows with used set never pivot).  piv[j]
@@ -758,6 +953,7 @@ constexpr int kMaxSwaps = 256;
 // block-column chain.  Smaller trailing matrices take 512-deep blocks.
 constexpr int kNBFP32 = 1024, kNBFP32Small = 512, kNBDeepAbove = 24576;
 constexpr int kNBInner = 512;
+constexpr int kNBFP64 = 256;            // FP64 block depth
 constexpr int kAheadFirstBelow = 20480;   // trailing width below which the next block column goes first
 
 // The 1024-deep block columns join their 512-column halves with split-bf16 products,
@@ -2169,13 +2365,9 @@ void check(const char *what)
 
 template <typename T>
 struct LUWork {
-    DevBuf<T> slot_val;
-    DevBuf<int> slot_row;
-    DevBuf<typename CT<T>::t> cand, diag;
-    DevBuf<unsigned> bar;
+    DevBuf<unsigned long long> slots;      // FP64 panels: the workgroups' candidates
+    DevBuf<int> moves;                     // FP64 panels: row moves of the last one
     DevBuf<int> info;
-    int maxG = 0;
-    int rpb_max = 0;
     DevBuf<int> plan;                      // row-interchange plan (k_swap_plan)
     DevBuf<int> tcnt;                      // tournament group counters (zero between panels)
     DevBuf<int> tidx;                      // tournament candidate sets (row ids), all levels
@@ -2246,32 +2438,49 @@ template <typename T>
 void trsm_unit(hipStream_t s, typename CT<T>::t *A, long long lda, int lr, int m, int br, int bc, int ncols)
 {
     if (ncols <= 0 || m <= 0) return;
-    k_trsm_unit<T><<<(ncols + 63) / 64, 64, 0, s>>>(A, lda, lr, lr, m, br, bc, ncols);
-    check("k_trsm_unit");
+    if constexpr (sizeof(T) == 8) {
+        BH_REQUIRE(lr == br, "block row %d solved with the triangle at row %d", br, lr);
+        k_apply64<<<(ncols + 15) / 16, 256, 0, s>>>(A, lda, br, lr, m, nullptr, bc, bc, bc, bc + ncols);
+        check("k_apply64");
+    } else {
+        k_trsm_unit<T><<<(ncols + 63) / 64, 64, 0, s>>>(A, lda, lr, lr, m, br, bc, ncols);
+        check("k_trsm_unit");
+    }
 }
 
-template <typename T>
-void panel(Ctx &ctx, LUWork<T> &W, typename CT<T>::t *A, long long lda, int n, int k0, int pw, long long *ipiv)
+// FP64 panel [c, c + pw) of the block column [k, k + kb): the panel, then the row moves and the
+// panel's block row in the block's other columns, then the update of the columns to its right.
+void panel64(Ctx &ctx, hipStream_t s, LUWork<double> &W, double2 *A, long long lda, int n, int k, int kb, int c, int pw,
+             long long *ipiv)
 {
-    const int rows = n - k0;
-    int G = (rows + W.rpb_max - 1) / W.rpb_max;
-    G = std::max(1, std::min(G, W.maxG));
-    const int rpb = (rows + G - 1) / G;
-    BH_REQUIRE(rpb <= W.rpb_max, "panel: %d rows per workgroup exceed %d", rpb, W.rpb_max);
-    PanelWork<T> pw_{W.slot_val.p, W.slot_row.p, W.cand.p, W.diag.p, W.bar.p, W.info.p};
-    const size_t shm = (size_t)rpb * kPW * sizeof(typename CT<T>::t);
-    void *args[] = {&A, (void *)&lda, (void *)&n, (void *)&k0, (void *)&pw, (void *)&rpb, &ipiv, &pw_};
-    ProfScope prof(ctx, "k_panel", (double)rows * pw * sizeof(typename CT<T>::t) * 2);
-    // A grid barrier needs all its workgroups resident at once.  Two cooperative
-    // panels on different streams could each hold part of the device and wait
-    // for the rest, so with several live contexts the panels run one at a time.
-    if (live_contexts() > 1) {
-        std::lock_guard<std::mutex> lock(coop_mutex());
-        BH_CHECK_HIP(hipLaunchCooperativeKernel((const void *)k_panel<T>, dim3(G), dim3(256), args, shm, ctx.stream));
-        BH_CHECK_HIP(hipStreamSynchronize(ctx.stream));
-    } else {
-        BH_CHECK_HIP(hipLaunchCooperativeKernel((const void *)k_panel<T>, dim3(G), dim3(256), args, shm, ctx.stream));
+    const int rows = n - c;
+    const int G = rows <= kP64TOne ? 1 : (rows + kP64T - 1) / kP64T;
+    const int stride = (n + kP64T - 1) / kP64T;
+    const Panel64Slots sl{stride, W.slots.p, W.slots.p + (size_t)4 * stride, W.info.p, W.moves.p};
+    {
+        ProfScope prof(ctx, "k_panel", (double)rows * pw * sizeof(double2) * 2, s);
+        if (G == 1) {
+            k_panel64<kP64TOne><<<1, kP64TOne, 0, s>>>(A, lda, n, c, pw, ipiv, sl);
+        } else if (live_contexts() > 1) {
+            // The workgroups wait for one another, so all must be resident at once.  One panel's are
+            // (checked in lu_factor), but panels of several contexts could each hold part of the
+            // device and wait for the rest: with several live contexts they run one at a time.
+            std::lock_guard<std::mutex> lock(coop_mutex());
+            k_panel64<kP64T><<<G, kP64T, 0, s>>>(A, lda, n, c, pw, ipiv, sl);
+            check("k_panel64");
+            BH_CHECK_HIP(hipStreamSynchronize(s));
+        } else {
+            k_panel64<kP64T><<<G, kP64T, 0, s>>>(A, lda, n, c, pw, ipiv, sl);
+        }
+        check("k_panel64");
     }
+    const int cols = (c - k) + (k + kb - (c + pw));
+    if (cols > 0) {
+        k_apply64<<<(cols + 15) / 16, 256, 0, s>>>(A, lda, c, c, pw, W.moves.p, k, c, c + pw, k + kb);
+        check("k_apply64");
+    }
+    if (c + pw < k + kb)
+        gemm<double>(ctx, s, A, lda, c + pw, c, c, c + pw, c + pw, c + pw, n - (c + pw), k + kb - (c + pw), pw);
 }
 
 // Panel of columns [c, c + pw) of the block column [k, k + kb) by tournament
@@ -2369,12 +2578,7 @@ void factor_block(Ctx &ctx, hipStream_t s, LUWork<T> &W, typename CT<T>::t *A, l
             // launch this panel's block row
             tslu_panel(ctx, s, W, A, lda, n, k, kb, c, pw, ipiv, sp > 0);
         } else {
-            panel<T>(ctx, W, A, lda, n, c, pw, ipiv);
-            laswp<T>(ctx, s, A, lda, c, c + pw, ipiv, k, c, c + pw, k + kb, W.plan.p);
-            if (c + pw < k + kb) {
-                trsm_unit<T>(s, A, lda, c, pw, c, c + pw, k + kb - (c + pw));
-                gemm<T>(ctx, s, A, lda, c + pw, c, c, c + pw, c + pw, c + pw, n - (c + pw), k + kb - (c + pw), pw);
-            }
+            panel64(ctx, s, W, A, lda, n, k, kb, c, pw, ipiv);
         }
     }
 }
@@ -2465,12 +2669,12 @@ void block_row_u12(Ctx &ctx, hipStream_t s, LUWork<T> &W, typename CT<T>::t *A, 
     }
 }
 
-// Right-looking blocked LU (block columns of NB = 256, panels of 32).  FP64
-// (LAPACK's partial pivoting) runs on the context stream.  FP32 (tournament
-// pivoting) looks one block ahead: after block k's U12 is formed, the next
-// block column is updated first and factored on a second stream while the rest
-// of the trailing matrix is updated on the context stream; the two touch
-// disjoint columns.
+// Right-looking blocked LU (panels of 32 columns; FP64: LAPACK's partial pivoting, FP32:
+// tournament pivoting), looking one block ahead: after block k's U12 is formed, the next
+// block column is updated first and factored on a second stream while the rest of the
+// trailing matrix is updated on the context stream; the two touch disjoint columns.  (FP64,
+// 17,406 rows: 578 ms for the whole solve with every step on one stream and the former
+// panel, 346 ms now.)
 void invert_diagonal_blocks(hipStream_t s, const float2 *LU, long long lda, int n, float2 *Dinv);
 
 template <typename T>
@@ -2479,10 +2683,11 @@ struct LUBuffers {
     DevBuf<__bf16> PA, PB;   // split planes of the trailing updates
 };
 
-// The FP32 factorisation's workspace and block-column stream, kept in the context.
+// The factorisations' workspaces and their block-column stream, kept in the context.
 struct LUCache {
     std::mutex mu;
     LUBuffers<float> b;
+    LUBuffers<double> b64;
     hipStream_t s2 = nullptr;
     hipEvent_t ready = nullptr, done = nullptr;
     ~LUCache() {
@@ -2508,48 +2713,29 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
                bool split = false, float2 *dinv = nullptr)
 {
     hipStream_t s = ctx.stream;
-    // FP32: the context's cached workspace unless another factorisation holds it
-    LUCache *cache = nullptr;
-    std::unique_lock<std::mutex> held;
+    // the context's cached workspace unless another factorisation holds it
+    LUCache *cache = &lu_cache(ctx);
+    std::unique_lock<std::mutex> held(cache->mu, std::try_to_lock);
     std::unique_ptr<LUBuffers<T>> own;
     LUBuffers<T> *buf = nullptr;
-    if constexpr (sizeof(T) == 4) {
-        cache = &lu_cache(ctx);
-        held = std::unique_lock<std::mutex>(cache->mu, std::try_to_lock);
-        if (held.owns_lock()) {
-            buf = &cache->b;
-            if (cache->s2) BH_CHECK_HIP(hipStreamSynchronize(cache->s2));   // after a failed call
-        } else {
-            cache = nullptr;
-        }
-    }
-    if (!buf) {
+    if (held.owns_lock()) {
+        if constexpr (sizeof(T) == 4) buf = &cache->b;
+        else buf = &cache->b64;
+        if (cache->s2) BH_CHECK_HIP(hipStreamSynchronize(cache->s2));   // after a failed call
+    } else {
+        cache = nullptr;
         own = std::make_unique<LUBuffers<T>>();
         buf = own.get();
     }
     LUWork<T> &W = buf->W;
     DevBuf<__bf16> &PA = buf->PA, &PB = buf->PB;
     W.eblk_of = W.eblk_side_of = -1;
-    // rows per workgroup kept in LDS: 64 KiB of panel slice
-    W.rpb_max = (int)(65536 / (kPW * sizeof(typename CT<T>::t)));
-    int per_cu = 0;
-    BH_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_panel<T>, 256,
-                                                              (size_t)W.rpb_max * kPW * sizeof(typename CT<T>::t)));
-    BH_REQUIRE(per_cu >= 1, "panel kernel cannot be resident");
-    W.maxG = per_cu * ctx.num_cus;
-    W.slot_val.ensure(2 * (size_t)W.maxG);
-    W.slot_row.ensure(2 * (size_t)W.maxG);
-    W.cand.ensure(2 * (size_t)W.maxG * kPW);
-    W.diag.ensure(2 * kPW);
-    W.bar.ensure(kBarWords);
     W.info.ensure(1);
     W.plan.ensure(4 * kMaxSwaps);
-    W.plan_side.ensure(4 * kMaxSwaps);
-    BH_CHECK_HIP(hipMemsetAsync(W.bar.p, 0, kBarWords * sizeof(unsigned), s));
     BH_CHECK_HIP(hipMemsetAsync(W.info.p, 0, sizeof(int), s));
     // block column of the right-looking LU (trailing-update depth); the FP32
     // path's deeper blocks halve the C traffic per flop of the trailing update
-    const int NB = sizeof(T) == 4 ? kNBFP32 : 256;   // deepest block (workspace sizes)
+    auto depth = [&](int k) { return sizeof(T) == 4 ? fp32_block_depth(n, k, split) : kNBFP64; };
     int planes_of = -1;   // block whose L21 planes PA holds
     auto trailing = [&](hipStream_t st, int k, int kb, int c0, int c1) {
         // A[k+kb:, c0:c1) -= L21 U12[:, c0:c1)
@@ -2565,15 +2751,15 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
         gemm<T>(ctx, st, A, lda, k + kb, k, k, c0, k + kb, c0, n - (k + kb), c1 - c0, kb);
     };
     if constexpr (sizeof(T) == 8) {
-        for (int k = 0; k < n; k += NB) {
-            const int kb = std::min(NB, n - k);
-            factor_block<T>(ctx, s, W, A, lda, n, k, kb, ipiv);
-            laswp<T>(ctx, s, A, lda, k, k + kb, ipiv, 0, k, k + kb, n, W.plan.p);
-            if (k + kb < n) {
-                block_row_u12<T>(ctx, s, W, A, lda, n, k, kb, k + kb, n);
-                trailing(s, k, kb, k + kb, n);
-            }
-        }
+        // panels exchange tagged words: cleared, so that no tag of an earlier factorisation is there
+        const int G = (n + kP64T - 1) / kP64T;
+        int per_cu = 0;
+        BH_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_panel64<kP64T>, kP64T, 0));
+        BH_REQUIRE(G <= per_cu * ctx.num_cus, "panel of %d rows: its workgroups cannot all be resident", n);
+        const size_t words = (size_t)G * (4 + 8 * kPW);
+        W.slots.ensure(words);
+        W.moves.ensure(2 * kPW);
+        BH_CHECK_HIP(hipMemsetAsync(W.slots.p, 0, words * sizeof(unsigned long long), s));
     } else {
         // FP32 factors only precondition GMRES-IR: their panels use tournament pivoting
         // candidate sets of all levels: n_0 + n_1 + ... < 2 n_0 + levels
@@ -2582,11 +2768,14 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
         W.tidx.ensure(sets * kPW);
         W.tval.ensure(sets * kPW * kPW);
         BH_CHECK_HIP(hipMemsetAsync(W.tcnt.p, 0, sets * sizeof(int), s));
+        W.plan_side.ensure(4 * kMaxSwaps);
         W.top.ensure((size_t)kPW * kPW);
         W.oldtop.ensure((size_t)kPW * kPW);
         W.tplan.ensure(1 + 2 * kPlanMax);
         W.eblk.ensure((size_t)(kNBInnerMax / kIB) * kIB * kIB);
         W.eblk_side.ensure((size_t)(kNBInnerMax / kIB) * kIB * kIB);
+    }
+    {
         hipStream_t s2 = nullptr;
         hipEvent_t ready = nullptr, done = nullptr;
         struct Cleanup {   // a stream and events of this call only (no cache)
@@ -2612,7 +2801,7 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
             BH_CHECK_HIP(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
             BH_CHECK_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
         }
-        factor_block<T>(ctx, s, W, A, lda, n, 0, std::min(fp32_block_depth(n, 0, split), n), ipiv);
+        factor_block<T>(ctx, s, W, A, lda, n, 0, std::min(depth(0), n), ipiv);
         // block k is factored; its interchanges reach the other columns (in pieces
         // of at most kMaxSwaps interchanges, applied in order) over [c0, c1) and [c2, c3)
         auto swaps = [&](int k, int kb, int c0, int c1, int c2, int c3) {
@@ -2620,17 +2809,17 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
                 laswp<T>(ctx, s, A, lda, q, std::min(q + kMaxSwaps, k + kb), ipiv, c0, c1, c2, c3, W.plan.p);
         };
         for (int k = 0, kb = 0; k < n; k += kb) {
-            kb = std::min(fp32_block_depth(n, k, split), n - k);
+            kb = std::min(depth(k), n - k);
             if (k + kb >= n) {
                 swaps(k, kb, 0, k, 0, 0);
                 break;
             }
-            const int nk = k + kb, nkb = std::min(fp32_block_depth(n, nk, split), n - nk);
+            const int nk = k + kb, nkb = std::min(depth(nk), n - nk);
             // near the end the block-column chain is the critical path: there the
             // next block column goes first on its own (interchanges, block row,
             // update) and the rest is brought up to date while it is factored;
             // earlier, one pass over all columns costs the context stream less
-            const bool ahead_first = n - nk <= kAheadFirstBelow;
+            const bool ahead_first = sizeof(T) == 8 || n - nk <= kAheadFirstBelow;
             if (ahead_first) {
                 swaps(k, kb, nk, nk + nkb, 0, 0);
                 block_row_u12<T>(ctx, s, W, A, lda, n, k, kb, nk, nk + nkb, split ? &PB : nullptr);
@@ -2662,6 +2851,7 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
     }
     BH_CHECK_HIP(hipMemcpyAsync(info_host, W.info.p, sizeof(int), hipMemcpyDeviceToHost, s));
     BH_CHECK_HIP(hipStreamSynchronize(s));
+    if (*info_host < 0) BH_FAIL(BH_ERR_HIP, "LU panel: a workgroup waited in vain for the others' pivot candidates");
 }
 
 // forward (unit lower) then backward (upper) substitution on X (n x nrhs, work precision)
@@ -3242,9 +3432,11 @@ extern "C" int bh_matrix_factor(bh_matrix *M, int precision)
         const unsigned cgrid = (unsigned)(((long long)n * n + 255) / 256);
         k_to_work<double><<<cgrid, 256, 0, ctx.stream>>>((const double2 *)M->a64.p, (int)n, (double2 *)M->lu64.p, lda);
         check("k_to_work");
+        M->factored = -1;
         lu_factor<double>(ctx, (double2 *)M->lu64.p, lda, (int)n, M->ipiv.p, &info);
     } else {
         fp32_prepare(ctx, M, lda);
+        M->factored = -1;
         lu_factor<float>(ctx, (float2 *)M->lu32.p, lda, (int)n, M->ipiv.p, &info, precision == BH_FP32_SPLIT,
                          (float2 *)M->dinv32.p);
     }
