@@ -17,14 +17,15 @@
 // two 512-column halves, then 512) pivot each 32-column panel by tournament
 // (communication-avoiding LU, Grigori, Demmel & Xiang, SIAM J. Matrix Anal. Appl.
 // 32 (2011)):
-//   k_tslu_panel    one launch per panel: 256 rows per workgroup, one per thread
+//   k_tslu_panel    one launch per panel: 512 rows per workgroup, two per thread
 //                   in registers, reduced to 32 candidates by partial pivoting;
-//                   the last workgroup of each group of 8 to finish merges the
-//                   group one level up, and the last merge emits L11\U11, ipiv and
-//                   a row plan.  Further workgroups carry the previous panel's
-//                   update of the block.
-//   k_tslu_apply    moves the planned rows in the block's other columns, solves the
-//                   panel's block row and turns the panel rows into L21 = A21 U11^-1.
+//                   the last workgroup of each group to finish merges the group one
+//                   level up, and the last merge emits L11\U11, ipiv and the row
+//                   moves.  Further workgroups carry the previous panel's update of
+//                   the block.
+//   k_tslu_apply    moves the rows in the block's other columns, solves the panel's
+//                   block row, turns the panel rows into L21 = A21 U11^-1 and brings
+//                   the next panel up to date.
 // Shared by both:
 //   The next block column is factored on a second stream while the trailing
 //   update of the current one runs (look-ahead by one block).
@@ -80,6 +81,22 @@ template <typename V>
 __device__ __forceinline__ V csubv(V a, V b)
 {
     return {a.x - b.x, a.y - b.y};
+}
+
+// a b and a - b c with the contraction written out: the same bits wherever they are inlined
+__device__ __forceinline__ float2 cmul_x(float2 a, float2 b)
+{
+    return {fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x)};
+}
+
+__device__ __forceinline__ float2 cfms_x(float2 a, float2 b, float2 c)
+{
+    return {fmaf(b.y, c.y, fmaf(-b.x, c.x, a.x)), fmaf(-b.y, c.x, fmaf(-b.x, c.y, a.y))};
+}
+
+__device__ __forceinline__ double2 cfms_x(double2 a, double2 b, double2 c)
+{
+    return {fma(b.y, c.y, fma(-b.x, c.x, a.x)), fma(-b.y, c.x, fma(-b.x, c.y, a.y))};
 }
 
 // Maximum over a wave of unsigned keys (DPP: quad, half-row and row mirrors, then
@@ -175,7 +192,6 @@ struct Panel64Lds {
     Cand64 key[2][NT / 64];
     double2 u[kPW];                   // the pivot row (several workgroups)
     int pos;                          // its position
-    double2 buf[NT / 64][64 * 9];     // eight columns of a wave's rows, for whole-line loads and stores
 };
 
 template <int NT, int C0>
@@ -323,24 +339,17 @@ __global__ __launch_bounds__(NT, 2) void k_panel64(double2 *A, long long lda, in
                                                    Panel64Slots w)
 {
     __shared__ Panel64Lds<NT> S;
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int wave0 = k0 + blockIdx.x * NT + wid * 64;   // the wave's first row
-    const int row = wave0 + lane;
+    const int row = k0 + blockIdx.x * NT + threadIdx.x;
     const bool valid = row < n;
-    double2 *buf = S.buf[wid];
     double2 v[kPW];
-    // eight columns (128 bytes) of eight rows per load, turned through the wave's own LDS
+    // each thread its own row, as it lies (turning whole-line loads through LDS is slower)
 #pragma unroll
-    for (int ch = 0; ch < 4; ++ch) {
+    for (int q = 0; q < kPW; ++q) v[q] = double2{0.0, 0.0};
+    if (valid) {
+        const double2 *src = A + (long long)row * lda + k0;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int r = i * 8 + (lane >> 3), col = ch * 8 + (lane & 7);
-            buf[r * 9 + (lane & 7)] = wave0 + r < n && col < pw ? A[(long long)(wave0 + r) * lda + k0 + col] : double2{0.0, 0.0};
-        }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int q = 0; q < 8; ++q) v[ch * 8 + q] = buf[lane * 9 + q];
-        __builtin_amdgcn_wave_barrier();
+        for (int q = 0; q < kPW; ++q)
+            if (q < pw) v[q] = src[q];
     }
     int pos = valid ? row : -1;
     bool used = false;
@@ -349,32 +358,31 @@ __global__ __launch_bounds__(NT, 2) void k_panel64(double2 *A, long long lda, in
     panel64_phase<NT, 16>(v, pos, used, valid, k0, pw, ipiv, w, S);
     panel64_phase<NT, 24>(v, pos, used, valid, k0, pw, ipiv, w, S);
     // every workgroup has read its rows before any gets here: it published columns formed from them
+    if (valid) {
+        double2 *dst = A + (long long)pos * lda + k0;
 #pragma unroll
-    for (int ch = 0; ch < 4; ++ch) {
-#pragma unroll
-        for (int q = 0; q < 8; ++q) buf[lane * 9 + q] = v[ch * 8 + q];
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int r = i * 8 + (lane >> 3), col = ch * 8 + (lane & 7);
-            const int to = __shfl(pos, r, 64);
-            const double2 x = buf[r * 9 + (lane & 7)];
-            if (to >= 0 && col < pw) A[(long long)to * lda + k0 + col] = x;
-        }
-        __builtin_amdgcn_wave_barrier();
+        for (int q = 0; q < kPW; ++q)
+            if (q < pw) dst[q] = v[q];
     }
     if (valid && pos < k0 + pw) w.moves[pos - k0] = row;
     if (valid && row < k0 + pw) w.moves[kPW + row - k0] = pos >= k0 + pw ? pos : -1;
 }
 
-// Columns beside an FP64 panel [c, c + pw), 16 per workgroup out of [a0, a1) and [b0, b1):
-// the panel's row moves (moves; NULL: none), and in the columns of [b0, b1) the panel's
-// block row, B := L^-1 B on the rows c .. c + pw with L the unit lower triangle at (c, lc).
+// Columns beside a panel [c, c + pw), 16 per workgroup out of [a0, a1) and [b0, b1): the
+// panel's row moves (moves: row that goes to c + i; position where row c + i goes below the
+// panel, -1: none; NULL: no moves), and in the columns of [b0, b1) the panel's block row,
+// B := L^-1 B on the rows c .. c + pw with L the unit lower triangle of Lp (stride ldl).
 // Four columns to a wave, 16 lanes to a column, each with two rows: the solved entry goes
-// to the column's lanes by a row broadcast.  (One thread per column took 23 us: a chain of
-// 528 complex multiplications; 224 columns take 7 us this way.)
+// to the column's lanes by a row broadcast.  (One thread per column took 23 us in FP64, a
+// chain of 528 complex multiplications; 224 columns take 7 us this way.)
 template <int K>
-__device__ __forceinline__ double row_bcast(double x)   // lane K of each 16
+__device__ __forceinline__ float row_bcast(float x)   // lane K of each 16
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + K, 0xF, 0xF, true));
+}
+
+template <int K>
+__device__ __forceinline__ double row_bcast(double x)
 {
     const long long b = __double_as_longlong(x);
     const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x150 + K, 0xF, 0xF, true);
@@ -382,30 +390,33 @@ __device__ __forceinline__ double row_bcast(double x)   // lane K of each 16
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-template <int I>
-__device__ __forceinline__ void unit_solve_step(double2 &x0, double2 &x1, const double2 (*L)[kPW + 1], int r)
+template <int I, typename V>
+__device__ __forceinline__ void unit_solve_step(V &x0, V &x1, const V (*L)[kPW + 1], int r)
 {
     if constexpr (I < kPW - 1) {
-        const double2 xs = I < 16 ? x0 : x1;
-        const double2 xi{row_bcast<I & 15>(xs.x), row_bcast<I & 15>(xs.y)};
+        const V xs = I < 16 ? x0 : x1;
+        const V xi{row_bcast<I & 15>(xs.x), row_bcast<I & 15>(xs.y)};
         if constexpr (I < 15) {
-            const double2 u = csubv(x0, cmulv(L[r][I], xi));
+            const V u = cfms_x(x0, L[r][I], xi);
             if (r > I) x0 = u;
         }
-        const double2 u = csubv(x1, cmulv(L[r + 16][I], xi));
+        const V u = cfms_x(x1, L[r + 16][I], xi);
         if (r + 16 > I) x1 = u;
         unit_solve_step<I + 1>(x0, x1, L, r);
     }
 }
 
-__global__ __launch_bounds__(256) void k_apply64(double2 *A, long long lda, int c, int lc, int pw, const int *moves,
-                                                 int a0, int a1, int b0, int b1)
+template <typename T>
+__device__ __forceinline__ void apply_strip(typename CT<T>::t *A, long long lda, int c, const typename CT<T>::t *Lp,
+                                            long long ldl, int pw, const int *moves, int a0, int a1, int b0, int b1,
+                                            int bid)
 {
-    __shared__ double2 s_buf[2 * kPW][17];
-    __shared__ double2 L[kPW][kPW + 1];
+    using V = typename CT<T>::t;
+    __shared__ V s_buf[2 * kPW][17];
+    __shared__ V L[kPW][kPW + 1];
     __shared__ int s_src[2 * kPW], s_dst[2 * kPW];
-    const int tid = threadIdx.x;
-    const bool solve = (int)blockIdx.x * 16 + 16 > a1 - a0;   // some of its columns are right of the panel
+    const int tid = threadIdx.x, w1 = a1 - a0;
+    const bool solve = bid * 16 + 16 > w1 && b1 > b0;   // some of its columns are right of the panel
     if (tid < 2 * kPW) {
         const int i = tid & (kPW - 1);
         int src = -1, dst = -1;
@@ -419,39 +430,38 @@ __global__ __launch_bounds__(256) void k_apply64(double2 *A, long long lda, int 
     if (solve)
         for (int e = tid; e < kPW * kPW; e += 256) {
             const int i = e / kPW, q = e % kPW;
-            L[i][q] = i < pw && q < pw ? A[(long long)(c + i) * lda + lc + q] : double2{0.0, 0.0};
+            L[i][q] = i < pw && q < pw ? Lp[i * ldl + q] : V{0, 0};
         }
     __syncthreads();
-    const int w1 = a1 - a0;
-    {
-        const int cl = tid & 15, t = blockIdx.x * 16 + cl;
-        const int col = t < w1 ? a0 + t : (t < w1 + (b1 - b0) ? b0 + (t - w1) : -1);
+    const int cl = tid & 15, t = bid * 16 + cl;
+    const int col = t < w1 ? a0 + t : (t < w1 + (b1 - b0) ? b0 + (t - w1) : -1);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int e = (tid >> 4) + 16 * k;
-            s_buf[e][cl] = col >= 0 && s_dst[e] >= 0 ? A[(long long)s_src[e] * lda + col] : double2{0.0, 0.0};
-        }
+    for (int k = 0; k < 4; ++k) {
+        const int e = (tid >> 4) + 16 * k;
+        s_buf[e][cl] = col >= 0 && s_dst[e] >= 0 ? A[(long long)s_src[e] * lda + col] : V{0, 0};
     }
     __syncthreads();
     if (solve) {
-        const int cl = tid >> 4, r = tid & 15;
-        double2 x0 = s_buf[r][cl], x1 = s_buf[r + 16][cl];
+        const int sc = tid >> 4, r = tid & 15;
+        V x0 = s_buf[r][sc], x1 = s_buf[r + 16][sc];
         unit_solve_step<0>(x0, x1, L, r);
-        if ((int)blockIdx.x * 16 + cl >= w1) {
-            s_buf[r][cl] = x0;
-            s_buf[r + 16][cl] = x1;
+        if (bid * 16 + sc >= w1) {
+            s_buf[r][sc] = x0;
+            s_buf[r + 16][sc] = x1;
         }
         __syncthreads();
     }
-    {
-        const int cl = tid & 15, t = blockIdx.x * 16 + cl;
-        const int col = t < w1 ? a0 + t : (t < w1 + (b1 - b0) ? b0 + (t - w1) : -1);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int e = (tid >> 4) + 16 * k;
-            if (col >= 0 && s_dst[e] >= 0 && (t >= w1 || s_src[e] != s_dst[e])) A[(long long)s_dst[e] * lda + col] = s_buf[e][cl];
-        }
+    for (int k = 0; k < 4; ++k) {
+        const int e = (tid >> 4) + 16 * k;
+        if (col >= 0 && s_dst[e] >= 0 && (t >= w1 || s_src[e] != s_dst[e])) A[(long long)s_dst[e] * lda + col] = s_buf[e][cl];
     }
+}
+
+__global__ __launch_bounds__(256) void k_apply64(double2 *A, long long lda, int c, int lc, int pw, const int *moves,
+                                                 int a0, int a1, int b0, int b1)
+{
+    apply_strip<double>(A, lda, c, A + (long long)c * lda + lc, lda, pw, moves, a0, a1, b0, b1, blockIdx.x);
 }
 
 // ---------------------------------------------------------------- tournament pivoting
@@ -459,177 +469,230 @@ __global__ __launch_bounds__(256) void k_apply64(double2 *A, long long lda, int 
 // Grigori, Demmel & Xiang, SIAM J. Matrix Anal. Appl. 32 (2011)), used by the
 // FP32 factorisations that GMRES-IR refines.  Partial pivoting needs one
 // grid-wide exchange per column; here the pw <= 32 pivot rows of a panel are chosen
-//   1. per workgroup of kTsluT rows: partial pivoting selects <= pw candidates,
-//   2. by a reduction tree: a workgroup stacks kTsluFan candidate sets (their
+//   1. per workgroup of kTsluRows rows: partial pivoting selects <= pw candidates,
+//   2. by a reduction tree: a workgroup stacks up to kTsluFan candidate sets (their
 //      rows as they entered the panel) and keeps the rows partial pivoting selects,
 // until one set remains.  Partial pivoting on the final stack picks its
 // pivots among the winners in order, and eliminating with winners only leaves
 // the winners' rows exactly as partial pivoting on the winners alone would
 // (no loser is ever a pivot row), so the final workgroup also emits
-// L11 \ U11, LAPACK-style sequential interchanges and a row-move plan.
-// k_tslu_apply then moves the rows and forms L21 = A21 U11^-1.
-constexpr int kTsluT = 256;             // rows (threads) per tournament workgroup
-constexpr int kTsluFan = kTsluT / kPW;  // candidate sets merged per workgroup
-constexpr int kPlanMax = 2 * kPW;       // row moves of one panel
+// L11 \ U11, LAPACK-style sequential interchanges and the row moves.
+// The panel's entries lie in an array of their own, P[n][kPW], which the launches of a panel
+// only read: a set is therefore its row numbers alone, whoever merges it takes the rows
+// from P, and nothing but those numbers and a counter passes between workgroups.
+// k_tslu_apply then moves the rows, forms L21 = P U11^-1 and writes the next panel's P.
+// Bound by latency, the chain of 32 columns per level.  Two rows per thread halve the
+// levels (512 rows to a set: two levels up to 8192 rows, three up to 131,072) for half as
+// many more instructions per column.  Measured on the MI355X per 32-column panel, before
+// (256 rows a workgroup, the previous panel's update in front of it) -> now: tournament
+// 107 -> 75 us at 4050 unknowns, 122 -> 87 us at 9003; apply 27 -> 14 and 27 -> 17 us.
+constexpr int kTsluT = 256;                   // threads of a tournament workgroup
+constexpr int kTsluRows = 2 * kTsluT;         // its rows
+constexpr int kTsluFan = kTsluRows / kPW;     // candidate sets merged per workgroup at most
 
-// Partial pivoting over up to kTsluT rows held in registers, one row per thread
-// (v: the row's first kPW entries; rows with used set never pivot).  piv[j]
-// (LDS) receives the thread whose row pivots column j (-1 if none is left).
-// Pivot choice: largest |Re|+|Im| at 2^-12 relative resolution (key = value bits
-// with the low 11 mantissa bits replaced by 2047 - thread), smaller thread on
-// ties.  One barrier per column: each wave finds its best key by DPP and that
-// lane stores its row in the wave's slot (slots and keys alternate between two
-// buffers by column parity), so after the barrier every thread reads the
-// winning wave's row and eliminates with it in registers.  The pivot rows keep
-// their factored entries (L left of the diagonal, U from it).  The columns run
-// in eight phases of four: phase P updates the columns [4P, kPW), those of the
-// phase under a predicate (a full unroll of the 32 x 32 elimination does not fit
-// the instruction cache).  The elimination has no branch (rows that take no part
-// subtract a zero multiple of the pivot row), and the next column's key and its
-// DPP reduction follow its own update, so they overlap the other columns' updates.
-// The slots must hold finite values before the first column (a column without a
-// pivot reads wave 0's slot).
-__device__ __forceinline__ unsigned pivot_key(float2 x, bool used, int tid)
+// rows per workgroup of k_tslu_apply
+__host__ __device__ inline int tslu_apply_row_count(int rows) { return rows <= 8192 ? 32 : 64; }
+
+// Groups that nl sets are merged in, as even as they get: the fewest levels, and among
+// those groups of at most kTsluFan / 2 sets, whose rows take one register row per thread
+// (21 us against 28 us for 32 columns).
+__host__ __device__ inline int tslu_groups(int nl)
 {
-    const float mag = fabsf(x.x) + fabsf(x.y);
-    return used ? 0u : ((__float_as_uint(mag) & ~2047u) | (unsigned)(2047 - tid));
+    const int most = nl <= kTsluFan ? kTsluFan : (nl <= kTsluFan * kTsluFan / 2 ? kTsluFan / 2 : kTsluFan);
+    return (nl + most - 1) / most;
 }
-
-template <int P>
-__device__ __forceinline__ void gepp_phase(float2 (&v)[kPW], bool &used, int pw, int *piv, unsigned (*s_key)[4],
-                                           float2 (*s_row)[4][kPW], unsigned &key, unsigned &wmax)
+__host__ __device__ inline int tslu_fan(int nl) { return (nl + tslu_groups(nl) - 1) / tslu_groups(nl); }
+// candidate sets of all levels, for n rows
+inline size_t tslu_sets(int n)
 {
-    constexpr int C0 = 4 * P, NW = kTsluT / 64;
-    static_assert(NW <= 4, "one key slot per wave");
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const int jend = min(C0 + 4, pw);
-#pragma unroll 1
-    for (int j = C0; j < jend; ++j) {
-        const int par = j & 1;
-        // key and wmax hold column j's key of this row and the wave's best
-        if (key == wmax && wmax != 0u) {
-#pragma unroll
-            for (int cc = C0; cc < kPW; ++cc) s_row[par][wid][cc] = v[cc];
-        }
-        if (lane == 0) s_key[par][wid] = wmax;
-        __syncthreads();
-        unsigned kmax = s_key[par][0];
-        int wbest = 0;
-#pragma unroll
-        for (int q = 1; q < NW; ++q) {
-            const unsigned kq = s_key[par][q];
-            wbest = kq > kmax ? q : wbest;
-            kmax = kq > kmax ? kq : kmax;
-        }
-        const int p = kmax ? 2047 - (int)(kmax & 2047u) : -1;
-        if (tid == 0) piv[j] = p;
-        if (tid == p) used = true;
-        float2 pr[kPW];   // the pivot row, read in one batch
-#pragma unroll
-        for (int cc = C0; cc < kPW; ++cc) pr[cc] = s_row[par][wbest][cc];
-        float2 d = pr[C0], vj = v[C0];
-        // column j of this row and of the pivot row (selects per component: a
-        // conditional struct copy makes the compiler move v to scratch memory)
-#pragma unroll
-        for (int q = 1; q < 4; ++q) {
-            d.x = (j == C0 + q) ? pr[C0 + q].x : d.x;
-            d.y = (j == C0 + q) ? pr[C0 + q].y : d.y;
-            vj.x = (j == C0 + q) ? v[C0 + q].x : vj.x;
-            vj.y = (j == C0 + q) ? v[C0 + q].y : vj.y;
-        }
-        const float den = fmaf(d.x, d.x, d.y * d.y);
-        const bool elim = !used && p >= 0 && den != 0.f;
-        // multiplier vj / d through the hardware reciprocal of |d|^2 (zero for rows
-        // that take no part)
-        const float rden = elim ? __builtin_amdgcn_rcpf(den) : 0.f;
-        const float2 l{fmaf(vj.x, d.x, vj.y * d.y) * rden, fmaf(vj.y, d.x, -vj.x * d.y) * rden};
-#pragma unroll
-        for (int cc = C0; cc < kPW; ++cc) {
-            const float ux = fmaf(l.y, pr[cc].y, fmaf(-l.x, pr[cc].x, v[cc].x));
-            const float uy = fmaf(-l.y, pr[cc].x, fmaf(-l.x, pr[cc].y, v[cc].y));
-            if (cc < C0 + 4) {
-                v[cc].x = cc == j ? (elim ? l.x : v[cc].x) : (cc > j ? ux : v[cc].x);
-                v[cc].y = cc == j ? (elim ? l.y : v[cc].y) : (cc > j ? uy : v[cc].y);
-            } else {
-                v[cc].x = ux;
-                v[cc].y = uy;
-            }
-        }
-        // the next column's key
-        if (j + 1 < pw) {
-            float2 vn = v[C0 + 1];
-#pragma unroll
-            for (int q = 2; q <= 4; ++q) {
-                if (C0 + q < kPW) {
-                    vn.x = (j + 1 == C0 + q) ? v[C0 + q].x : vn.x;
-                    vn.y = (j + 1 == C0 + q) ? v[C0 + q].y : vn.y;
-                }
-            }
-            key = pivot_key(vn, used, tid);
-            wmax = wave_max_u32(key);
-        }
+    size_t t = 0;
+    for (int nl = (n + kTsluRows - 1) / kTsluRows;; nl = tslu_groups(nl)) {
+        t += nl;
+        if (nl <= 1) return t;
     }
 }
 
-__device__ __forceinline__ void block_gepp(float2 (&v)[kPW], bool used, int pw, int *piv, unsigned (*s_key)[4],
-                                           float2 (*s_row)[4][kPW])
+// Partial pivoting over R kTsluT rows held in registers, R = 1 or 2 per thread (v: the rows'
+// kPW entries; rows with used set never pivot; slot: a row's number in the workgroup).
+// piv[j] (LDS) receives the slot whose row pivots column j (-1 if none is left), j_of[h]
+// the column that a row pivots.
+// Pivot choice: largest |Re|+|Im| at 2^-13 relative resolution (key = value bits with the
+// low 10 mantissa bits replaced by 1023 - slot), smaller slot on ties.  Two barriers per
+// column: after the first every wave knows the others' best keys (found by DPP), and the
+// winning lane stores its row; after the second every wave reads that row, one entry per
+// lane, and takes its entries from there into scalar registers, with which it eliminates.
+// (One barrier, with every wave's best row stored before it, costs 620 cycles of LDS
+// writes per column; a broadcast read of the row by every wave would fill the LDS pipe.)
+// The next column's own update, key and reduction go first, and the rest of the update
+// runs between the next barrier and the use of the keys read behind it.  In each of four
+// phases of eight columns the live columns shift down by one register per column and the
+// multipliers enter at the end, so that the column in hand is always the phase's first
+// register; finished columns meet zeros in the pivot row.  The elimination has no branch
+// (rows that take no part subtract a zero multiple).
+struct __align__(16) GeppLds {
+    unsigned key[2][4];
+    float2 row[2][kPW];
+    int piv[kPW];
+    int zero;   // first column whose pivot is exactly zero (INT_MAX: none)
+};
+
+__device__ __forceinline__ unsigned pivot_key(float2 x, bool used, int slot)
 {
-    unsigned key = pivot_key(v[0], used, threadIdx.x);
-    unsigned wmax = wave_max_u32(key);
-    gepp_phase<0>(v, used, pw, piv, s_key, s_row, key, wmax);
-    gepp_phase<1>(v, used, pw, piv, s_key, s_row, key, wmax);
-    gepp_phase<2>(v, used, pw, piv, s_key, s_row, key, wmax);
-    gepp_phase<3>(v, used, pw, piv, s_key, s_row, key, wmax);
-    gepp_phase<4>(v, used, pw, piv, s_key, s_row, key, wmax);
-    gepp_phase<5>(v, used, pw, piv, s_key, s_row, key, wmax);
-    gepp_phase<6>(v, used, pw, piv, s_key, s_row, key, wmax);
-    gepp_phase<7>(v, used, pw, piv, s_key, s_row, key, wmax);
+    const float mag = fabsf(x.x) + fabsf(x.y);
+    return used ? 0u : ((__float_as_uint(mag) & ~1023u) | (unsigned)(1023 - slot));
+}
+
+__device__ __forceinline__ float lane_f(float v, int l)
+{
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// the waves' best keys of one column, and the best of this thread's rows
+template <int R>
+__device__ __forceinline__ void gepp_keys(const float2 (&v)[2][kPW], int c, const bool (&used)[2], const int (&slot)[2],
+                                          int par, GeppLds &S, unsigned (&key)[2])
+{
+    unsigned kb = 0;
+#pragma unroll
+    for (int h = 0; h < R; ++h) {
+        key[h] = pivot_key(v[h][c], used[h], slot[h]);
+        kb = max(kb, key[h]);
+    }
+    const unsigned wmax = wave_max_u32(kb);
+    if ((threadIdx.x & 63) == 0) S.key[par][threadIdx.x >> 6] = wmax;
+}
+
+template <int R, int C0>
+__device__ __forceinline__ void gepp_phase(float2 (&v)[2][kPW], bool (&used)[2], const int (&slot)[2], int (&j_of)[2],
+                                           int pw, GeppLds &S, unsigned (&key)[2], unsigned &kmax)
+{
+    constexpr int W = kPW - C0, kPhase = 8;
+    static_assert(kTsluT / 64 == 4, "one key per wave");
+    const int tid = threadIdx.x, lane = tid & 63;
+#pragma unroll 1
+    for (int t = 0; t < kPhase; ++t) {
+        const int j = C0 + t, par = j & 1;
+        if (j >= pw) {   // past the last column of a narrow panel: only the shift
+#pragma unroll
+            for (int h = 0; h < R; ++h) {
+                const float2 v0 = v[h][C0];
+#pragma unroll
+                for (int q = 1; q < W; ++q) v[h][C0 + q - 1] = v[h][C0 + q];
+                v[h][kPW - 1] = v0;
+            }
+            continue;
+        }
+        // kmax: column j's best key; key: those of this thread's rows
+        const int p = kmax ? 1023 - (int)(kmax & 1023u) : -1;
+#pragma unroll
+        for (int h = 0; h < R; ++h)
+            if (key[h] == kmax && kmax != 0u) {
+#pragma unroll
+                for (int q = 0; q < W; ++q) S.row[par][q] = v[h][C0 + q];
+            }
+        __syncthreads();
+        float2 pl = S.row[par][min(lane, W - 1)];        // the pivot row, entry q in lane q
+        if (p < 0 || lane >= W - t) pl = float2{0, 0};   // no pivot, finished columns
+        const float2 d{lane_f(pl.x, 0), lane_f(pl.y, 0)};
+        if (tid == 0) {
+            S.piv[j] = p;
+            if (d.x == 0.f && d.y == 0.f) S.zero = min(S.zero, j);
+        }
+        const float den = fmaf(d.x, d.x, d.y * d.y);
+        const float rd = den != 0.f ? __builtin_amdgcn_rcpf(den) : 0.f;
+        float2 l[R], last[R];
+        const float ux1 = lane_f(pl.x, 1), uy1 = lane_f(pl.y, 1);
+#pragma unroll
+        for (int h = 0; h < R; ++h) {
+            if (slot[h] == p) {
+                used[h] = true;
+                j_of[h] = j;
+            }
+            const float2 v0 = v[h][C0];
+            const bool elim = !used[h] && den != 0.f;
+            // multiplier v0 / d through the hardware reciprocal of |d|^2 (zero for rows
+            // that take no part)
+            const float rden = elim ? rd : 0.f;
+            l[h] = float2{fmaf(v0.x, d.x, v0.y * d.y) * rden, fmaf(v0.y, d.x, -v0.x * d.y) * rden};
+            last[h] = float2{elim ? l[h].x : v0.x, elim ? l[h].y : v0.y};
+            v[h][C0] = float2{fmaf(l[h].y, uy1, fmaf(-l[h].x, ux1, v[h][C0 + 1].x)),
+                              fmaf(-l[h].y, ux1, fmaf(-l[h].x, uy1, v[h][C0 + 1].y))};
+        }
+        // the next column's keys (after the last column nothing reads them)
+        gepp_keys<R>(v, C0, used, slot, par ^ 1, S, key);
+        __syncthreads();
+        const uint4 kq = *(const uint4 *)S.key[par ^ 1];
+#pragma unroll
+        for (int q = 2; q < W; ++q) {
+            const float ux = lane_f(pl.x, q), uy = lane_f(pl.y, q);
+#pragma unroll
+            for (int h = 0; h < R; ++h)
+                v[h][C0 + q - 1] = float2{fmaf(l[h].y, uy, fmaf(-l[h].x, ux, v[h][C0 + q].x)),
+                                          fmaf(-l[h].y, ux, fmaf(-l[h].x, uy, v[h][C0 + q].y))};
+        }
+#pragma unroll
+        for (int h = 0; h < R; ++h) v[h][kPW - 1] = last[h];
+        kmax = max(max(kq.x, kq.y), max(kq.z, kq.w));
+    }
+    // the live columns are now first, the finished ones last: put them in order
+#pragma unroll
+    for (int h = 0; h < R; ++h) {
+        float2 f[kPhase];
+#pragma unroll
+        for (int q = 0; q < kPhase; ++q) f[q] = v[h][kPW - kPhase + q];
+#pragma unroll
+        for (int q = kPW - 1; q >= C0 + kPhase; --q) v[h][q] = v[h][q - kPhase];
+#pragma unroll
+        for (int q = 0; q < kPhase; ++q) v[h][C0 + q] = f[q];
+    }
+}
+
+template <int R>
+__device__ __forceinline__ void block_gepp(float2 (&v)[2][kPW], bool (&used)[2], const int (&slot)[2], int (&j_of)[2],
+                                           int pw, GeppLds &S)
+{
+    unsigned key[2];
+    j_of[0] = j_of[1] = -1;
+    if (threadIdx.x == 0) S.zero = INT_MAX;
+    gepp_keys<R>(v, 0, used, slot, 0, S, key);
+    __syncthreads();
+    const uint4 kq = *(const uint4 *)S.key[0];
+    unsigned kmax = max(max(kq.x, kq.y), max(kq.z, kq.w));
+    gepp_phase<R, 0>(v, used, slot, j_of, pw, S, key, kmax);
+    gepp_phase<R, 8>(v, used, slot, j_of, pw, S, key, kmax);
+    gepp_phase<R, 16>(v, used, slot, j_of, pw, S, key, kmax);
+    gepp_phase<R, 24>(v, used, slot, j_of, pw, S, key, kmax);
     __syncthreads();
 }
 
-// x := x U^-1 for one row x (registers) and U upper triangular (LDS), column by
-// column, in four phases of eight; row i of U is read in one batch.
-template <int P>
-__device__ __forceinline__ void right_trsv_phase(float2 (&x)[kPW], int pw, const float2 (*U)[kPW + 1])
+// x := x U^-1 for one row x on the 16 lanes of a row group, lane r with the entries r and
+// r + 16, U upper triangular (LDS); i0, i1: the reciprocals of U's diagonal entries r, r + 16.
+template <int I>
+__device__ __forceinline__ void right_solve_step(float2 &x0, float2 &x1, const float2 (*U)[kPW + 1], int r, float2 i0,
+                                                 float2 i1)
 {
-    constexpr int C0 = 8 * P;
-    const int iend = min(C0 + 8, pw);
-#pragma unroll 1
-    for (int i = C0; i < iend; ++i) {
-        float2 ur[kPW];
-#pragma unroll
-        for (int cc = C0; cc < kPW; ++cc) ur[cc] = U[i][cc];
-        float2 xi = x[C0], d = ur[C0];
-#pragma unroll
-        for (int q = 1; q < 8; ++q) {
-            xi.x = (i == C0 + q) ? x[C0 + q].x : xi.x;
-            xi.y = (i == C0 + q) ? x[C0 + q].y : xi.y;
-            d.x = (i == C0 + q) ? ur[C0 + q].x : d.x;
-            d.y = (i == C0 + q) ? ur[C0 + q].y : d.y;
+    if constexpr (I < kPW) {
+        const float2 y = I < 16 ? cmul_x(x0, i0) : cmul_x(x1, i1);
+        const float2 xi{row_bcast<I & 15>(y.x), row_bcast<I & 15>(y.y)};
+        if constexpr (I < 16) {
+            const float2 u = cfms_x(x0, xi, U[I][r]);
+            x0.x = r > I ? u.x : (r == I ? y.x : x0.x);
+            x0.y = r > I ? u.y : (r == I ? y.y : x0.y);
+            x1 = cfms_x(x1, xi, U[I][r + 16]);
+        } else {
+            const float2 u = cfms_x(x1, xi, U[I][r + 16]);
+            x1.x = r + 16 > I ? u.x : (r + 16 == I ? y.x : x1.x);
+            x1.y = r + 16 > I ? u.y : (r + 16 == I ? y.y : x1.y);
         }
-        const float den = fmaf(d.x, d.x, d.y * d.y);
-        const float rden = den != 0.f ? __builtin_amdgcn_rcpf(den) : 0.f;
-        xi = float2{fmaf(xi.x, d.x, xi.y * d.y) * rden, fmaf(xi.y, d.x, -xi.x * d.y) * rden};
-#pragma unroll
-        for (int cc = C0; cc < kPW; ++cc) {
-            const float ux = fmaf(xi.y, ur[cc].y, fmaf(-xi.x, ur[cc].x, x[cc].x));
-            const float uy = fmaf(-xi.y, ur[cc].x, fmaf(-xi.x, ur[cc].y, x[cc].y));
-            if (cc < C0 + 8) {
-                x[cc].x = cc == i ? xi.x : (cc > i ? ux : x[cc].x);
-                x[cc].y = cc == i ? xi.y : (cc > i ? uy : x[cc].y);
-            } else {
-                x[cc].x = ux;
-                x[cc].y = uy;
-            }
-        }
+        right_solve_step<I + 1>(x0, x1, U, r, i0, i1);
     }
 }
 
+// What the tournament leaves: sequential interchanges, the factored winners, the row moves.
 struct TsluFinal {
     long long *ipiv;   // rows c .. c+pw receive the sequential interchanges
     float2 *top;       // [kPW][kPW] L11 \ U11, row j = the row that goes to c + j
-    float2 *oldtop;    // [kPW][kPW] panel entries of rows c .. c+pw before the interchanges
-    int *plan;         // [0] = m, then m destinations, then m sources (rows before the moves)
+    int *moves;        // [2 kPW]: row that goes to c + i; position where row c + i goes below the panel (-1: none)
     int *info;         // first zero pivot (1-based), 0 if none
 };
 
@@ -639,301 +702,302 @@ __device__ __forceinline__ void cgemm_tile(int id, const typename CT<T>::t *__re
                                            typename CT<T>::t *Cp, long long ldc, int M, int N, int K);
 
 // Counters and candidate sets of the tournament.  Level l holds n_l sets
-// (n_0 = workgroups of the first stage, n_{l+1} = ceil(n_l / kTsluFan)); its sets
-// start at set offset n_0 + ... + n_{l-1} and its group counters at
-// ceil(n_0 / kTsluFan) + ... + ceil(n_{l-1} / kTsluFan).
+// (n_0 = workgroups of the first stage, n_{l+1} = tslu_groups(n_l)); its sets start at set
+// n_0 + ... + n_{l-1} and its group counters at n_1 + ... + n_l.
 struct TsluWork {
-    int *cnt;      // arrivals per group; every counter is zero between panels
-    int *idx;      // [sets][kPW] candidate row ids, -1 for none
-    float2 *val;   // [sets][kPW][kPW] their panel entries (after the previous panel's update)
+    int *cnt;                  // arrivals per group; every counter is zero between panels
+    unsigned long long *idx;   // [sets][kPW] candidate row numbers (-1: none) << 32 | tag of the panel
 };
 
-// The tournament of the panel [c, c + pw) as one launch, and the previous
-// panel's update of the block columns to its right.
-// Workgroups [0, nsets0) each take kTsluT rows (r >= c): with prev set they first
-// apply the previous panel's update to their rows of the panel columns
-// (A[r, c:c+pw) -= L21(r) U12, L21 = A[r, c-kPW:c), U12 = A[c-kPW:c, c:c+pw)) and
-// write it back, then select <= pw candidates by partial pivoting.  A workgroup
-// publishes its set and counts itself into its group of kTsluFan sets (agent-scope
-// release / acquire); the last to arrive merges the group's sets at the next
-// level, and so on, so no workgroup waits for another.  The workgroup that
-// partial-pivots the last single set writes L11 \ U11, ipiv, the panel rows
-// before the moves and the row-move plan.
-// Workgroups [nsets0, ...) are the tiles of A[c:, c+kPW : c+kPW+upd_n) -=
-// L21 U12 with the same L21 and U12 (the rest of the previous panel's update).
+// The tournament of the panel [c, c + pw) with entries P as one launch, and the rest of the
+// previous panel's update.
+// Workgroups [0, nsets0) each take kTsluRows rows (r >= c) and select <= pw candidates by
+// partial pivoting.  A workgroup publishes its set's row numbers, each with the panel's tag,
+// and counts itself into its group; the last to arrive reads the group's numbers as their
+// tags appear, takes the rows from P and merges them at the next level, and so on, so no
+// workgroup waits for one that has not run.  The workgroup that partial-pivots the last
+// single set writes L11 \ U11, ipiv and the row moves.
+// Workgroup nsets0 (prev set) stores the previous panel's block row in this panel's columns
+// (unext), and those behind it are the tiles of A[c:, c+kPW : c+kPW+upd_n) -= L21 U12 with
+// the previous panel's L21 and U12 (this panel's columns had theirs from k_tslu_apply).
 __device__ __forceinline__ void tslu_panel_body(float2 *A, long long lda, int n, int c, int pw, int nsets0, int prev,
-                                                int upd_n, const TsluWork &tw, const TsluFinal &fin, int bid)
+                                                int upd_n, const float2 *P, const float2 *unext, const TsluWork &tw,
+                                                const TsluFinal &fin, int bid)
 {
-    if (bid >= nsets0) {
-        cgemm_tile<float, 4, 2, true>(bid - nsets0, A + (long long)c * lda + c - kPW, lda,
+    if (bid > nsets0) {
+        cgemm_tile<float, 4, 2, true>(bid - nsets0 - 1, A + (long long)c * lda + c - kPW, lda,
                                       A + (long long)(c - kPW) * lda + c + kPW, lda, A + (long long)c * lda + c + kPW,
                                       lda, n - c, upd_n, kPW);
         return;
     }
-    __shared__ unsigned s_key[2][4];
-    __shared__ __align__(16) float2 s_row[2][4][kPW];
-    __shared__ int piv[kPW], s_rowid[kTsluT], zero_at, s_next;
-    __shared__ int s_win[kPW], s_at[kPW], s_pos[kPW];
-    __shared__ __align__(16) float2 s_u[kPW][kPW];
-    const int tid = threadIdx.x;
-    for (int e = tid; e < 2 * 4 * kPW; e += kTsluT) (&s_row[0][0][0])[e] = float2{0, 0};   // finite slots
-    __syncthreads();
-    int g = bid, nl = nsets0, off = 0, coff = 0;
-    int rowid = -1;
-    float2 v[kPW], orig[kPW];
-    {
-        const long long r = (long long)c + (long long)g * kTsluT + tid;
-        if (r < n) rowid = (int)r;
-#pragma unroll
-        for (int cc = 0; cc < kPW; ++cc) v[cc] = (rowid >= 0 && cc < pw) ? A[r * lda + c + cc] : float2{0, 0};
-        if (prev) {
-            for (int idx = tid; idx < kPW * kPW; idx += kTsluT) {
-                const int i = idx / kPW, cc = idx % kPW;
-                s_u[i][cc] = cc < pw ? A[(long long)(c - kPW + i) * lda + c + cc] : float2{0, 0};
-            }
-            __syncthreads();
-            if (rowid >= 0) {
-                const float2 *lrow = A + r * lda + c - kPW;
-                float2 l = lrow[0];
-#pragma unroll 1
-                for (int i = 0; i < kPW; ++i) {
-                    const float2 ln = lrow[min(i + 1, kPW - 1)];   // the next multiplier, loaded ahead
-                    float2 ur[kPW];                                 // row i of U12, read in one batch
-#pragma unroll
-                    for (int cc = 0; cc < kPW; ++cc) ur[cc] = s_u[i][cc];
-#pragma unroll
-                    for (int cc = 0; cc < kPW; ++cc) {
-                        v[cc].x = fmaf(l.y, ur[cc].y, fmaf(-l.x, ur[cc].x, v[cc].x));
-                        v[cc].y = fmaf(-l.y, ur[cc].x, fmaf(-l.x, ur[cc].y, v[cc].y));
-                    }
-                    l = ln;
-                }
-#pragma unroll
-                for (int cc = 0; cc < kPW; ++cc)
-                    if (cc < pw) A[r * lda + c + cc] = v[cc];
-            }
-        }
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    if (bid == nsets0) {
+        for (int e = tid; e < kPW * kPW; e += kTsluT)
+            if (e % kPW < pw) A[(long long)(c - kPW + e / kPW) * lda + c + e % kPW] = unext[e];
+        return;
     }
-#pragma unroll
-    for (int cc = 0; cc < kPW; ++cc) orig[cc] = v[cc];
-    s_rowid[tid] = rowid;
-    if (tid == 0) zero_at = INT_MAX;
+    __shared__ GeppLds S;
+    __shared__ int s_rowid[kTsluRows], s_next;
+    const unsigned tag = (unsigned)c + 1u;
+    int g = bid, nl = nsets0, off = 0, coff = 0;
+    size_t first = 0;   // first set of the group being merged
+    int nrows = -1;     // its rows (-1: the first stage)
+    float2 v[2][kPW];
+    bool used[2];
+    int slot[2], j_of[2];   // j_of: the column the row pivots, -1 for none
     for (;;) {
-        block_gepp(v, rowid < 0, pw, piv, s_key, s_row);
+        // each thread reads its rows as they lie (turning coalesced loads through LDS took 7 us
+        // for 512 rows, these 3.5 us); a row that is none takes no part, whatever its registers hold
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            slot[h] = tid + h * kTsluT;
+            used[h] = true;
+            if (h == 1 && nrows >= 0 && nrows <= kTsluT) continue;
+            int id = -1;
+            if (nrows < 0) {
+                const int row = c + g * kTsluRows + slot[h];
+                id = row < n ? row : -1;
+            } else if (slot[h] < nrows) {
+                const unsigned long long *w = tw.idx + first * kPW + slot[h];
+                unsigned long long x;
+                // its workgroup stored it before it counted itself: on its way at most
+                do x = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                while ((unsigned)x != tag);
+                id = (int)(x >> 32);
+            }
+            const char *Pb = (const char *)P;
+            const unsigned at = (unsigned)max(id, 0) * (unsigned)(kPW * sizeof(float2));
+#pragma unroll
+            for (int q = 0; q < kPW / 2; ++q) {
+                const float4 x = *(const float4 *)(Pb + at + q * 16);
+                v[h][2 * q] = float2{x.x, x.y};
+                v[h][2 * q + 1] = float2{x.z, x.w};
+            }
+            s_rowid[slot[h]] = id;
+            used[h] = id < 0;
+        }
+        // two rows per thread, or one where they suffice
+        if (nrows >= 0 && nrows <= kTsluT) {
+            block_gepp<1>(v, used, slot, j_of, pw, S);
+        } else {
+            block_gepp<2>(v, used, slot, j_of, pw, S);
+        }
         if (nl == 1) break;
-        // publish this set: the owner of pivot j stages its entries in LDS (s_u is free
-        // after the first stage), and wave 0 writes the row ids and entries, so that
-        // thread 0's release fence covers every store of the set (a barrier does not wait
-        // for other waves' stores, and a fence orders its own wave's)
-        const size_t set = (size_t)(off + g);
-        int j_of = -1;
-        for (int j = 0; j < pw; ++j)
-            if (piv[j] == tid) j_of = j;
-        if (j_of >= 0) {
-#pragma unroll
-            for (int cc = 0; cc < kPW; ++cc) s_u[j_of][cc] = orig[cc];
+        if (tid < kPW) {
+            const int p = tid < pw ? S.piv[tid] : -1;
+            const int id = p >= 0 ? s_rowid[p] : -1;
+            __hip_atomic_store(tw.idx + (size_t)(off + g) * kPW + tid, ((unsigned long long)(unsigned)id << 32) | tag,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        __syncthreads();
-        if (tid < 64) {
-            if (tid < kPW) {
-                const int p = tid < pw ? piv[tid] : -1;
-                tw.idx[set * kPW + tid] = p >= 0 ? s_rowid[p] : -1;
-            }
-            for (int e = tid; e < kPW * kPW; e += 64) {
-                const int j = e / kPW;
-                if (j < pw && piv[j] >= 0) tw.val[set * kPW * kPW + e] = s_u[j][e % kPW];
-            }
-        }
+        const int fan = tslu_fan(nl), grp = g / fan, members = min(fan, nl - grp * fan);
         if (tid == 0) {
-            const int grp = g / kTsluFan, members = min(kTsluFan, nl - grp * kTsluFan);
-            __threadfence();
-            const int arrived = __hip_atomic_fetch_add(tw.cnt + coff + grp, 1, __ATOMIC_ACQ_REL,
-                                                       __HIP_MEMORY_SCOPE_AGENT);
-            int next = -1;
-            if (arrived == members - 1) {
+            const int arrived = __hip_atomic_fetch_add(tw.cnt + coff + grp, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (arrived == members - 1)
                 __hip_atomic_store(tw.cnt + coff + grp, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __threadfence();
-                next = grp;
-            }
-            s_next = next;
+            s_next = arrived == members - 1;
         }
         __syncthreads();
-        const int grp = s_next;
-        if (grp < 0) return;
+        if (!s_next) return;
         // the last of its group: merge the group's sets one level up
-        const size_t first = (size_t)off + (size_t)grp * kTsluFan;
-        const int nrows = min(kTsluFan, nl - grp * kTsluFan) * kPW;
-        coff += (nl + kTsluFan - 1) / kTsluFan;
+        first = (size_t)off + (size_t)grp * fan;
+        nrows = members * kPW;
+        coff += tslu_groups(nl);
         off += nl;
-        nl = (nl + kTsluFan - 1) / kTsluFan;
+        nl = tslu_groups(nl);
         g = grp;
-        rowid = tid < nrows ? tw.idx[first * kPW + tid] : -1;
-#pragma unroll
-        for (int cc = 0; cc < kPW; ++cc) v[cc] = rowid >= 0 ? tw.val[(first * kPW + tid) * kPW + cc] : float2{0, 0};
-#pragma unroll
-        for (int cc = 0; cc < kPW; ++cc) orig[cc] = v[cc];
-        s_rowid[tid] = rowid;
     }
     // last stage: the owners of the pivot rows write L11 \ U11
-    int j_of = -1;
-    for (int j = 0; j < pw; ++j)
-        if (piv[j] == tid) j_of = j;
-    if (j_of >= 0) {
 #pragma unroll
-        for (int cc = 0; cc < kPW; ++cc) {
-            fin.top[j_of * kPW + cc] = cc < pw ? v[cc] : float2{0, 0};
-            if (cc == j_of && v[cc].x == 0.f && v[cc].y == 0.f) atomicMin(&zero_at, j_of);
+    for (int h = 0; h < 2; ++h)
+        if (j_of[h] >= 0) {   // (columns past pw are zero)
+            float4 *o = (float4 *)(fin.top + j_of[h] * kPW);
+#pragma unroll
+            for (int q = 0; q < kPW / 2; ++q)
+                o[q] = float4{v[h][2 * q].x, v[h][2 * q].y, v[h][2 * q + 1].x, v[h][2 * q + 1].y};
         }
-    }
-    for (int idx = tid; idx < kPW * kPW; idx += kTsluT) {
-        const int j = idx / kPW, cc = idx % kPW;
-        if (j >= pw) fin.top[idx] = float2{0, 0};
-        const long long r = (long long)c + j;
-        fin.oldtop[idx] = (j < pw && cc < pw) ? A[r * lda + c + cc] : float2{0, 0};
-    }
-    if (tid < kPW) {
-        const int p = tid < pw ? piv[tid] : -1;
-        s_win[tid] = p >= 0 ? s_rowid[p] : -1;
-        s_at[tid] = c + tid;    // row now at position c + tid
-        s_pos[tid] = c + tid;   // position of row c + tid
-    }
-    __syncthreads();
-    if (tid == 0) {
-        // sequential interchanges bringing winner j to position c + j: rows of the
-        // panel's own positions are tracked in s_at / s_pos; a winner from further
-        // down has not moved before its own step
-        int first_bad = zero_at;
+    for (int e = tid; e < kPW * kPW; e += kTsluT)
+        if (e / kPW >= pw) fin.top[e] = float2{0, 0};
+    if (wid == 0) {
+        // sequential interchanges bringing winner j to position c + j: lane t < pw follows the row
+        // that began at c + t; a winner from further down has not moved before its own step
+        const int pv = lane < pw ? S.piv[lane] : -1;
+        const int win = pv >= 0 ? s_rowid[pv] : -1;
+        int pos = c + lane, mine = c + lane;   // position of row c + lane; interchange of column lane
         for (int j = 0; j < pw; ++j) {
-            const int here = c + j, w = s_win[j];
-            if (w < 0) {   // fewer candidates than columns: cannot happen for pw <= n - c
-                fin.ipiv[here] = here;
-                first_bad = min(first_bad, j);
-                continue;
-            }
-            const int p = (w < c + pw) ? s_pos[w - c] : w;
-            fin.ipiv[here] = p;
-            if (p != here) {
-                const int occupant = s_at[j];   // a row of the panel's own positions
-                s_at[j] = w;
-                if (p < c + pw) s_at[p - c] = occupant;
-                if (w < c + pw) s_pos[w - c] = here;
-                s_pos[occupant - c] = p;
-            }
+            const int here = c + j, w = __builtin_amdgcn_readlane(win, j);
+            if (w < 0) continue;   // fewer candidates than columns: cannot happen for pw <= n - c
+            const int own = w < c + pw ? w - c : -1;
+            const int at = own >= 0 ? __builtin_amdgcn_readlane(pos, own) : w;
+            if (lane == j) mine = at;
+            if (lane == own) pos = here;
+            else if (lane < pw && pos == here) pos = at;
         }
-        // moves: positions c + j receive the winners; a panel row that ended
-        // below the panel's positions moves there
-        int m = 0;
-        for (int j = 0; j < pw; ++j) {
-            const int w = s_win[j] >= 0 ? s_win[j] : c + j;
-            if (w != c + j) {
-                fin.plan[1 + m] = c + j;
-                fin.plan[1 + kPlanMax + m] = w;
-                ++m;
-            }
+        if (lane < pw) fin.ipiv[c + lane] = mine;
+        if (lane == 0 && S.zero != INT_MAX && *fin.info == 0) *fin.info = c + S.zero + 1;
+        if (lane < kPW) {
+            fin.moves[lane] = lane < pw && win >= 0 ? win : c + lane;
+            fin.moves[kPW + lane] = lane < pw && pos >= c + pw ? pos : -1;
         }
-        for (int t = 0; t < pw; ++t) {
-            if (s_pos[t] >= c + pw) {
-                fin.plan[1 + m] = s_pos[t];
-                fin.plan[1 + kPlanMax + m] = c + t;
-                ++m;
-            }
-        }
-        fin.plan[0] = m;
-        if (first_bad != INT_MAX && *fin.info == 0) *fin.info = c + first_bad + 1;
     }
 }
 
 __global__ __launch_bounds__(kTsluT, 2) void k_tslu_panel(float2 *A, long long lda, int n, int c, int pw, int nsets0,
-                                                          int prev, int upd_n, TsluWork tw, TsluFinal fin)
+                                                          int prev, int upd_n, const float2 *P, const float2 *unext,
+                                                          TsluWork tw, TsluFinal fin)
 {
-    tslu_panel_body(A, lda, n, c, pw, nsets0, prev, upd_n, tw, fin, blockIdx.x);
+    tslu_panel_body(A, lda, n, c, pw, nsets0, prev, upd_n, P, unext, tw, fin, blockIdx.x);
 }
 
-// After a tournament: workgroups [0, nsw) move the planned rows in the columns
-// [a0, a1) and [b0, b1) (16 columns each, all sources read before any
-// destination is written); the others finish the panel rows r >= c: rows
-// c .. c+pw become L11 \ U11, every other row x (its pre-move panel entries,
-// from oldtop when it was a panel row) becomes L21 = x U11^-1.
-__device__ __forceinline__ void tslu_apply_body(float2 *A, long long lda, int n, int c, int pw, const float2 *top,
-                                                const float2 *oldtop, const int *plan, int a0, int a1, int b0, int b1,
-                                                int nsw, int bid)
+// A block column's first panel: its entries into P.
+__device__ __forceinline__ void tslu_load_body(const float2 *A, long long lda, int n, int c, int pw, float2 *P, int bid)
 {
-    __shared__ int s_dst[kPlanMax], s_src[kPlanMax], s_m;
-    __shared__ float2 s_buf[kPlanMax][16];
+    const long long e = (long long)bid * 256 + threadIdx.x;
+    const long long r = c + e / kPW;
+    const int q = (int)(e % kPW);
+    if (r < n) P[r * kPW + q] = q < pw ? A[r * lda + c + q] : float2{0, 0};
+}
+
+__global__ __launch_bounds__(256) void k_tslu_load(const float2 *A, long long lda, int n, int c, int pw, float2 *P)
+{
+    tslu_load_body(A, lda, n, c, pw, P, blockIdx.x);
+}
+
+// After a tournament.  Workgroups [0, nsw): the row moves and the panel's block row in the
+// block's columns [a0, a1) left of the panel and [b0, b1) right of the next panel
+// (apply_strip).  The others take ROWS panel rows r >= c each: rows c .. c+pw become
+// L11 \ U11, every other row x (its entries in P, those of the panel row that moves here where
+// one does) becomes L21 = x U11^-1, 16 lanes to a row; every workgroup forms the block row
+// U12 in the next panel's nextw columns for itself; then the next panel's entries are
+// Pn = (moved rows) - L21 U12.  In A the next panel's columns stay as they are (other
+// workgroups read the rows that move); U12 goes to unext and from there into A with the next
+// launch.  Bound by the chains of the two solves, 32 steps each; with 32 rows a workgroup
+// they are halved while that still gives each CU one (8192 rows), beyond that 64 rows share
+// a block row.
+struct TsluApply {
+    float2 *A;
+    long long lda;
+    int n, c, pw;
+    const float2 *top;
+    const int *moves;
+    int a0, a1, b0, b1, nsw, nextw;
+    const float2 *P;
+    float2 *Pn, *unext;
+};
+
+template <int ROWS>
+__device__ __forceinline__ void tslu_apply_rows(const TsluApply &a, int bid)
+{
+    constexpr int SETS = ROWS / 16, NC = kPW * ROWS / 256;   // rows per row group; next columns per thread
     __shared__ float2 U[kPW][kPW + 1];
-    const int tid = threadIdx.x;
-    if (tid == 0) s_m = plan[0];
-    if (tid < kPlanMax) {
-        s_dst[tid] = plan[1 + tid];
-        s_src[tid] = plan[1 + kPlanMax + tid];
+    __shared__ __align__(16) float2 Un[kPW][kPW];
+    __shared__ float2 xs[ROWS][kPW + 1];
+    __shared__ int s_win[kPW], s_src[ROWS];
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, r = lane & 15;
+    const int c = a.c, pw = a.pw, n = a.n, nextw = a.nextw;
+    const long long lda = a.lda;
+    const int row0 = c + (bid - a.nsw) * ROWS;
+    for (int i = tid; i < ROWS; i += 256) s_src[i] = row0 + i;
+    if (tid < kPW) s_win[tid] = a.moves[tid];
+    for (int e = tid; e < kPW * kPW; e += 256) U[e / kPW][e % kPW] = a.top[e];
+    __syncthreads();
+    if (tid < pw) {   // a panel row that moves into these rows
+        const int to = a.moves[kPW + tid] - row0;
+        if (to >= 0 && to < ROWS) s_src[to] = c + tid;
     }
     __syncthreads();
-    const int m = s_m;
-    if (bid < nsw) {
-        const int cl = tid & 15, rl = tid >> 4;
-        const int t = bid * 16 + cl, w1 = a1 - a0;
-        int col = -1;
-        if (t < w1) col = a0 + t;
-        else if (t < w1 + (b1 - b0)) col = b0 + (t - w1);
-        for (int s = rl; s < m; s += 16)
-            if (col >= 0) s_buf[s][cl] = A[(long long)s_src[s] * lda + col];
-        __syncthreads();
-        for (int s = rl; s < m; s += 16)
-            if (col >= 0) A[(long long)s_dst[s] * lda + col] = s_buf[s][cl];
-        if (bid * 16 + 16 <= w1 || b1 <= b0) return;   // no columns right of the panel
-        // the panel's block row in the columns to its right: U12 = L11^-1 (moved rows c .. c+pw),
-        // L11 the unit lower part of top; one thread per column, the column in registers
-        for (int idx = tid; idx < kPW * kPW; idx += 256) U[idx / kPW][idx % kPW] = top[idx];
-        __syncthreads();
-        if (rl != 0 || t < w1 || col < 0) return;
-        float2 x[kPW];
+    // all loads first: the panel rows, the winners' and the moved rows' next columns
+    float2 x0[SETS], x1[SETS], w0[2], w1[2], v[NC];
+    int row[SETS];
 #pragma unroll
-        for (int i = 0; i < kPW; ++i) x[i] = i < pw ? A[(long long)(c + i) * lda + col] : float2{0, 0};
+    for (int k = 0; k < SETS; ++k) {
+        const int i = (k * 4 + wid) * 4 + (lane >> 4);
+        row[k] = row0 + i;
+        const float2 *src = a.P + (size_t)min(s_src[i], n - 1) * kPW;
+        x0[k] = src[r];
+        x1[k] = src[r + 16];
+    }
 #pragma unroll
-        for (int i = 1; i < kPW; ++i) {
-            if (i < pw) {   // uniform
-                float2 acc = x[i];
-#pragma unroll
-                for (int j = 0; j < i; ++j) acc = csubv(acc, cmulv(U[i][j], x[j]));
-                x[i] = acc;
-            }
+    for (int k = 0; k < 2; ++k) {
+        const int col = k * 16 + wid * 4 + (lane >> 4);
+        w0[k] = w1[k] = float2{0, 0};
+        if (col < nextw) {
+            w0[k] = a.A[(long long)s_win[r] * lda + c + kPW + col];
+            w1[k] = a.A[(long long)s_win[r + 16] * lda + c + kPW + col];
         }
-#pragma unroll
-        for (int i = 0; i < kPW; ++i)
-            if (i < pw) A[(long long)(c + i) * lda + col] = x[i];
-        return;
     }
-    for (int idx = tid; idx < kPW * kPW; idx += 256) U[idx / kPW][idx % kPW] = top[idx];
+    const int vi = tid % ROWS, vc = tid / ROWS * NC, vr = row0 + vi;
+    const bool below = vr >= c + pw && vr < n;
+    const long long vs = (long long)min(s_src[vi], n - 1) * lda + c + kPW + vc;
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+        v[q] = float2{0, 0};
+        if (below && vc + q < nextw) v[q] = a.A[vs + q];
+    }
+    if (nextw > 0) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int col = k * 16 + wid * 4 + (lane >> 4);
+            unit_solve_step<0>(w0[k], w1[k], U, r);
+            Un[r][col] = w0[k];
+            Un[r + 16][col] = w1[k];
+        }
+    }
+    auto recip = [](float2 d) {
+        const float den = fmaf(d.x, d.x, d.y * d.y), q = den != 0.f ? __builtin_amdgcn_rcpf(den) : 0.f;
+        return float2{d.x * q, -d.y * q};
+    };
+    const float2 i0 = recip(U[r][r]), i1 = recip(U[r + 16][r + 16]);
+#pragma unroll
+    for (int k = 0; k < SETS; ++k) {
+        right_solve_step<0>(x0[k], x1[k], U, r, i0, i1);
+        const int at = row[k] - c;
+        if (at < pw) {
+            x0[k] = U[min(at, kPW - 1)][r];
+            x1[k] = U[min(at, kPW - 1)][r + 16];
+        }
+        xs[row[k] - row0][r] = x0[k];
+        xs[row[k] - row0][r + 16] = x1[k];
+        if (row[k] < n) {
+            float2 *o = a.A + (long long)row[k] * lda + c;
+            if (r < pw) o[r] = x0[k];
+            if (r + 16 < pw) o[r + 16] = x1[k];
+        }
+    }
+    if (nextw <= 0) return;
     __syncthreads();
-    const long long r = (long long)c + (long long)(bid - nsw) * 256 + tid;
-    if (r >= n) return;
-    float2 *row = A + r * lda + c;
-    if (r < c + pw) {
-        const int j = (int)(r - c);
-        for (int cc = 0; cc < pw; ++cc) row[cc] = U[j][cc];
-        return;
+    if (bid == a.nsw)
+        for (int e = tid; e < kPW * kPW; e += 256) a.unext[e] = Un[e / kPW][e % kPW];
+    if (!below) return;
+#pragma unroll 4
+    for (int i = 0; i < kPW; ++i) {
+        const float2 l = xs[vi][i];
+        float2 u[NC];
+#pragma unroll
+        for (int q = 0; q < NC; ++q) u[q] = Un[i][vc + q];
+#pragma unroll
+        for (int q = 0; q < NC; ++q) {
+            v[q].x = fmaf(l.y, u[q].y, fmaf(-l.x, u[q].x, v[q].x));
+            v[q].y = fmaf(-l.y, u[q].x, fmaf(-l.x, u[q].y, v[q].y));
+        }
     }
-    int from = -1;   // panel row whose entries move here
-    for (int s = 0; s < m; ++s)
-        if (s_dst[s] == r) from = s_src[s] - c;
-    const float2 *srow = from >= 0 ? oldtop + (size_t)from * kPW : row;
-    float2 x[kPW];
+    float4 *o = (float4 *)(a.Pn + (size_t)vr * kPW + vc);
 #pragma unroll
-    for (int cc = 0; cc < kPW; ++cc) x[cc] = cc < pw ? srow[cc] : float2{0, 0};
-    right_trsv_phase<0>(x, pw, U);
-    right_trsv_phase<1>(x, pw, U);
-    right_trsv_phase<2>(x, pw, U);
-    right_trsv_phase<3>(x, pw, U);
-#pragma unroll
-    for (int cc = 0; cc < kPW; ++cc)
-        if (cc < pw) row[cc] = x[cc];
+    for (int q = 0; q < NC / 2; ++q) o[q] = float4{v[2 * q].x, v[2 * q].y, v[2 * q + 1].x, v[2 * q + 1].y};
 }
 
-__global__ __launch_bounds__(256) void k_tslu_apply(float2 *A, long long lda, int n, int c, int pw, const float2 *top,
-                                                    const float2 *oldtop, const int *plan, int a0, int a1, int b0,
-                                                    int b1, int nsw)
+__device__ __forceinline__ void tslu_apply_body(const TsluApply &a, int bid)
 {
-    tslu_apply_body(A, lda, n, c, pw, top, oldtop, plan, a0, a1, b0, b1, nsw, blockIdx.x);
+    if (bid < a.nsw)
+        apply_strip<float>(a.A, a.lda, a.c, a.top, kPW, a.pw, a.moves, a.a0, a.a1, a.b0, a.b1, bid);
+    else if (tslu_apply_row_count(a.n - a.c) == 32)
+        tslu_apply_rows<32>(a, bid);
+    else
+        tslu_apply_rows<64>(a, bid);
+}
+
+__global__ __launch_bounds__(256) void k_tslu_apply(TsluApply a)
+{
+    tslu_apply_body(a, blockIdx.x);
 }
 
 // ---------------------------------------------------------------- row interchanges
@@ -2366,14 +2430,13 @@ void check(const char *what)
 template <typename T>
 struct LUWork {
     DevBuf<unsigned long long> slots;      // FP64 panels: the workgroups' candidates
-    DevBuf<int> moves;                     // FP64 panels: row moves of the last one
+    DevBuf<int> moves;                     // row moves of the last panel
     DevBuf<int> info;
     DevBuf<int> plan;                      // row-interchange plan (k_swap_plan)
     DevBuf<int> tcnt;                      // tournament group counters (zero between panels)
-    DevBuf<int> tidx;                      // tournament candidate sets (row ids), all levels
-    DevBuf<float2> tval;                   // their panel rows
-    DevBuf<float2> top, oldtop;            // factored winners; panel rows before the moves
-    DevBuf<int> tplan;                     // row moves of the last tournament
+    DevBuf<unsigned long long> tidx;       // tournament candidate sets (tagged row numbers), all levels
+    DevBuf<float2> tpan;                   // the panels' entries, two arrays in turn
+    DevBuf<float2> top, unext;             // factored winners; block row in the next panel's columns
     DevBuf<int> plan_side;                 // row-interchange plan of the block-column stream
     DevBuf<__bf16> pa_side, pb_side;       // split planes of the block-column stream
     DevBuf<__bf16> pa_u12;                 // split planes of L for the block row
@@ -2483,31 +2546,58 @@ void panel64(Ctx &ctx, hipStream_t s, LUWork<double> &W, double2 *A, long long l
         gemm<double>(ctx, s, A, lda, c + pw, c, c, c + pw, c + pw, c + pw, n - (c + pw), k + kb - (c + pw), pw);
 }
 
-// Panel of columns [c, c + pw) of the block column [k, k + kb) by tournament
-// pivoting.  One launch applies the previous panel's update to the block's
-// columns right of it (prev) and runs the tournament, which writes ipiv[c .. c+pw);
-// the apply launch moves the rows in the block's other columns, finishes the
-// panel rows and forms the panel's block row U12 right of the panel.
-void tslu_panel(Ctx &ctx, hipStream_t s, LUWork<float> &W, float2 *A, long long lda, int n, int k, int kb, int c,
-                int pw, long long *ipiv, bool prev)
+// One panel's launches, for the single and the batched schedule: the tournament's workgroups
+// and k_tslu_apply's arguments and workgroups for the panel [c, c + pw) of the block column
+// [k, k + kb).
+struct TsluPanel {
+    int nsets0, prev, upd_n, blocks, apply_blocks;
+    const float2 *P;
+    TsluApply ap;
+};
+
+TsluPanel tslu_plan(float2 *A, long long lda, int n, int k, int kb, int c, int pw, float2 *tpan, const float2 *top,
+                    const int *moves, float2 *unext)
 {
-    const TsluFinal fin{ipiv, W.top.p, W.oldtop.p, W.tplan.p, W.info.p};
-    const TsluWork tw{W.tcnt.p, W.tidx.p, W.tval.p};
+    TsluPanel t{};
+    float2 *P[2] = {tpan, tpan + (size_t)n * kPW};
+    const int turn = (c / kPW) & 1;
+    t.P = P[turn];
+    t.nsets0 = (n - c + kTsluRows - 1) / kTsluRows;
+    t.prev = c > k ? 1 : 0;
+    t.upd_n = t.prev ? std::max(0, k + kb - (c + kPW)) : 0;
+    const long long tiles = t.upd_n > 0 ? (long long)((n - c + 127) / 128) * ((t.upd_n + 63) / 64) : 0;
+    BH_REQUIRE(t.nsets0 + 1 + tiles < (1LL << 31), "tournament grid too large");
+    t.blocks = (int)(t.nsets0 + t.prev + tiles);
+    const int nextw = std::min(kPW, k + kb - (c + pw));
+    const int b0 = std::min(c + pw + kPW, k + kb), w = (c - k) + (k + kb - b0), nsw = (w + 15) / 16;
+    t.ap = TsluApply{A, lda, n, c, pw, top, moves, k, c, b0, k + kb, nsw, nextw, t.P, P[turn ^ 1], unext};
+    const int ar = tslu_apply_row_count(n - c);
+    t.apply_blocks = nsw + (n - c + ar - 1) / ar;
+    return t;
+}
+
+// Panel of columns [c, c + pw) of the block column [k, k + kb) by tournament
+// pivoting.  One launch runs the tournament, which writes ipiv[c .. c+pw), and applies the
+// previous panel's update to the block's columns right of this panel; the apply launch
+// moves the rows in the block's other columns, finishes the panel rows, forms the panel's
+// block row and brings the next panel up to date.
+void tslu_panel(Ctx &ctx, hipStream_t s, LUWork<float> &W, float2 *A, long long lda, int n, int k, int kb, int c,
+                int pw, long long *ipiv)
+{
+    const TsluFinal fin{ipiv, W.top.p, W.moves.p, W.info.p};
+    const TsluPanel t = tslu_plan(A, lda, n, k, kb, c, pw, W.tpan.p, W.top.p, W.moves.p, W.unext.p);
     {
-        const int nsets0 = (n - c + kTsluT - 1) / kTsluT;
-        const int upd_n = prev ? std::max(0, k + kb - (c + kPW)) : 0;
-        const long long tiles = upd_n > 0 ? (long long)((n - c + 127) / 128) * ((upd_n + 63) / 64) : 0;
-        BH_REQUIRE(nsets0 + tiles < (1LL << 31), "tournament grid too large");
-        ProfScope prof(ctx, "k_tslu_panel", (double)(n - c) * pw * sizeof(float2) * (prev ? 3 : 1), s);
-        k_tslu_panel<<<(unsigned)(nsets0 + tiles), kTsluT, 0, s>>>(A, lda, n, c, pw, nsets0, prev ? 1 : 0, upd_n, tw,
-                                                                  fin);
+        ProfScope prof(ctx, "k_tslu_panel", (double)(n - c) * pw * sizeof(float2), s);
+        if (!t.prev) {
+            k_tslu_load<<<(unsigned)(((long long)(n - c) * kPW + 255) / 256), 256, 0, s>>>(A, lda, n, c, pw, (float2 *)t.P);
+            check("k_tslu_load");
+        }
+        k_tslu_panel<<<(unsigned)t.blocks, kTsluT, 0, s>>>(A, lda, n, c, pw, t.nsets0, t.prev, t.upd_n, t.P, W.unext.p,
+                                                          TsluWork{W.tcnt.p, W.tidx.p}, fin);
         check("k_tslu_panel");
     }
-    ProfScope prof(ctx, "k_tslu_apply", (double)(n - c) * pw * sizeof(float2) * 2, s);
-    const int w = (c - k) + (k + kb - (c + pw));
-    const int nsw = (w + 15) / 16;
-    const int grid = nsw + (n - c + 255) / 256;
-    k_tslu_apply<<<grid, 256, 0, s>>>(A, lda, n, c, pw, W.top.p, W.oldtop.p, W.tplan.p, k, c, c + pw, k + kb, nsw);
+    ProfScope prof(ctx, "k_tslu_apply", (double)(n - c) * pw * sizeof(float2) * (t.ap.nextw ? 4 : 2), s);
+    k_tslu_apply<<<(unsigned)t.apply_blocks, 256, 0, s>>>(t.ap);
     check("k_tslu_apply");
 }
 
@@ -2574,9 +2664,7 @@ void factor_block(Ctx &ctx, hipStream_t s, LUWork<T> &W, typename CT<T>::t *A, l
     for (int sp = 0; sp < kb; sp += kPW) {
         const int c = k + sp, pw = std::min(kPW, kb - sp);
         if constexpr (sizeof(T) == 4) {
-            // the tournament launch carries the previous panel's update, the apply
-            // launch this panel's block row
-            tslu_panel(ctx, s, W, A, lda, n, k, kb, c, pw, ipiv, sp > 0);
+            tslu_panel(ctx, s, W, A, lda, n, k, kb, c, pw, ipiv);
         } else {
             panel64(ctx, s, W, A, lda, n, k, kb, c, pw, ipiv);
         }
@@ -2731,6 +2819,7 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
     DevBuf<__bf16> &PA = buf->PA, &PB = buf->PB;
     W.eblk_of = W.eblk_side_of = -1;
     W.info.ensure(1);
+    W.moves.ensure(2 * kPW);
     W.plan.ensure(4 * kMaxSwaps);
     BH_CHECK_HIP(hipMemsetAsync(W.info.p, 0, sizeof(int), s));
     // block column of the right-looking LU (trailing-update depth); the FP32
@@ -2758,20 +2847,20 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
         BH_REQUIRE(G <= per_cu * ctx.num_cus, "panel of %d rows: its workgroups cannot all be resident", n);
         const size_t words = (size_t)G * (4 + 8 * kPW);
         W.slots.ensure(words);
-        W.moves.ensure(2 * kPW);
         BH_CHECK_HIP(hipMemsetAsync(W.slots.p, 0, words * sizeof(unsigned long long), s));
     } else {
-        // FP32 factors only precondition GMRES-IR: their panels use tournament pivoting
-        // candidate sets of all levels: n_0 + n_1 + ... < 2 n_0 + levels
-        const size_t sets = 2 * ((size_t)(n + kTsluT - 1) / kTsluT) + 8;
+        // FP32 factors only precondition GMRES-IR: their panels use tournament pivoting.
+        // Counters start at zero; candidate words are cleared, so that no tag of an earlier
+        // factorisation is there
+        const size_t sets = tslu_sets(n);
         W.tcnt.ensure(sets);
         W.tidx.ensure(sets * kPW);
-        W.tval.ensure(sets * kPW * kPW);
+        W.tpan.ensure((size_t)2 * n * kPW);
         BH_CHECK_HIP(hipMemsetAsync(W.tcnt.p, 0, sets * sizeof(int), s));
+        BH_CHECK_HIP(hipMemsetAsync(W.tidx.p, 0, sets * kPW * sizeof(unsigned long long), s));
         W.plan_side.ensure(4 * kMaxSwaps);
         W.top.ensure((size_t)kPW * kPW);
-        W.oldtop.ensure((size_t)kPW * kPW);
-        W.tplan.ensure(1 + 2 * kPlanMax);
+        W.unext.ensure((size_t)kPW * kPW);
         W.eblk.ensure((size_t)(kNBInnerMax / kIB) * kIB * kIB);
         W.eblk_side.ensure((size_t)(kNBInnerMax / kIB) * kIB * kIB);
     }
@@ -2950,20 +3039,19 @@ long long padded_ld(int64_t n) { return (n + 63) / 64 * 64; }
 // issued once for all matrices that have it at that step.  A workgroup finds its matrix in
 // the table of each matrix's first workgroup and runs the single-matrix kernel's body on
 // that matrix's arguments, so each matrix gets the factors (and pivots) it gets alone.
+struct LoadBA {
+    const float2 *A;
+    long long lda;
+    int n, c, pw;
+    float2 *P;
+};
 struct PanelBA {
     float2 *A;
     long long lda;
     int n, c, pw, nsets0, prev, upd_n;
+    const float2 *P, *unext;
     TsluWork tw;
     TsluFinal fin;
-};
-struct ApplyBA {
-    float2 *A;
-    long long lda;
-    int n, c, pw;
-    const float2 *top, *oldtop;
-    const int *plan;
-    int a0, a1, b0, b1, nsw;
 };
 struct SwapBA {
     const long long *ipiv;
@@ -3026,16 +3114,22 @@ struct CouplingBA {
     const auto &a = ARGS[r_];                            \
     const int bid = (int)blockIdx.x - first[r_];
 
+__global__ __launch_bounds__(256) void k_tslu_load_batch(const LoadBA *args, const int *first, int count)
+{
+    BH_BATCH_ITEM(args)
+    tslu_load_body(a.A, a.lda, a.n, a.c, a.pw, a.P, bid);
+}
+
 __global__ __launch_bounds__(kTsluT, 2) void k_tslu_panel_batch(const PanelBA *args, const int *first, int count)
 {
     BH_BATCH_ITEM(args)
-    tslu_panel_body(a.A, a.lda, a.n, a.c, a.pw, a.nsets0, a.prev, a.upd_n, a.tw, a.fin, bid);
+    tslu_panel_body(a.A, a.lda, a.n, a.c, a.pw, a.nsets0, a.prev, a.upd_n, a.P, a.unext, a.tw, a.fin, bid);
 }
 
-__global__ __launch_bounds__(256) void k_tslu_apply_batch(const ApplyBA *args, const int *first, int count)
+__global__ __launch_bounds__(256) void k_tslu_apply_batch(const TsluApply *args, const int *first, int count)
 {
     BH_BATCH_ITEM(args)
-    tslu_apply_body(a.A, a.lda, a.n, a.c, a.pw, a.top, a.oldtop, a.plan, a.a0, a.a1, a.b0, a.b1, a.nsw, bid);
+    tslu_apply_body(a, bid);
 }
 
 __global__ __launch_bounds__(256) void k_swap_plan_batch(const SwapBA *args, const int *first, int count)
@@ -3108,7 +3202,7 @@ constexpr int kBatchMaxN = kNBDeepAbove;
 namespace {
 
 enum BatchKind : int {
-    kBkPanel, kBkApply, kBkSwap, kBkLaswp, kBkTrinvL, kBkTrinvU, kBkToE, kBkCgemm, kBkSplitRows, kBkSplitCols,
+    kBkLoad, kBkPanel, kBkApply, kBkSwap, kBkLaswp, kBkTrinvL, kBkTrinvU, kBkToE, kBkCgemm, kBkSplitRows, kBkSplitCols,
     kBkBf16, kBkCoupleL, kBkCoupleU
 };
 
@@ -3157,8 +3251,9 @@ struct BatchMat {
     float2 *A;
     long long *ipiv;
     // workspace (device)
-    int *tcnt, *tidx, *tplan, *plan, *info;
-    float2 *tval, *top, *oldtop, *eblk, *dinv;
+    int *tcnt, *moves, *plan, *info;
+    unsigned long long *tidx;
+    float2 *tpan, *top, *unext, *eblk, *dinv;
     __bf16 *pa, *pb;
 };
 
@@ -3169,28 +3264,26 @@ void plan_factor(BatchPlan &P, std::vector<BatchMat> &mats)
     for (int k = 0; k < nmax; k += kNBInner) {
         // the block column [k, k + kb) of every matrix that has it: its panels
         for (int sp = 0; sp < kNBInner; sp += kPW) {
+            std::vector<std::pair<LoadBA, long long>> ld;
             std::vector<std::pair<PanelBA, long long>> pan;
-            std::vector<std::pair<ApplyBA, long long>> app;
+            std::vector<std::pair<TsluApply, long long>> app;
             double wp = 0, wa = 0;
             for (auto &m : mats) {
                 if (m.n <= k) continue;
                 const int kb = std::min(kNBInner, m.n - k);
                 if (sp >= kb) continue;
-                const int c = k + sp, pw = std::min(kPW, kb - sp), prev = sp > 0;
-                const int nsets0 = (m.n - c + kTsluT - 1) / kTsluT;
-                const int upd_n = prev ? std::max(0, k + kb - (c + kPW)) : 0;
-                const long long tiles = upd_n > 0 ? (long long)((m.n - c + 127) / 128) * ((upd_n + 63) / 64) : 0;
-                PanelBA a{m.A, m.lda, m.n, c, pw, nsets0, prev, upd_n, TsluWork{m.tcnt, m.tidx, m.tval},
-                          TsluFinal{m.ipiv, m.top, m.oldtop, m.tplan, m.info}};
-                pan.push_back({a, nsets0 + tiles});
-                wp += (double)(m.n - c) * pw * sizeof(float2) * (prev ? 3 : 1);
-                const int w = (c - k) + (k + kb - (c + pw));
-                const int nsw = (w + 15) / 16;
-                ApplyBA b{m.A, m.lda, m.n, c, pw, m.top, m.oldtop, m.tplan, k, c, c + pw, k + kb, nsw};
-                app.push_back({b, nsw + (m.n - c + 255) / 256});
-                wa += (double)(m.n - c) * pw * sizeof(float2) * 2;
+                const int c = k + sp, pw = std::min(kPW, kb - sp);
+                const TsluPanel t = tslu_plan(m.A, m.lda, m.n, k, kb, c, pw, m.tpan, m.top, m.moves, m.unext);
+                if (!t.prev)
+                    ld.push_back({LoadBA{m.A, m.lda, m.n, c, pw, (float2 *)t.P}, ((long long)(m.n - c) * kPW + 255) / 256});
+                pan.push_back({PanelBA{m.A, m.lda, m.n, c, pw, t.nsets0, t.prev, t.upd_n, t.P, m.unext,
+                                       TsluWork{m.tcnt, m.tidx}, TsluFinal{m.ipiv, m.top, m.moves, m.info}}, t.blocks});
+                wp += (double)(m.n - c) * pw * sizeof(float2);
+                app.push_back({t.ap, t.apply_blocks});
+                wa += (double)(m.n - c) * pw * sizeof(float2) * (t.ap.nextw ? 4 : 2);
             }
             if (pan.empty()) break;
+            P.add(kBkLoad, ld);
             P.add(kBkPanel, pan, 0, wp);
             P.add(kBkApply, app, 0, wa);
         }
@@ -3298,6 +3391,7 @@ void plan_factor(BatchPlan &P, std::vector<BatchMat> &mats)
 const char *batch_kernel_name(int kind)
 {
     switch (kind) {
+    case kBkLoad: return "k_tslu_load";
     case kBkPanel: return "k_tslu_panel";
     case kBkApply: return "k_tslu_apply";
     case kBkSwap: return "k_swap_plan";
@@ -3322,8 +3416,9 @@ void run_plan(Ctx &ctx, const BatchPlan &P, const char *dtab)
         const void *a = dtab + L.args;
         ProfScope prof(ctx, batch_kernel_name(L.kind), L.work, s);
         switch (L.kind) {
+        case kBkLoad: k_tslu_load_batch<<<g, 256, 0, s>>>((const LoadBA *)a, first, L.count); break;
         case kBkPanel: k_tslu_panel_batch<<<g, kTsluT, 0, s>>>((const PanelBA *)a, first, L.count); break;
-        case kBkApply: k_tslu_apply_batch<<<g, 256, 0, s>>>((const ApplyBA *)a, first, L.count); break;
+        case kBkApply: k_tslu_apply_batch<<<g, 256, 0, s>>>((const TsluApply *)a, first, L.count); break;
         case kBkSwap: k_swap_plan_batch<<<g, 256, 0, s>>>((const SwapBA *)a, first, L.count); break;
         case kBkLaswp: k_laswp_apply_batch<<<g, 256, L.shm, s>>>((const LaswpBA *)a, first, L.count); break;
         case kBkTrinvL:
@@ -3483,18 +3578,18 @@ extern "C" int bh_matrix_factor_batch(bh_ctx *ctxh, int64_t count, bh_matrix *co
     if (!shared.empty()) {
         std::vector<std::unique_lock<std::mutex>> locks;
         for (bh_matrix *M : shared) locks.emplace_back(M->mu);
-        // workspace of each matrix, one allocation: counters and info first (cleared together)
+        // workspace of each matrix, one allocation: counters, info and candidate words first
+        // (cleared together)
         std::vector<BatchMat> bm(shared.size());
         size_t ints = 0, rest = 0;
         auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
         std::vector<size_t> sets(shared.size());
         for (size_t i = 0; i < shared.size(); ++i) {
             const int n = (int)shared[i]->n;
-            sets[i] = 2 * ((size_t)(n + kTsluT - 1) / kTsluT) + 8;
-            ints += al((sets[i] + 1) * sizeof(int));
+            sets[i] = tslu_sets(n);
+            ints += al((sets[i] + 1) * sizeof(int)) + al(sets[i] * kPW * sizeof(unsigned long long));
             const size_t trail = n > kNBInner ? (size_t)(n - kNBInner) : 0;
-            rest += al(sets[i] * kPW * sizeof(int)) + al((1 + 2 * kPlanMax) * sizeof(int)) +
-                    al(4 * kMaxSwaps * sizeof(int)) + al(sets[i] * kPW * kPW * sizeof(float2)) +
+            rest += al(2 * kPW * sizeof(int)) + al(4 * kMaxSwaps * sizeof(int)) + al((size_t)2 * n * kPW * sizeof(float2)) +
                     2 * al(kPW * kPW * sizeof(float2)) + al((size_t)(kNBInner / kIB) * kIB * kIB * sizeof(float2)) +
                     2 * al(4 * trail * kNBInner * sizeof(__bf16));
         }
@@ -3528,13 +3623,13 @@ extern "C" int bh_matrix_factor_batch(bh_ctx *ctxh, int64_t count, bh_matrix *co
             b.dinv = (float2 *)M->dinv32.p;
             b.tcnt = (int *)take(oi, (sets[i] + 1) * sizeof(int));
             b.info = b.tcnt + sets[i];
+            b.tidx = (unsigned long long *)take(oi, sets[i] * kPW * sizeof(unsigned long long));
             const size_t trail = n > kNBInner ? (size_t)(n - kNBInner) : 0;
-            b.tidx = (int *)take(orest, sets[i] * kPW * sizeof(int));
-            b.tplan = (int *)take(orest, (1 + 2 * kPlanMax) * sizeof(int));
+            b.moves = (int *)take(orest, 2 * kPW * sizeof(int));
             b.plan = (int *)take(orest, 4 * kMaxSwaps * sizeof(int));
-            b.tval = (float2 *)take(orest, sets[i] * kPW * kPW * sizeof(float2));
+            b.tpan = (float2 *)take(orest, (size_t)2 * n * kPW * sizeof(float2));
             b.top = (float2 *)take(orest, kPW * kPW * sizeof(float2));
-            b.oldtop = (float2 *)take(orest, kPW * kPW * sizeof(float2));
+            b.unext = (float2 *)take(orest, kPW * kPW * sizeof(float2));
             b.eblk = (float2 *)take(orest, (size_t)(kNBInner / kIB) * kIB * kIB * sizeof(float2));
             b.pa = (__bf16 *)take(orest, 4 * trail * kNBInner * sizeof(__bf16));
             b.pb = (__bf16 *)take(orest, 4 * trail * kNBInner * sizeof(__bf16));

@@ -56,6 +56,48 @@ def test_singular_pivot(bj, precision):
         M.factor(precision)
 
 
+def _plain_pivots(A):
+    """Row interchanges of Gaussian elimination, column by column: largest |Re|+|Im|, first on ties."""
+    A, piv = A.copy(), np.zeros(len(A), dtype=np.int64)
+    for j in range(len(A)):
+        piv[j] = j + np.argmax(np.abs(A[j:, j].real) + np.abs(A[j:, j].imag))
+        A[[j, piv[j]]] = A[[piv[j], j]]
+        A[j + 1:, j + 1:] -= (A[j + 1:, j] / A[j, j])[:, None] * A[j, j + 1:]
+    return piv
+
+
+@pytest.mark.parametrize("n", [512, 513, 1100])
+def test_lu_fp64_pivots_across_workgroups(bj, n):
+    """Panels of one workgroup and of several, with exact ties: columns whose entries all have
+    one magnitude, and rows that agree in all but their last columns, so that the first of
+    equal rows is the pivot wherever it lies.  The interchanges equal those of the plain
+    elimination, which rounds equal rows alike (LAPACK's blocked one does not)."""
+    A = _rand(n, n + 5)
+    A[:, 0] = 1.0
+    A[n // 2:, 0] = 2.0j
+    A[n - 40:, 1:n - 50] = A[n - 80:n - 40, 1:n - 50]
+    M = bj.DeviceMatrix.from_host(A).factor("fp64")
+    assert np.array_equal(M.pivots(), _plain_pivots(A) + 1)
+    b = _rand(n, n + 6)[:, 0]
+    assert relfro(M.solve(b), np.linalg.solve(A, b)) < 1e-9
+
+
+@pytest.mark.parametrize("n", [481, 513, 1537, 5000])
+def test_fp32_tournament_group_sizes(bj, n):
+    """One candidate set, a set of a single row, groups merged at one and at two rows per
+    thread: the dominant rows of a permuted matrix are found."""
+    rng = np.random.default_rng(n)
+    B = 0.01 * (rng.standard_normal((n, n)) + 1j * rng.standard_normal((n, n))) / np.sqrt(n)
+    B += np.diag(1.0 + rng.uniform(0, 1, n)) * np.exp(2j * np.pi * rng.uniform(0, 1, n))
+    sigma = rng.permutation(n)
+    A = np.asfortranarray(B[sigma])
+    M = bj.DeviceMatrix.from_host(A).factor("fp32")
+    assert np.array_equal(sigma[_perm_from_ipiv(M.pivots())], np.arange(n))
+    b = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    M.solve(b, tol=1e-12, maxit=10)
+    assert M.stats["residual"] <= 1e-12
+
+
 def _perm_from_ipiv(ipiv1):
     """(P A)[i] = A[perm[i]] from 1-based sequential interchanges (LAPACK getrf convention)."""
     perm = np.arange(len(ipiv1))
