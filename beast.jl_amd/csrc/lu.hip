@@ -2259,72 +2259,99 @@ __global__ __launch_bounds__(kTrsvT) void k_trsv_flag(const float2 *A, long long
     }
 }
 
-// r = b - A x in FP64 (A row-major n x n), one wave per row; x, b, r are n x nrhs row-major.
-// r = b - A x (RESID) or r = A x, for nrhs columns (x, b, r row-major n x nrhs)
-template <bool RESID>
-__device__ __forceinline__ void apply_a_body(const double2 *__restrict__ A, int n, const double2 *__restrict__ x,
-                                             const double2 *__restrict__ b, double2 *__restrict__ r, int nrhs)
+// r = b - A x (RESID) or r = A x in FP64 (A row-major n x n; x, b, r row-major n x NRHS).
+// A workgroup takes kAxRows rows; its four waves take the 64-column pieces in turn, so an
+// entry of x is loaded once for all the rows (with a wave per row, the 16 NRHS bytes of x per
+// 16 bytes of A came from the caches for every row).  Bound by the one read of A: at 12,000
+// unknowns and four columns 1.07 -> 0.50 ms (4.6 TB/s), at 39,996 and one 4.43 -> 4.11 ms
+// (6.2 TB/s).  The waves' sums meet in LDS.  Explicit FMAs, the same for every NRHS:
+// a column's bits do not depend on the others.
+constexpr int kAxRows = 4;
+
+template <bool RESID, int NRHS>
+__global__ __launch_bounds__(256) void k_apply_a(const double2 *__restrict__ A, int n, const double2 *__restrict__ x,
+                                                 const double2 *__restrict__ b, double2 *__restrict__ r)
 {
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= n) return;
-    const int lane = threadIdx.x & 63;
-    const double2 *a = A + (size_t)row * n;
-    double2 acc[kMaxRhs];
+    __shared__ double2 red[4][kAxRows][NRHS];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, row0 = blockIdx.x * kAxRows;
+    const double2 *a[kAxRows];
 #pragma unroll
-    for (int q = 0; q < kMaxRhs; ++q) acc[q] = {0, 0};
-    auto step = [&](const double2 av, int cc) {
+    for (int k = 0; k < kAxRows; ++k) a[k] = A + (size_t)min(row0 + k, n - 1) * n;
+    double2 acc[kAxRows][NRHS];
 #pragma unroll
-        for (int q = 0; q < kMaxRhs; ++q) {
-            if (q < nrhs) {
-                const double2 xv = x[(size_t)cc * nrhs + q];
-                acc[q].x += av.x * xv.x - av.y * xv.y;
-                acc[q].y += av.x * xv.y + av.y * xv.x;
+    for (int k = 0; k < kAxRows; ++k)
+#pragma unroll
+        for (int q = 0; q < NRHS; ++q) acc[k][q] = {0, 0};
+    auto step = [&](const double2 (&av)[kAxRows], int c) {
+#pragma unroll
+        for (int q = 0; q < NRHS; ++q) {
+            const double2 xv = x[(size_t)c * NRHS + q];
+#pragma unroll
+            for (int k = 0; k < kAxRows; ++k) {
+                acc[k][q].x = fma(av[k].x, xv.x, fma(-av[k].y, xv.y, acc[k][q].x));
+                acc[k][q].y = fma(av[k].x, xv.y, fma(av[k].y, xv.x, acc[k][q].y));
             }
         }
     };
-    int c = lane;
-    // four row loads in flight per lane, summed in the same order as one at a time
-    for (; c + 192 < n; c += 256) {
-        double2 av[4];
+    int c = 64 * wid + lane;
+    // two pieces of every row in flight
+    for (; c + 256 < n; c += 512) {
+        double2 u[kAxRows], v[kAxRows];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) av[u] = a[c + 64 * u];
+        for (int k = 0; k < kAxRows; ++k) u[k] = a[k][c];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) step(av[u], c + 64 * u);
+        for (int k = 0; k < kAxRows; ++k) v[k] = a[k][c + 256];
+        step(u, c);
+        step(v, c + 256);
     }
-    for (; c < n; c += 64) step(a[c], c);
+    if (c < n) {
+        double2 u[kAxRows];
 #pragma unroll
-    for (int q = 0; q < kMaxRhs; ++q) {
-        if (q >= nrhs) break;
-        double sx = acc[q].x, sy = acc[q].y;
-        for (int off = 32; off >= 1; off >>= 1) {
-            sx += __shfl_xor(sx, off, 64);
-            sy += __shfl_xor(sy, off, 64);
-        }
-        if (lane == 0) {
-            if constexpr (RESID) {
-                const double2 bv = b[(size_t)row * nrhs + q];
-                r[(size_t)row * nrhs + q] = {bv.x - sx, bv.y - sy};
-            } else {
-                r[(size_t)row * nrhs + q] = {sx, sy};
+        for (int k = 0; k < kAxRows; ++k) u[k] = a[k][c];
+        step(u, c);
+    }
+#pragma unroll
+    for (int k = 0; k < kAxRows; ++k) {
+#pragma unroll
+        for (int q = 0; q < NRHS; ++q) {
+            double sx = acc[k][q].x, sy = acc[k][q].y;
+            for (int off = 32; off >= 1; off >>= 1) {
+                sx += __shfl_xor(sx, off, 64);
+                sy += __shfl_xor(sy, off, 64);
             }
+            if (lane == 0) red[wid][k][q] = {sx, sy};
         }
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < kAxRows * NRHS && row0 + t / NRHS < n) {
+        const int k = t / NRHS, q = t % NRHS;
+        const double sx = (red[0][k][q].x + red[1][k][q].x) + (red[2][k][q].x + red[3][k][q].x);
+        const double sy = (red[0][k][q].y + red[1][k][q].y) + (red[2][k][q].y + red[3][k][q].y);
+        const size_t o = (size_t)(row0 + k) * NRHS + q;
+        if constexpr (RESID) r[o] = {b[o].x - sx, b[o].y - sy};
+        else r[o] = {sx, sy};
     }
 }
 
-__global__ __launch_bounds__(256) void k_residual(const double2 *__restrict__ A, int n, const double2 *__restrict__ x,
-                                                  const double2 *__restrict__ b, double2 *__restrict__ r, int nrhs)
+template <bool RESID>
+void apply_a(hipStream_t s, const double2 *A, int n, const double2 *x, const double2 *b, double2 *r, int nrhs)
 {
-    apply_a_body<true>(A, n, x, b, r, nrhs);
+    const unsigned g = (unsigned)((n + kAxRows - 1) / kAxRows);
+    switch (nrhs) {
+    case 1: k_apply_a<RESID, 1><<<g, 256, 0, s>>>(A, n, x, b, r); break;
+    case 2: k_apply_a<RESID, 2><<<g, 256, 0, s>>>(A, n, x, b, r); break;
+    case 3: k_apply_a<RESID, 3><<<g, 256, 0, s>>>(A, n, x, b, r); break;
+    case 4: k_apply_a<RESID, 4><<<g, 256, 0, s>>>(A, n, x, b, r); break;
+    case 5: k_apply_a<RESID, 5><<<g, 256, 0, s>>>(A, n, x, b, r); break;
+    case 6: k_apply_a<RESID, 6><<<g, 256, 0, s>>>(A, n, x, b, r); break;
+    case 7: k_apply_a<RESID, 7><<<g, 256, 0, s>>>(A, n, x, b, r); break;
+    case 8: k_apply_a<RESID, 8><<<g, 256, 0, s>>>(A, n, x, b, r); break;
+    default: BH_FAIL(BH_ERR_INVALID, "nrhs %d out of range", nrhs);
+    }
 }
 
-__global__ __launch_bounds__(256) void k_matvec_cols(const double2 *__restrict__ A, int n,
-                                                     const double2 *__restrict__ x, double2 *__restrict__ y, int nrhs)
-{
-    apply_a_body<false>(A, n, x, nullptr, y, nrhs);
-}
-
-// y = A x for one vector (FP64), used by GMRES.
-// The same for q columns side by side (row-major n x q blocks): one Krylov space per
+// GMRES vectors: q columns side by side (row-major n x q blocks), one Krylov space per
 // column, all advanced by the same launches.
 struct ColScale {
     double s[kMaxRhs];
@@ -3786,7 +3813,7 @@ int gmres_block(bh_matrix *M, const double2 *R0, int q, const double *r0norm, do
             apply_factors(M, Vb + (size_t)k * nq, zk, q);
             {
                 ProfScope prof(*M->ctx, "k_matvec", 16.0 * n * (double)n);
-                k_matvec_cols<<<(n + 3) / 4, 256, 0, s>>>((const double2 *)M->a64.p, n, zk, w, q);
+                apply_a<false>(s, (const double2 *)M->a64.p, n, zk, nullptr, w, q);
             }
             check("k_matvec");
             std::vector<std::vector<C>> h(q, std::vector<C>(k + 1, 0.0));
@@ -3879,7 +3906,7 @@ int gmres_block(bh_matrix *M, const double2 *R0, int q, const double *r0norm, do
         // restart from the true residuals R0 - A D
         {
             ProfScope prof(*M->ctx, "k_residual", 16.0 * n * (double)n);
-            k_residual<<<(n + 3) / 4, 256, 0, s>>>((const double2 *)M->a64.p, n, D, R0, r, q);
+            apply_a<true>(s, (const double2 *)M->a64.p, n, D, R0, r, q);
         }
         check("k_residual");
         k_dots_cols<<<256, 256, 0, s>>>(r, n, 1, q, r, part);
@@ -3993,7 +4020,7 @@ void solve_impl(bh_matrix *M, int64_t nrhs, const double *B, double *X, double t
         for (;;) {
             {
                 ProfScope prof(*M->ctx, "k_residual", 16.0 * n * (double)n);   // one FP64 read of A
-                k_residual<<<(n + 3) / 4, 256, 0, s>>>((const double2 *)M->a64.p, n, W.dx, W.db, W.dr, q);
+                apply_a<true>(s, (const double2 *)M->a64.p, n, W.dx, W.db, W.dr, q);
             }
             check("k_residual");
             std::vector<double2> hr(cnt);

@@ -273,3 +273,22 @@ def test_right_hand_sides_in_lockstep_equal_one_at_a_time(bj, precision, tol):
         assert np.array_equal(X[:, c], x), c
         assert np.linalg.norm(A @ x - B[:, c]) / np.linalg.norm(B[:, c]) < 1e-11
     assert inner_all == inner_sum
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [1, 3, 63, 65, 129, 255, 257, 385, 770])
+def test_columns_together_and_alone(bj, n, precision):
+    """1 to 8 right-hand sides at the edges of the solves' blocks (64 and 128 rows) and of the
+    residual's pieces (4 rows, 256 columns): solved to the tolerance by the host's own residual,
+    and each column's bits those it has alone."""
+    A = _rand(n, 11 * n)
+    rng = np.random.default_rng(n)
+    B = rng.standard_normal((n, 8)) + 1j * rng.standard_normal((n, 8))
+    M = bj.DeviceMatrix.from_host(A).factor(precision)
+    tol = 1e-12
+    for nrhs in range(1, 9):
+        x = M.solve(B[:, :nrhs], tol=tol, maxit=10)
+        # the tolerance, plus the rounding of the host's n-term sums
+        slack = n * np.finfo(float).eps * np.linalg.norm(A) * np.linalg.norm(x, axis=0)
+        assert np.all(np.linalg.norm(A @ x - B[:, :nrhs], axis=0) <= tol * np.linalg.norm(B[:, :nrhs], axis=0) + slack)
+        assert np.array_equal(x[:, -1], M.solve(B[:, nrhs - 1], tol=tol, maxit=10))
