@@ -18,9 +18,9 @@ struct bh_matrix {
     bool lu32_fresh = false;       // lu32 holds the current matrix rounded to FP32 (written by the assembly)
     bh::DevBuf<float> dinv32;      // FP32 factors: inverted 128 x 128 diagonal blocks of L and U, then G = Dinv x (block beside it)
     bh::DevBuf<float> x32;         // FP32 solve vector (n x 8 complex)
-    bh::DevBuf<int> tsync;         // FP32 solves: ticket counter, error flag, one ready flag per 128-row block
+    bh::DevBuf<unsigned long long> tsync;   // solves: ticket counter and error flag, then the solved rows as tagged words
     long long tsync_tickets = 0;   // tickets handed out so far
-    int tsync_epoch = 0;           // value of the ready flags of the last solve
+    int tsync_epoch = 0;           // tag of the last triangle
     bh::DevBuf<long long> ipiv;    // 0-based pivot rows (sequential interchanges)
     bh::DevBuf<int> perm;          // (P b)[i] = b[perm[i]]
     long long lda = 0;             // leading dimension of the factors
@@ -34,5 +34,6 @@ struct bh_matrix {
         bh::pool_release(*ctx, lu64);
         bh::pool_release(*ctx, lu32);
         bh::pool_release(*ctx, dinv32);
+        bh::pool_release(*ctx, tsync);
     }
 };

@@ -94,6 +94,11 @@ __device__ __forceinline__ float2 cfms_x(float2 a, float2 b, float2 c)
     return {fmaf(b.y, c.y, fmaf(-b.x, c.x, a.x)), fmaf(-b.y, c.x, fmaf(-b.x, c.y, a.y))};
 }
 
+__device__ __forceinline__ double2 cfma_x(double2 a, double2 b, double2 c)   // a + b c
+{
+    return {fma(-b.y, c.y, fma(b.x, c.x, a.x)), fma(b.y, c.x, fma(b.x, c.y, a.y))};
+}
+
 __device__ __forceinline__ double2 cfms_x(double2 a, double2 b, double2 c)
 {
     return {fma(b.y, c.y, fma(-b.x, c.x, a.x)), fma(-b.y, c.x, fma(-b.x, c.y, a.y))};
@@ -1760,108 +1765,248 @@ __global__ void k_permute_in(const double2 *__restrict__ b, int n, int nrhs, con
 constexpr int kTB = 64;   // triangular-solve block
 constexpr int kMaxRhs = 8;
 
-// Solve the diagonal block `blk` on xs (LDS, kTB x nrhs, holding the updated
-// right-hand side of the block): unit lower (forward) or upper (backward).
-// The block is first staged in LDS (coalesced), so the serial row sweep runs at
-// LDS latency.  All 256 threads call it; wave 0 does the sweep.
-template <typename T, bool LOWER>
-__device__ void trsv_diag(const typename CT<T>::t *A, long long lda, int n, typename CT<T>::t *xs, int nrhs, int blk,
-                          typename CT<T>::t (*D)[kTB + 1])
+// The triangular solves run one launch per triangle, one workgroup per CU.  A workgroup takes
+// a block in the order of a ticket counter, solves it and takes the next, until none is left
+// (so a block never waits for a workgroup that has not started: every block it waits for has
+// an earlier ticket, held by a running workgroup).  Tickets handed out per launch: the blocks
+// plus one final ticket per workgroup.  Solved rows travel as 64-bit words, 32 bits of value
+// over the launch's epoch: a word is valid by itself, so that neither fences nor flags are
+// needed (the writeback and invalidation of two fences per block took longer than the block's
+// products), and a block waits on the values themselves.  A wait that exceeds kTrsvSpin polls
+// sets the error word and gives up, so every workgroup ends.
+constexpr int kTrsvT = 512;                // threads of a workgroup
+constexpr long long kTrsvSpin = 1LL << 24;
+constexpr int kTrsvHead = 8;               // words before the values: [0] ticket counter and error flag
+
+// the words tid, tid + kTrsvT, .. of the cnt words at src, as they are
+template <int U>
+__device__ __forceinline__ void words_fetch(const unsigned long long *src, int cnt, unsigned long long (&w)[U])
 {
-    using V = typename CT<T>::t;
-    const int lane = threadIdx.x & 63;
-    const int b0 = blk * kTB, bs = min(kTB, n - b0);
-    for (int idx = threadIdx.x; idx < bs * kTB; idx += blockDim.x) {
-        const int i = idx / kTB, j = idx % kTB;
-        D[i][j] = j < bs ? A[(long long)(b0 + i) * lda + b0 + j] : V{0, 0};
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int t = threadIdx.x + kTrsvT * u;
+        w[u] = t < cnt ? get_word(src + t) : 0ull;
     }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-        for (int r = 0; r < nrhs; ++r) {
-            for (int s = 0; s < bs; ++s) {
-                const int i = LOWER ? s : bs - 1 - s;
-                V prod{0, 0};
-                const bool use = LOWER ? (lane < i) : (lane > i && lane < bs);
-                if (use) prod = cmulv(D[i][lane], xs[lane * nrhs + r]);
-                for (int off = 32; off >= 1; off >>= 1) {
-                    prod.x += __shfl_xor(prod.x, off, 64);
-                    prod.y += __shfl_xor(prod.y, off, 64);
+}
+
+// waits for them, all of a thread's in one round, and stores their values (zeros beyond cnt, up
+// to total), that of word t at dst[place(t)]
+template <int U, typename Place>
+__device__ __forceinline__ void words_settle(const unsigned long long *src, int cnt, int total, int epoch,
+                                             unsigned long long (&w)[U], unsigned *dst, const Place &place, int *err)
+{
+    long long it = 0;
+    for (;;) {
+        bool late = false;
+#pragma unroll
+        for (int u = 0; u < U; ++u) late = late || ((int)threadIdx.x + kTrsvT * u < cnt && (int)(unsigned)w[u] != epoch);
+        if (!late) break;
+        if (++it > kTrsvSpin) {
+            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            break;
+        }
+        // once a wait has given up, the others do not wait out their own limits
+        if ((it & 63) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
+        __builtin_amdgcn_s_sleep(1);
+        words_fetch<U>(src, cnt, w);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int t = threadIdx.x + kTrsvT * u;
+        if (t < total) dst[place(t)] = t < cnt ? (unsigned)(w[u] >> 32) : 0u;
+    }
+}
+
+// Sum over the eight lanes 8 m .. 8 m + 7 of a value, in each of them: DPP quad_perm 1,0,3,2
+// and 2,3,0,1 make each quad uniform, then the half-row mirror adds the other quad.
+template <int CTRL>
+__device__ __forceinline__ float dpp_lane(float v)
+{
+    const int i = __float_as_int(v);
+    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, CTRL, 0xF, 0xF, false));
+}
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_lane(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = (int)b, hi = (int)(b >> 32);
+    const int l2 = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false);
+    const int h2 = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false);
+    return __longlong_as_double(((long long)h2 << 32) | (unsigned)l2);
+}
+
+template <typename T>
+__device__ __forceinline__ T sum8_lanes(T v)
+{
+    v += dpp_lane<0xB1>(v);
+    v += dpp_lane<0x4E>(v);
+    v += dpp_lane<0x141>(v);
+    return v;
+}
+
+__device__ __forceinline__ double lane_value(double v, int l)   // l uniform
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// FP64: blocks of 64 rows.  Thread (row t / 8, c8 = t % 8) holds of a 64 x 64 block the
+// columns c8 + 8 j (j < 8); eight lanes read 128 bytes of a row at once.  Two blocks are in
+// flight per workgroup, and the products with all solved blocks stay in the lanes until one
+// sum over a row's eight at the end.  Then wave q substitutes column q in the diagonal block,
+// a row per lane, the solved entry going round by readlane (no LDS and no division in the
+// chain: the diagonal block lies in LDS by columns, U's reciprocals are formed before the wait).
+// Bound by the chain of blocks, about 6 us each.  One triangle, before (a launch per block with
+// a serial sweep through LDS) and now: 17,406 unknowns 12.6 -> 1.7 ms, 702 unknowns 420 -> 62 us.
+constexpr int kBlk64Chunks = kTB / 8, kBlk64Ld = kTB + 1;
+static_assert(kTrsvT == 8 * kTB, "a row of a block is eight threads");
+static_assert(kMaxRhs <= kTrsvT / 64, "a wave per right-hand side");
+using Blk64Regs = double2[kBlk64Chunks];
+
+__device__ __forceinline__ void blk64_load(const double2 *Mx, long long ld, int rs, int cs, Blk64Regs &a)
+{
+    const int r = threadIdx.x >> 3, c8 = threadIdx.x & 7;
+    const double2 *row = Mx + (long long)min(r, rs - 1) * ld;
+#pragma unroll
+    for (int j = 0; j < kBlk64Chunks; ++j) a[j] = c8 + 8 * j < cs ? row[c8 + 8 * j] : double2{0.0, 0.0};
+}
+
+// a + v into a, the rounding error added to e
+__device__ __forceinline__ void add_two(double &a, double &e, double v)
+{
+    const double s = a + v, t = s - a;
+    e += (a - (s - t)) + (v - t);
+    a = s;
+}
+
+// acc[q] += this thread's part of its row times column q of x.  A block's part is summed by
+// itself first (one sum over all of a row's blocks would round at its full size at every
+// entry), and what the sum over the blocks rounds off is kept in low[q].
+template <int NRHS>
+__device__ __forceinline__ void blk64_acc(const Blk64Regs &a, const double2 *x, double2 (&acc)[NRHS], double2 (&low)[NRHS])
+{
+    const int c8 = threadIdx.x & 7;
+#pragma unroll
+    for (int q = 0; q < NRHS; ++q) {
+        double2 v{0.0, 0.0};
+#pragma unroll
+        for (int j = 0; j < kBlk64Chunks; ++j) v = cfma_x(v, a[j], x[(c8 + 8 * j) * NRHS + q]);
+        add_two(acc[q].x, low[q].x, v.x);
+        add_two(acc[q].y, low[q].y, v.y);
+        // else the sums sink below the loads that follow, all of x waits in registers, and they spill
+        asm volatile("" : "+v"(acc[q].x), "+v"(acc[q].y)::"memory");
+    }
+}
+
+template <bool LOWER, int NRHS>
+__global__ __launch_bounds__(kTrsvT) void k_trsv64(const double2 *A, long long lda, int n, double2 *X,
+                                                   unsigned long long *sync, int ticket0, int epoch)
+{
+    constexpr int kUnits = kTB * NRHS * 4, kU = (kUnits + kTrsvT - 1) / kTrsvT;
+    __shared__ double2 D[kTB * kBlk64Ld];   // D[j kBlk64Ld + i]: row i, column j
+    __shared__ double2 xs[kTB * NRHS];
+    __shared__ double2 xb[2][kTB * NRHS];
+    __shared__ int s_idx;
+    int *counter = (int *)sync, *err = counter + 1;
+    unsigned long long *xw = sync + kTrsvHead;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nblk = (n + kTB - 1) / kTB;
+    for (;;) {
+        __syncthreads();   // the previous block's LDS reads are done
+        if (tid == 0) s_idx = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - ticket0;
+        __syncthreads();
+        const int idx = s_idx;
+        if (idx < 0 || idx >= nblk) return;   // no block left
+        const int r0 = (LOWER ? idx : nblk - 1 - idx) * kTB, rs = min(kTB, n - r0);
+        // dependency d < idx: the block solved d-th
+        auto first = [&](int d) { return (LOWER ? d : nblk - 1 - d) * kTB; };
+        auto load = [&](int d, Blk64Regs &a) { blk64_load(A + (long long)r0 * lda + first(d), lda, rs, min(kTB, n - first(d)), a); };
+        unsigned long long w[kU];
+        auto fetch = [&](int d) { words_fetch<kU>(xw + (size_t)first(d) * NRHS * 4, min(kTB, n - first(d)) * NRHS * 4, w); };
+        Blk64Regs ra, rb;
+        if (idx > 0) fetch(0);
+        if (idx > 0) load(0, ra);
+        if (idx > 1) load(1, rb);
+        for (int e = tid; e < kTB * kTB; e += kTrsvT) {
+            const int i = e / kTB, j = e % kTB;
+            D[j * kBlk64Ld + i] = i < rs && j < rs ? A[(long long)(r0 + i) * lda + r0 + j] : double2{0.0, 0.0};
+        }
+        for (int t = tid; t < kTB * NRHS; t += kTrsvT) xs[t] = t < rs * NRHS ? X[(long long)r0 * NRHS + t] : double2{0.0, 0.0};
+        __syncthreads();
+        double2 rinv{1.0, 0.0};
+        if (!LOWER && lane < rs) {
+            const double2 d = D[lane * kBlk64Ld + lane];
+            const double den = d.x * d.x + d.y * d.y;
+            rinv = {d.x / den, -d.y / den};
+        }
+        double2 acc[NRHS], low[NRHS];
+#pragma unroll
+        for (int q = 0; q < NRHS; ++q) acc[q] = low[q] = {0.0, 0.0};
+        auto one = [&](int d, Blk64Regs &a, double2 *x) {
+            const int c0 = first(d), cnt = min(kTB, n - c0) * NRHS * 4;
+            const unsigned long long *src = xw + (size_t)c0 * NRHS * 4;
+            words_settle<kU>(src, cnt, kUnits, epoch, w, (unsigned *)x, [](int t) { return t; }, err);
+            __syncthreads();
+            if (d + 1 < idx) fetch(d + 1);
+            blk64_acc<NRHS>(a, x, acc, low);
+            if (d + 2 < idx) load(d + 2, a);
+        };
+        for (int d = 0; d < idx; d += 2) {
+            one(d, ra, xb[0]);
+            if (d + 1 < idx) one(d + 1, rb, xb[1]);
+        }
+        if (idx > 0) {
+            const int r = tid >> 3, c8 = tid & 7;
+#pragma unroll
+            for (int q = 0; q < NRHS; ++q) {
+                const double2 v{sum8_lanes(acc[q].x), sum8_lanes(acc[q].y)};
+                const double2 w8{sum8_lanes(low[q].x), sum8_lanes(low[q].y)};
+                if (c8 == q) {
+                    xs[r * NRHS + q].x = (xs[r * NRHS + q].x - v.x) - w8.x;
+                    xs[r * NRHS + q].y = (xs[r * NRHS + q].y - v.y) - w8.y;
                 }
-                if (lane == 0) {
-                    V v = csubv(xs[i * nrhs + r], prod);
-                    if (!LOWER) {
-                        const V d = D[i][i];
-                        const T den = d.x * d.x + d.y * d.y;
-                        v = {(v.x * d.x + v.y * d.y) / den, (v.y * d.x - v.x * d.y) / den};
-                    }
-                    xs[i * nrhs + r] = v;
+            }
+            __syncthreads();
+        }
+        if (wid < NRHS) {
+            // x: the solved entries, b - t before (t from zero: as in blk64_acc)
+            const double2 b = xs[lane * NRHS + wid];
+            double2 x = b, t{0.0, 0.0};
+            if constexpr (LOWER) {
+#pragma unroll 8
+                for (int s = 0; s < rs - 1; ++s) {
+                    t = cfma_x(t, D[s * kBlk64Ld + lane], double2{lane_value(x.x, s), lane_value(x.y, s)});
+                    if (lane > s) x = csubv(b, t);
                 }
-                // LDS accesses of one wave complete in order; the shuffle above already
-                // orders lane 0's read after every lane's product
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            } else {
+                x = double2{fma(b.x, rinv.x, -(b.y * rinv.y)), fma(b.x, rinv.y, b.y * rinv.x)};
+#pragma unroll 8
+                for (int s = rs - 1; s > 0; --s) {
+                    t = cfma_x(t, D[s * kBlk64Ld + lane], double2{lane_value(x.x, s), lane_value(x.y, s)});
+                    const double2 u = csubv(b, t);
+                    if (lane < s) x = double2{fma(u.x, rinv.x, -(u.y * rinv.y)), fma(u.x, rinv.y, u.y * rinv.x)};
+                }
+            }
+            if (lane < rs) {
+                const size_t o = (size_t)(r0 + lane) * NRHS + wid;
+                const unsigned long long bx = (unsigned long long)__double_as_longlong(x.x),
+                                         by = (unsigned long long)__double_as_longlong(x.y), tag = (unsigned)epoch;
+                put_word(xw + 4 * o, (bx << 32) | tag);
+                put_word(xw + 4 * o + 1, (bx & 0xffffffff00000000ull) | tag);
+                put_word(xw + 4 * o + 2, (by << 32) | tag);
+                put_word(xw + 4 * o + 3, (by & 0xffffffff00000000ull) | tag);
+                X[o] = x;
             }
         }
     }
-    __syncthreads();
-}
-
-template <typename T, bool LOWER>
-__global__ __launch_bounds__(256) void k_trsv_first(const typename CT<T>::t *A, long long lda, int n,
-                                                    typename CT<T>::t *X, int nrhs, int blk)
-{
-    using V = typename CT<T>::t;
-    __shared__ V xs[kTB * kMaxRhs];
-    __shared__ V D[kTB][kTB + 1];
-    const int b0 = blk * kTB, bs = min(kTB, n - b0);
-    for (int t = threadIdx.x; t < bs * nrhs; t += blockDim.x) xs[t] = X[(long long)b0 * nrhs + t];
-    __syncthreads();
-    trsv_diag<T, LOWER>(A, lda, n, xs, nrhs, blk, D);
-    for (int t = threadIdx.x; t < bs * nrhs; t += blockDim.x) X[(long long)b0 * nrhs + t] = xs[t];
-}
-
-// Update the rows of the blocks after (LOWER) / before (upper) block `blk` with
-// its solved values; workgroup 0 owns the next block, keeps its rows in LDS and
-// then solves that diagonal block.
-template <typename T, bool LOWER>
-__global__ __launch_bounds__(256) void k_trsv_step(const typename CT<T>::t *A, long long lda, int n,
-                                                   typename CT<T>::t *X, int nrhs, int blk, int nblk)
-{
-    using V = typename CT<T>::t;
-    __shared__ V xs[kTB * kMaxRhs];
-    __shared__ V xb[kTB * kMaxRhs];
-    __shared__ V D[kTB][kTB + 1];
-    const int next = LOWER ? blk + 1 : blk - 1;
-    const int ch = LOWER ? next + (int)blockIdx.x : next - (int)blockIdx.x;
-    if (ch < 0 || ch >= nblk) return;   // uniform per workgroup
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int c0 = blk * kTB, cs = min(kTB, n - c0);
-    const int r0 = ch * kTB, rs = min(kTB, n - r0);
-    for (int t = threadIdx.x; t < cs * nrhs; t += blockDim.x) xb[t] = X[(long long)c0 * nrhs + t];
-    for (int t = threadIdx.x; t < rs * nrhs; t += blockDim.x) xs[t] = X[(long long)r0 * nrhs + t];
-    __syncthreads();
-    for (int i = wv; i < rs; i += 4) {
-        const V a = lane < cs ? A[(long long)(r0 + i) * lda + c0 + lane] : V{0, 0};
-        for (int r = 0; r < nrhs; ++r) {
-            V prod = lane < cs ? cmulv(a, xb[lane * nrhs + r]) : V{0, 0};
-            for (int off = 32; off >= 1; off >>= 1) {
-                prod.x += __shfl_xor(prod.x, off, 64);
-                prod.y += __shfl_xor(prod.y, off, 64);
-            }
-            if (lane == 0) xs[i * nrhs + r] = csubv(xs[i * nrhs + r], prod);
-        }
-    }
-    __syncthreads();
-    if (blockIdx.x == 0) trsv_diag<T, LOWER>(A, lda, n, xs, nrhs, next, D);
-    for (int t = threadIdx.x; t < rs * nrhs; t += blockDim.x) X[(long long)r0 * nrhs + t] = xs[t];
 }
 
 // ---------------------------------------------------------------- FP32 solves with inverted diagonal blocks
 // The FP32 factors only precondition GMRES-IR, so their triangular solves use
 // explicit inverses of the 128 x 128 diagonal blocks (computed once per
 // factorisation): each block step is then two small matrix-vector products with
-// no serial sweep, one launch per block.
+// no serial sweep.
 constexpr int kIB = 128;
 constexpr int kTrinvParts = 4;   // lanes per column in k_trinv
 
@@ -2003,90 +2148,76 @@ __global__ __launch_bounds__(kIB * kTrinvParts) void k_trinv(const float2 *A, lo
     trinv_body<LOWER>(A, lda, n, Dinv, blockIdx.x);
 }
 
-// out[i] = (SUB ? out[i] : 0) - / + sum_c Mx[i][c] xin[c] for rows i < rs, columns
-// c < cs (xin, out: distinct LDS vectors, row-major x nrhs).  The kTrsvT threads of a
-// workgroup hold the 128 x 128 block in registers, loaded at once (one memory round
-// trip per block instead of one per entry): thread t (wave w, lane l) takes the rows
-// (kTrsvT / 8) p + 8 w + l / 8 (p < kBlkRows) and of each the 16-byte chunks
-// l % 8 + 8 j (j < 8), i.e. the columns 2 (l % 8 + 8 j) and the one after.  Eight
-// lanes read one 128-byte line of a row, so each load of a wave touches 8 cache
-// lines (a layout with a row per lane touches 64, and the vector memory pipeline
-// then takes four times as long over the block); the eight lanes of a row then sum
-// their parts by DPP within the half-row.
-constexpr int kTrsvT = 512, kBlkRowStep = kTrsvT / 8, kBlkRows = kIB / kBlkRowStep, kBlkChunks = 8;
+// The kTrsvT threads of a workgroup hold a 128 x 128 block in registers, loaded at once (one
+// memory round trip per block instead of one per entry): thread t (wave w, lane l) takes the
+// rows (kTrsvT / 8) p + 8 w + l / 8 (p < kBlkRows) and of each the 16-byte chunks
+// l % 8 + 8 j (j < 8), i.e. the columns 2 (l % 8 + 8 j) and the one after.  Eight lanes read
+// one 128-byte line of a row, so each load of a wave touches 8 cache lines (a layout with a
+// row per lane touches 64, and the vector memory pipeline then takes four times as long over
+// the block); the eight lanes of a row then sum their parts by DPP within the half-row.
+constexpr int kBlkRowStep = kTrsvT / 8, kBlkRows = kIB / kBlkRowStep, kBlkChunks = 8;
 static_assert(kBlkRows * kBlkRowStep == kIB, "rows of a block split evenly over the threads");
 using BlkRegs = float4[kBlkRows][kBlkChunks];
 
-__device__ __forceinline__ void blk_load(const float2 *Mx, long long ld, int rs, int cs, BlkRegs &a)
+// Rows r < rs and columns c < cs of Mx (1 <= rs, cs <= 128), zeros elsewhere.  Every load is
+// issued, from rows and columns that are there (the last row again; the columns up to 64 or,
+// with wide, 128: rows are padded to multiples of 64), so that nothing but an incomplete block
+// waits for its values here.
+__device__ __forceinline__ void blk_load(const float2 *Mx, long long ld, int rs, int cs, bool wide, BlkRegs &a)
 {
     const int t = threadIdx.x, w = t >> 6, l = t & 63, rl = 8 * w + (l >> 3), c8 = l & 7;
-    if (rs == kIB && cs == kIB) {
+    const float2 *M2 = Mx + (wide ? kIB / 2 : 0);
 #pragma unroll
-        for (int p = 0; p < kBlkRows; ++p) {
-            const float4 *row4 = (const float4 *)(Mx + (long long)(kBlkRowStep * p + rl) * ld);   // 16-byte aligned: ld and block origins are multiples of 64
+    for (int p = 0; p < kBlkRows; ++p) {
+        const long long o = (long long)min(kBlkRowStep * p + rl, rs - 1) * ld + 2 * c8;   // 16-byte aligned
 #pragma unroll
-            for (int j = 0; j < kBlkChunks; ++j) a[p][j] = row4[c8 + 8 * j];
-        }
-    } else {
+        for (int j = 0; j < kBlkChunks; ++j)
+            a[p][j] = *(const float4 *)((j < kBlkChunks / 2 ? Mx : M2) + o + 16 * (j % (kBlkChunks / 2)));
+    }
+    if (rs < kIB || cs < kIB) {
 #pragma unroll
-        for (int p = 0; p < kBlkRows; ++p) {
-            const int r = kBlkRowStep * p + rl;
-            const float2 *row = Mx + (long long)min(r, max(rs - 1, 0)) * ld;
+        for (int p = 0; p < kBlkRows; ++p)
 #pragma unroll
             for (int j = 0; j < kBlkChunks; ++j) {
-                const int c = 2 * (c8 + 8 * j);
-                const float2 u = (r < rs && c < cs) ? row[c] : float2{0, 0};
-                const float2 v = (r < rs && c + 1 < cs) ? row[c + 1] : float2{0, 0};
-                a[p][j] = float4{u.x, u.y, v.x, v.y};
+                const int r = kBlkRowStep * p + rl, c = 2 * (c8 + 8 * j);
+                if (r >= rs || c >= cs) a[p][j].x = a[p][j].y = 0.f;
+                if (r >= rs || c + 1 >= cs) a[p][j].z = a[p][j].w = 0.f;
             }
-        }
     }
 }
 
-// Sum over the eight lanes 8 m .. 8 m + 7 of a value: DPP quad_perm 1,0,3,2 and
-// 2,3,0,1 make each quad uniform, then the half-row mirror adds the other quad.
-__device__ __forceinline__ float sum8_lanes(float v)
-{
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v),
-                                                               0xB1, 0xF, 0xF, false));
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v),
-                                                               0x4E, 0xF, 0xF, false));
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v),
-                                                               0x141, 0xF, 0xF, false));
-    return v;
-}
-
+// acc[p][q] += (SUB: -=) this thread's part of row p times column q of xin (LDS, [NRHS][kIB]: a
+// row pair in one 16-byte read, the eight lanes' reads on different banks);
+// a: the thread's share of the block, in registers (stride 1) or in LDS (stride kTrsvT)
 template <bool SUB, int NRHS>
-__device__ __forceinline__ void blk_apply(const BlkRegs &a, int rs, const float2 *xin, float2 *out)
+__device__ __forceinline__ void blk_acc(const float4 *a, int stride, const float2 *xin, float2 (&acc)[kBlkRows][NRHS])
 {
-    const int t = threadIdx.x, w = t >> 6, l = t & 63, rl = 8 * w + (l >> 3), c8 = l & 7;
+    const int c8 = threadIdx.x & 7;
 #pragma unroll
     for (int q = 0; q < NRHS; ++q) {
-        float2 acc[kBlkRows];
+        float2 v[kBlkRows];
 #pragma unroll
-        for (int p = 0; p < kBlkRows; ++p) acc[p] = {0, 0};
+        for (int p = 0; p < kBlkRows; ++p) v[p] = {0, 0};
 #pragma unroll
         for (int j = 0; j < kBlkChunks; ++j) {
             const int c = 2 * (c8 + 8 * j);
-            const float2 x0 = xin[c * NRHS + q], x1 = xin[(c + 1) * NRHS + q];
+            const float4 x01 = *(const float4 *)(xin + q * kIB + c);
+            const float2 x0{x01.x, x01.y}, x1{x01.z, x01.w};
 #pragma unroll
             for (int p = 0; p < kBlkRows; ++p) {   // explicit FMAs: the same bits for every NRHS
-                const float4 m = a[p][j];
-                acc[p].x = fmaf(-m.w, x1.y, fmaf(m.z, x1.x, fmaf(-m.y, x0.y, fmaf(m.x, x0.x, acc[p].x))));
-                acc[p].y = fmaf(m.w, x1.x, fmaf(m.z, x1.y, fmaf(m.y, x0.x, fmaf(m.x, x0.y, acc[p].y))));
+                const float4 m = a[(p * kBlkChunks + j) * stride];
+                v[p].x = fmaf(-m.w, x1.y, fmaf(m.z, x1.x, fmaf(-m.y, x0.y, fmaf(m.x, x0.x, v[p].x))));
+                v[p].y = fmaf(m.w, x1.x, fmaf(m.z, x1.y, fmaf(m.y, x0.x, fmaf(m.x, x0.y, v[p].y))));
             }
         }
 #pragma unroll
         for (int p = 0; p < kBlkRows; ++p) {
-            const float2 v{sum8_lanes(acc[p].x), sum8_lanes(acc[p].y)};
-            const int i = kBlkRowStep * p + rl;
-            if (c8 == 0 && i < rs) {
-                float2 &o = out[i * NRHS + q];
-                o = SUB ? float2{o.x - v.x, o.y - v.y} : v;
-            }
+            float2 &o = acc[p][q];
+            o = SUB ? float2{o.x - v[p].x, o.y - v[p].y} : float2{o.x + v[p].x, o.y + v[p].y};
+            // else the sums sink below the loads that follow, all of xin waits in registers, and they spill
+            asm volatile("" : "+v"(o.x), "+v"(o.y)::"memory");
         }
     }
-    __syncthreads();
 }
 
 // G[i] = Dinv[i] M[i][i -/+ 1] for the blocks with a neighbour (LOWER: the
@@ -2141,120 +2272,124 @@ __global__ __launch_bounds__(256) void k_blk_coupling(const float2 *A, long long
     blk_coupling_body<LOWER>(A, lda, n, Dinv, G, blockIdx.x, blockIdx.y);
 }
 
-// One launch per triangle, one workgroup per CU.  A workgroup takes a block in the
-// order of a ticket counter, solves it and takes the next, until none is left (so a
-// block never waits for a workgroup that has not started: every block it waits for
-// has an earlier ticket, held by a running workgroup).  Block i subtracts the
-// products with the blocks it depends on as their ready flags appear, applies its
-// inverted diagonal block and publishes its rows with a ready flag (agent scope
-// release / acquire).  A wait that exceeds kTrsvSpin polls sets the error word and
-// gives up, so every workgroup ends.  Tickets handed out per launch: the blocks plus
-// one final ticket per workgroup.
-constexpr long long kTrsvSpin = 1LL << 24;
-
+// FP32: blocks of 128 rows.  Block i subtracts the products with the blocks it depends on as
+// their rows appear, two blocks of the factor in flight, the sums kept in the lanes until one
+// sum over a row's eight; then x = Dinv b - G x_adjacent, with the coupling G to the adjacent
+// block loaded and Dinv b formed before the adjacent rows are waited for, so that the chain
+// from block to block is one exchange and one product.  Bound by that chain, and at 40,000
+// unknowns by the reads of the factor.  One triangle, before (ready flags between fences) and
+// now: 39,996 unknowns, one column 2.75 -> 1.42 ms (4.5 TB/s); 12,000, four columns 0.85 ->
+// 0.51 ms; 4050, two columns 0.16 -> 0.12 ms.
 template <bool LOWER, int NRHS>
 __global__ __launch_bounds__(kTrsvT) void k_trsv_flag(const float2 *A, long long lda, int n, const float2 *Dinv,
-                                                      const float2 *G, float2 *X, int *sync, int ticket0, int epoch)
+                                                      const float2 *G, float2 *X, unsigned long long *sync,
+                                                      int ticket0, int epoch)
 {
-    __shared__ float2 xs[kIB * NRHS];
-    __shared__ float2 xb[kIB * NRHS];
+    constexpr int kUnits = kIB * NRHS * 2, kU = (kUnits + kTrsvT - 1) / kTrsvT;
+    __shared__ __align__(16) float2 xs[kIB * NRHS];   // [NRHS][kIB]
+    __shared__ __align__(16) float2 xb[2][kIB * NRHS];
     // the inverted diagonal block, each thread's share at a place of its own (read back
     // by the thread that wrote it: no barrier, no bank conflicts)
     __shared__ float4 dsh[kBlkRows][kBlkChunks][kTrsvT];
-    __shared__ int s_idx, s_ready;
-    int *counter = sync, *err = sync + 1, *flag = sync + 2;
-    const int nblk = (n + kIB - 1) / kIB;
+    __shared__ int s_idx;
+    int *counter = (int *)sync, *err = counter + 1;
+    unsigned long long *xw = sync + kTrsvHead;
+    const int tid = threadIdx.x, nblk = (n + kIB - 1) / kIB;
+    const int rl = 8 * (tid >> 6) + ((tid & 63) >> 3), c8 = tid & 7;
     for (;;) {
         __syncthreads();   // the previous block's LDS reads are done
-        if (threadIdx.x == 0)
-            s_idx = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - ticket0;
+        if (tid == 0) s_idx = __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - ticket0;
         __syncthreads();
         const int idx = s_idx;
         if (idx < 0 || idx >= nblk) return;   // no block left
         const int blk = LOWER ? idx : nblk - 1 - idx;
         const int r0 = blk * kIB, rs = min(kIB, n - r0);
-        const int jadj = LOWER ? blk - 1 : blk + 1, cadj = jadj * kIB, csadj = min(kIB, n - cadj);
-        auto wait_flag = [&](int j) {   // thread 0
-            long long it = 0;
-            while (__hip_atomic_load(flag + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch) {
-                if (++it > kTrsvSpin) {
-                    __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    break;
-                }
-                // once a wait has given up, the others do not wait out their own limits
-                if ((it & 63) == 0 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
-                __builtin_amdgcn_s_sleep(1);
-            }
+        const int adj = idx - 1;   // dependency d: the block solved d-th; the last one is adjacent
+        auto first = [&](int d) { return (LOWER ? d : nblk - 1 - d) * kIB; };
+        auto load = [&](int d, BlkRegs &a) {
+            const int c0 = first(d), cs = min(kIB, n - c0);
+            const bool far = d < adj;
+            if (d <= adj) blk_load(far ? A + (long long)r0 * lda + c0 : G + (size_t)blk * kIB * kIB, far ? lda : kIB, rs, cs,
+                                   !far || c0 + kIB <= lda, a);
         };
-        // the block's own operands, held for the whole solve: the inverted diagonal block
-        // (LDS) and the coupling G to the adjacent block (registers), so that neither is
-        // loaded after a wait
-        BlkRegs a, g;
-        blk_load(Dinv + (size_t)blk * kIB * kIB, kIB, rs, rs, a);
-        if (idx > 0) blk_load(G + (size_t)blk * kIB * kIB, kIB, rs, csadj, g);
+        unsigned long long w[kU];
+        auto fetch = [&](int d) { words_fetch<kU>(xw + (size_t)first(d) * NRHS * 2, min(kIB, n - first(d)) * NRHS * 2, w); };
+        BlkRegs ra, rb;
+        blk_load(Dinv + (size_t)blk * kIB * kIB, kIB, rs, rs, true, ra);
 #pragma unroll
         for (int p = 0; p < kBlkRows; ++p)
 #pragma unroll
-            for (int j = 0; j < kBlkChunks; ++j) dsh[p][j][threadIdx.x] = a[p][j];
-        for (int t = threadIdx.x; t < kIB * NRHS; t += blockDim.x) xs[t] = t < rs * NRHS ? X[(long long)r0 * NRHS + t] : float2{0, 0};
+            for (int j = 0; j < kBlkChunks; ++j) dsh[p][j][tid] = ra[p][j];
+        if (idx > 0) fetch(0);
+        load(0, ra);
+        load(1, rb);
+        for (int t = tid; t < kIB * NRHS; t += kTrsvT)
+            xs[(t % NRHS) * kIB + t / NRHS] = t < rs * NRHS ? X[(long long)r0 * NRHS + t] : float2{0, 0};
         __syncthreads();
-        // every dependency but the adjacent block, taken as their ready flags appear; the
-        // next block of L (or U) is loaded before its flag is waited for
-        const int early = max(idx - 1, 0);
-        int done = 0;
-        auto load_early = [&](int d) {
-            const int c0 = (LOWER ? d : nblk - 1 - d) * kIB;
-            blk_load(A + (long long)r0 * lda + c0, lda, rs, min(kIB, n - c0), a);
-        };
-        if (early > 0) load_early(0);
-        while (done < early) {
-            if (threadIdx.x == 0) {
-                wait_flag(LOWER ? done : nblk - 1 - done);
-                // blocks publish in order, so every further flag already set is usable too
-                int ready = done + 1;
-                while (ready < early &&
-                       __hip_atomic_load(flag + (LOWER ? ready : nblk - 1 - ready), __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT) == epoch)
-                    ++ready;
-                __threadfence();   // acquire: the rows of those blocks
-                s_ready = ready;
-            }
-            __syncthreads();
-            const int ready = s_ready;
-            for (; done < ready; ++done) {
-                const int j = LOWER ? done : nblk - 1 - done;
-                const int c0 = j * kIB, cs = min(kIB, n - c0);
-                for (int t = threadIdx.x; t < kIB * NRHS; t += blockDim.x)
-                    xb[t] = t < cs * NRHS ? X[(long long)c0 * NRHS + t] : float2{0, 0};
-                __syncthreads();
-                blk_apply<true, NRHS>(a, rs, xb, xs);
-                if (done + 1 < early) load_early(done + 1);
-            }
-        }
-        // y = Dinv x without the adjacent block (into xb); then x = y - G x_adjacent
+        float2 acc[kBlkRows][NRHS];
 #pragma unroll
         for (int p = 0; p < kBlkRows; ++p)
 #pragma unroll
-            for (int j = 0; j < kBlkChunks; ++j) a[p][j] = dsh[p][j][threadIdx.x];
-        blk_apply<false, NRHS>(a, rs, xs, xb);
-        if (idx > 0) {
-            if (threadIdx.x == 0) {
-                wait_flag(jadj);
-                __threadfence();   // acquire: the adjacent block's rows
+            for (int q = 0; q < NRHS; ++q) acc[p][q] = {0, 0};
+        auto settle = [&](int d, float2 *x) {
+            words_settle<kU>(xw + (size_t)first(d) * NRHS * 2, min(kIB, n - first(d)) * NRHS * 2, kUnits, epoch, w, (unsigned *)x,
+                             [](int t) { return ((t >> 1) % NRHS * kIB + (t >> 1) / NRHS) * 2 + (t & 1); }, err);
+        };
+        auto one = [&](int d, BlkRegs &a, float2 *x) {
+            settle(d, x);
+            __syncthreads();
+            fetch(d + 1);
+            blk_acc<false, NRHS>(&a[0][0], 1, x, acc);
+            load(d + 2, a);
+        };
+        auto finish = [&](const BlkRegs &g, float2 *x) {   // the rest, with the coupling in g
+            if (adj > 0) {
+#pragma unroll
+                for (int p = 0; p < kBlkRows; ++p)
+#pragma unroll
+                    for (int q = 0; q < NRHS; ++q) {
+                        const float2 v{sum8_lanes(acc[p][q].x), sum8_lanes(acc[p][q].y)};
+                        if (c8 == q) {   // rows from rs on: zeros
+                            float2 &o = xs[q * kIB + kBlkRowStep * p + rl];
+                            o = {o.x - v.x, o.y - v.y};
+                        }
+                        acc[p][q] = {0, 0};
+                    }
+                __syncthreads();
             }
-            __syncthreads();
-            for (int t = threadIdx.x; t < kIB * NRHS; t += blockDim.x)
-                xs[t] = t < csadj * NRHS ? X[(long long)cadj * NRHS + t] : float2{0, 0};
-            __syncthreads();
-            blk_apply<true, NRHS>(g, rs, xs, xb);
+            blk_acc<false, NRHS>(&dsh[0][0][tid], kTrsvT, xs, acc);
+            if (adj >= 0) {
+                settle(adj, x);
+                __syncthreads();
+                blk_acc<true, NRHS>(&g[0][0], 1, x, acc);
+            }
+#pragma unroll
+            for (int p = 0; p < kBlkRows; ++p) {   // lane c8 of a row publishes column c8
+                float2 v{0, 0};
+#pragma unroll
+                for (int q = 0; q < NRHS; ++q) {
+                    const float2 u{sum8_lanes(acc[p][q].x), sum8_lanes(acc[p][q].y)};
+                    if (c8 == q) v = u;
+                }
+                const int i = kBlkRowStep * p + rl;
+                if (c8 < NRHS && i < rs) {
+                    const size_t o = (size_t)(r0 + i) * NRHS + c8;
+                    put_word(xw + 2 * o, ((unsigned long long)__float_as_uint(v.x) << 32) | (unsigned)epoch);
+                    put_word(xw + 2 * o + 1, ((unsigned long long)__float_as_uint(v.y) << 32) | (unsigned)epoch);
+                    X[o] = v;
+                }
+            }
+        };
+        int d = 0;
+        for (; d + 1 < adj; d += 2) {
+            one(d, ra, xb[0]);
+            one(d + 1, rb, xb[1]);
         }
-        // wave 0 writes the rows, so that thread 0's release fence covers every store (a
-        // barrier does not wait for other waves' stores, and a fence orders its own wave's)
-        if (threadIdx.x < 64)
-            for (int t = threadIdx.x; t < rs * NRHS; t += 64) X[(long long)r0 * NRHS + t] = xb[t];
-        if (threadIdx.x == 0) {
-            __threadfence();   // release: this block's rows
-            __hip_atomic_store(flag + blk, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (d < adj) {
+            one(d, ra, xb[0]);
+            finish(rb, xb[1]);
+        } else {
+            finish(ra, xb[0]);
         }
     }
 }
@@ -2971,24 +3106,6 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
 }
 
 // forward (unit lower) then backward (upper) substitution on X (n x nrhs, work precision)
-template <typename T>
-void lu_solve_inplace(hipStream_t s, const typename CT<T>::t *A, long long lda, int n, typename CT<T>::t *X, int nrhs)
-{
-    const int nb = (n + kTB - 1) / kTB;
-    k_trsv_first<T, true><<<1, 256, 0, s>>>(A, lda, n, X, nrhs, 0);
-    check("k_trsv_first");
-    for (int b = 0; b + 1 < nb; ++b) {
-        k_trsv_step<T, true><<<nb - 1 - b, 256, 0, s>>>(A, lda, n, X, nrhs, b, nb);
-        check("k_trsv_step");
-    }
-    k_trsv_first<T, false><<<1, 256, 0, s>>>(A, lda, n, X, nrhs, nb - 1);
-    check("k_trsv_first");
-    for (int b = nb - 1; b > 0; --b) {
-        k_trsv_step<T, false><<<b, 256, 0, s>>>(A, lda, n, X, nrhs, b, nb);
-        check("k_trsv_step");
-    }
-}
-
 // Inverses of the diagonal blocks of both FP32 factors: Dinv[0 .. nb) lower, [nb .. 2nb) upper.
 void invert_diagonal_blocks(hipStream_t s, const float2 *LU, long long lda, int n, float2 *Dinv)
 {
@@ -3004,7 +3121,6 @@ void invert_diagonal_blocks(hipStream_t s, const float2 *LU, long long lda, int 
     check("k_blk_coupling");
 }
 
-// Synchronisation words of the one-launch triangular solves of one matrix.
 // words[0 .. cnt) = 0 (a kernel rather than a memset node, for callers that capture graphs)
 __global__ void k_fill_int(int *words, long long cnt)
 {
@@ -3012,47 +3128,57 @@ __global__ void k_fill_int(int *words, long long cnt)
     if (i < cnt) words[i] = 0;
 }
 
-struct TrsvSync {
-    int *words;           // [0] ticket counter, [1] error flag, [2 ..] ready flags
-    long long &tickets;   // tickets handed out so far
-    int &epoch;           // ready-flag value of the last triangle
-    int cus;              // workgroups of a launch at most (one per CU)
-};
+// The words of one matrix's triangular solves: kTrsvHead, then 2 (FP32) or 4 (FP64) per value.
+size_t trsv_words(int64_t n, bool fp64) { return kTrsvHead + (size_t)n * kMaxRhs * (fp64 ? 4 : 2); }
 
-template <int NRHS>
-void lu_solve_inv_n(hipStream_t s, const float2 *A, long long lda, int n, const float2 *Dinv, float2 *X, TrsvSync &ts)
+void trsv_restart(hipStream_t s, bh_matrix *M)
 {
-    const int nb = (n + kIB - 1) / kIB;
-    const size_t bsz = (size_t)nb * kIB * kIB;
-    const float2 *DL = Dinv, *DU = Dinv + bsz, *GL = Dinv + 2 * bsz, *GU = Dinv + 3 * bsz;
+    const long long cnt = 2 * (long long)M->tsync.n;
+    k_fill_int<<<(unsigned)((cnt + 255) / 256), 256, 0, s>>>((int *)M->tsync.p, cnt);
+    check("k_fill_int");
+    M->tsync_tickets = 0;
+    M->tsync_epoch = 0;
+}
+
+// X := U^-1 L^-1 X with the factors of M, X device n x NRHS row-major
+template <typename T, int NRHS>
+void lu_solve_n(hipStream_t s, bh_matrix *M, typename CT<T>::t *X)
+{
+    constexpr bool kF64 = std::is_same<T, double>::value;
+    const int n = (int)M->n, nb = kF64 ? (n + kTB - 1) / kTB : (n + kIB - 1) / kIB;
+    const int grid = std::max(1, std::min(nb, M->ctx->num_cus));   // one workgroup per CU at most
     for (int tri = 0; tri < 2; ++tri) {
-        if (ts.tickets + 2LL * nb >= (1LL << 30) || ts.epoch >= (1 << 30)) {   // restart the counters
-            k_fill_int<<<(unsigned)((nb + 2 + 255) / 256), 256, 0, s>>>(ts.words, nb + 2);
-            check("k_fill_int");
-            ts.tickets = 0;
-            ts.epoch = 0;
+        if (M->tsync_tickets + 2LL * nb >= (1LL << 30) || M->tsync_epoch >= (1 << 30)) trsv_restart(s, M);
+        const int ticket0 = (int)M->tsync_tickets, epoch = ++M->tsync_epoch;
+        M->tsync_tickets += nb + grid;
+        if constexpr (kF64) {
+            const double2 *A = (const double2 *)M->lu64.p;
+            if (tri == 0) k_trsv64<true, NRHS><<<grid, kTrsvT, 0, s>>>(A, M->lda, n, X, M->tsync.p, ticket0, epoch);
+            else k_trsv64<false, NRHS><<<grid, kTrsvT, 0, s>>>(A, M->lda, n, X, M->tsync.p, ticket0, epoch);
+            check("k_trsv64");
+        } else {
+            const float2 *A = (const float2 *)M->lu32.p, *DL = (const float2 *)M->dinv32.p;
+            const size_t bsz = (size_t)nb * kIB * kIB;
+            const float2 *DU = DL + bsz, *GL = DL + 2 * bsz, *GU = DL + 3 * bsz;
+            if (tri == 0) k_trsv_flag<true, NRHS><<<grid, kTrsvT, 0, s>>>(A, M->lda, n, DL, GL, X, M->tsync.p, ticket0, epoch);
+            else k_trsv_flag<false, NRHS><<<grid, kTrsvT, 0, s>>>(A, M->lda, n, DU, GU, X, M->tsync.p, ticket0, epoch);
+            check("k_trsv_flag");
         }
-        const int grid = std::max(1, std::min(nb, ts.cus));
-        const int ticket0 = (int)ts.tickets, epoch = ++ts.epoch;
-        ts.tickets += nb + grid;
-        if (tri == 0) k_trsv_flag<true, NRHS><<<grid, kTrsvT, 0, s>>>(A, lda, n, DL, GL, X, ts.words, ticket0, epoch);
-        else k_trsv_flag<false, NRHS><<<grid, kTrsvT, 0, s>>>(A, lda, n, DU, GU, X, ts.words, ticket0, epoch);
-        check("k_trsv_flag");
     }
 }
 
-void lu_solve_inv(hipStream_t s, const float2 *A, long long lda, int n, const float2 *Dinv, float2 *X, int nrhs,
-                  TrsvSync &ts)
+template <typename T>
+void lu_solve(hipStream_t s, bh_matrix *M, typename CT<T>::t *X, int nrhs)
 {
     switch (nrhs) {
-    case 1: lu_solve_inv_n<1>(s, A, lda, n, Dinv, X, ts); break;
-    case 2: lu_solve_inv_n<2>(s, A, lda, n, Dinv, X, ts); break;
-    case 3: lu_solve_inv_n<3>(s, A, lda, n, Dinv, X, ts); break;
-    case 4: lu_solve_inv_n<4>(s, A, lda, n, Dinv, X, ts); break;
-    case 5: lu_solve_inv_n<5>(s, A, lda, n, Dinv, X, ts); break;
-    case 6: lu_solve_inv_n<6>(s, A, lda, n, Dinv, X, ts); break;
-    case 7: lu_solve_inv_n<7>(s, A, lda, n, Dinv, X, ts); break;
-    case 8: lu_solve_inv_n<8>(s, A, lda, n, Dinv, X, ts); break;
+    case 1: lu_solve_n<T, 1>(s, M, X); break;
+    case 2: lu_solve_n<T, 2>(s, M, X); break;
+    case 3: lu_solve_n<T, 3>(s, M, X); break;
+    case 4: lu_solve_n<T, 4>(s, M, X); break;
+    case 5: lu_solve_n<T, 5>(s, M, X); break;
+    case 6: lu_solve_n<T, 6>(s, M, X); break;
+    case 7: lu_solve_n<T, 7>(s, M, X); break;
+    case 8: lu_solve_n<T, 8>(s, M, X); break;
     default: BH_FAIL(BH_ERR_INVALID, "nrhs %d out of range", nrhs);
     }
 }
@@ -3505,16 +3631,10 @@ void fp32_prepare(Ctx &ctx, bh_matrix *M, long long lda)
 void factor_finish(Ctx &ctx, bh_matrix *M, long long lda, int precision, int info)
 {
     const int64_t n = M->n;
-    if (precision != BH_FP64) {
-        if (M->x32.n < (size_t)n * kMaxRhs * 2) M->x32.alloc((size_t)n * kMaxRhs * 2);
-        const size_t nflags = (size_t)((n + kIB - 1) / kIB) + 2;
-        if (M->tsync.n < nflags) {
-            M->tsync.alloc(nflags);
-            k_fill_int<<<(unsigned)((nflags + 255) / 256), 256, 0, ctx.stream>>>(M->tsync.p, (long long)nflags);
-            check("k_fill_int");
-            M->tsync_tickets = 0;
-            M->tsync_epoch = 0;
-        }
+    if (precision != BH_FP64 && M->x32.n < (size_t)n * kMaxRhs * 2) M->x32.alloc((size_t)n * kMaxRhs * 2);
+    if (M->tsync.n < trsv_words(n, precision == BH_FP64)) {
+        pool_alloc(ctx, M->tsync, trsv_words(n, precision == BH_FP64));
+        trsv_restart(ctx.stream, M);
     }
     std::vector<long long> ip(n);
     BH_CHECK_HIP(hipMemcpy(ip.data(), M->ipiv.p, sizeof(long long) * n, hipMemcpyDeviceToHost));
@@ -3709,24 +3829,15 @@ void apply_factors(bh_matrix *M, const double2 *B, double2 *Xd, int nrhs)
     if (M->factored == BH_FP64) {
         k_permute_in<double><<<g, 256, 0, s>>>(B, n, nrhs, M->perm.p, Xd);
         check("k_permute_in");
-        lu_solve_inplace<double>(s, (const double2 *)M->lu64.p, M->lda, n, Xd, nrhs);
+        ProfScope prof(*M->ctx, "k_trsv64", 16.0 * n * (double)n);   // one read of both factors
+        lu_solve<double>(s, M, Xd, nrhs);
     } else {
-        if (M->x32.n < (size_t)cnt * 2) M->x32.alloc((size_t)n * kMaxRhs * 2);
         float2 *x32 = (float2 *)M->x32.p;
         k_permute_in<float><<<g, 256, 0, s>>>(B, n, nrhs, M->perm.p, x32);
         check("k_permute_in");
         {
-            const int nb = (n + kIB - 1) / kIB;
-            if (M->tsync.n < (size_t)nb + 2) {
-                M->tsync.alloc((size_t)nb + 2);
-                k_fill_int<<<(unsigned)((nb + 2 + 255) / 256), 256, 0, s>>>(M->tsync.p, (long long)nb + 2);
-                check("k_fill_int");
-                M->tsync_tickets = 0;
-                M->tsync_epoch = 0;
-            }
-            TrsvSync ts{M->tsync.p, M->tsync_tickets, M->tsync_epoch, M->ctx->num_cus};
             ProfScope prof(*M->ctx, "k_trsv_inv", 8.0 * n * (double)n);   // one read of both FP32 factors
-            lu_solve_inv(s, (const float2 *)M->lu32.p, M->lda, n, (const float2 *)M->dinv32.p, x32, nrhs, ts);
+            lu_solve<float>(s, M, x32, nrhs);
         }
         k_widen<float><<<g, 256, 0, s>>>(x32, cnt, Xd);
         check("k_widen");
@@ -3997,22 +4108,18 @@ void solve_impl(bh_matrix *M, int64_t nrhs, const double *B, double *X, double t
     double res = 0;
     std::vector<double> bn(q);
     for (int r = 0; r < q; ++r) bn[r] = host_norm(hb, n, q, r);
-    // the FP32 triangular solves report a block wait that gave up in tsync[1]; it is
+    // the triangular solves report a block wait that gave up in the error word; it is
     // read (and cleared) after every synchronisation that ends a use of the solves,
     // before anything derived from their results is judged
     auto check_trsv = [&]() {
-        if (M->factored != BH_FP32 || !M->tsync.p) return;
         int trsv_err = 0;
-        BH_CHECK_HIP(hipMemcpyAsync(&trsv_err, M->tsync.p + 1, sizeof(int), hipMemcpyDeviceToHost, s));
+        BH_CHECK_HIP(hipMemcpyAsync(&trsv_err, (int *)M->tsync.p + 1, sizeof(int), hipMemcpyDeviceToHost, s));
         BH_CHECK_HIP(hipStreamSynchronize(s));
         if (!trsv_err) return;
         // results are void; the counters restart
-        k_fill_int<<<(unsigned)((M->tsync.n + 255) / 256), 256, 0, s>>>(M->tsync.p, (long long)M->tsync.n);
-        check("k_fill_int");
+        trsv_restart(s, M);
         BH_CHECK_HIP(hipStreamSynchronize(s));
-        M->tsync_tickets = 0;
-        M->tsync_epoch = 0;
-        BH_FAIL(BH_ERR_HIP, "FP32 triangular solve: a block wait exceeded its limit");
+        BH_FAIL(BH_ERR_HIP, "triangular solve: a block wait exceeded its limit");
     };
     const bool refine = M->factored == BH_FP32 || tol > 0;
     if (refine) {
@@ -4130,10 +4237,10 @@ extern "C" int bh_matrix_solve_noalloc(bh_matrix *M, int64_t nrhs, const double 
     BH_REQUIRE(M && B && X, "NULL argument");
     BH_REQUIRE(M->factored == BH_FP64 || M->factored == BH_FP32, "matrix is not factored");
     BH_REQUIRE(nrhs >= 1 && nrhs <= 8, "nrhs must be 1..8");
-    // apply_factors allocates nothing when bh_matrix_factor has sized these buffers
-    BH_REQUIRE(M->factored == BH_FP64 ||
-                   (M->x32.n >= (size_t)M->n * nrhs * 2 && M->tsync.n >= (size_t)((M->n + kIB - 1) / kIB) + 2),
-               "FP32 factors without their solve buffers");
+    // apply_factors allocates nothing: bh_matrix_factor has sized these buffers
+    BH_REQUIRE((M->factored == BH_FP64 || M->x32.n >= (size_t)M->n * nrhs * 2) &&
+                   M->tsync.n >= trsv_words(M->n, M->factored == BH_FP64),
+               "factors without their solve buffers");
     const size_t need = solve_work_layout((int)M->n, (int)nrhs, nullptr, nullptr);
     BH_REQUIRE(need <= kScratchBytes,
                "bh_matrix_solve_noalloc: n = %lld with %lld right-hand sides needs %zu bytes of scratch, more than "
