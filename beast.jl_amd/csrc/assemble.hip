@@ -802,7 +802,7 @@ struct FarArgs {
     int Qo, Qi;
     int mode;
     double k2;
-    int shifted;                  // FP64, lossless: phases taken relative to the centroid distance
+    int shifted;                  // FP64, lossless: phases taken relative to the centroid distance (level of cos_sinc)
     const int *nptr;              // CSR of non-far pairs per test cell
     const int4 *nent;
     const double *nblk;           // 18 doubles per entry
@@ -822,11 +822,56 @@ struct RowStage {
     int rc;               // the test cell's place in the tile
 };
 
+// cos(sqrt u) and sin(sqrt u) / sqrt u on 0 <= u <= kShiftMax[LEVEL - 1]^2 by their Taylor
+// series, to u^6, to u^8 and u^7 (as sincos_f64), and to u^10; the remainders stay below 1e-17,
+// 5e-17 and 3e-17.  Levels, since a step of both is two of about sixty operations per point
+// pair; Taylor coefficients, since those of sincos_f64 are in scalar registers already
+// (polynomials of the same length with coefficients of their own: 63 -> 70 ms at 26,664 cells).
+constexpr int kShiftLevels = 3;
+constexpr double kShiftMax[kShiftLevels] = {0.369, 0.785, 1.55};
+
+template <int LEVEL, typename R>
+__device__ __forceinline__ void cos_sinc(R u, R &c, R &s)
+{
+    if constexpr (LEVEL == 1) {
+        c = (R)(1.0 / 479001600.0);
+        s = (R)(1.0 / 6227020800.0);
+    } else {
+        if constexpr (LEVEL == 2) {
+            c = (R)(1.0 / 20922789888000.0);
+            s = (R)(-1.0 / 1307674368000.0);
+        } else {
+            c = (R)(1.0 / 2432902008176640000.0);
+            s = (R)(1.0 / 51090942171709440000.0);
+            c = c * u - (R)(1.0 / 6402373705728000.0);
+            s = s * u - (R)(1.0 / 121645100408832000.0);
+            c = c * u + (R)(1.0 / 20922789888000.0);
+            s = s * u + (R)(1.0 / 355687428096000.0);
+            s = s * u - (R)(1.0 / 1307674368000.0);
+        }
+        c = c * u - (R)(1.0 / 87178291200.0);
+        s = s * u + (R)(1.0 / 6227020800.0);
+        c = c * u + (R)(1.0 / 479001600.0);
+    }
+    c = c * u - (R)(1.0 / 3628800.0);
+    s = s * u - (R)(1.0 / 39916800.0);
+    c = c * u + (R)(1.0 / 40320.0);
+    s = s * u + (R)(1.0 / 362880.0);
+    c = c * u - (R)(1.0 / 720.0);
+    s = s * u - (R)(1.0 / 5040.0);
+    c = c * u + (R)(1.0 / 24.0);
+    s = s * u + (R)(1.0 / 120.0);
+    c = c * u - (R)0.5;
+    s = s * u - (R)(1.0 / 6.0);
+    c = c * u + (R)1;
+    s = s * u + (R)1;
+}
+
 // Far-field 3x3 block of (test p, trial q) by double Gauss, written to z[k*stride].
 // QO, QI: the point counts when fixed at compile time (0: read from A).
 // maybe_near = false: the caller knows the pair is not in p's non-far list.
 // STAGED: the test cell's data come from st (LDS) instead of A's arrays.
-template <typename R, int OPK, int QO = 0, int QI = 0, bool SHIFT = false, bool STAGED = false>
+template <typename R, int OPK, int QO = 0, int QI = 0, int SHIFT = 0, bool STAGED = false>
 __device__ __forceinline__ void far_block(const FarArgs &A, int p, int q, cx<R> *z, int stride, bool maybe_near = true,
                                           RowStage<R> st = {})
 {
@@ -866,10 +911,9 @@ __device__ __forceinline__ void far_block(const FarArgs &A, int p, int q, cx<R> 
     };
     const R gr = (R)A.op.gr, gi = (R)A.op.gi;
     // shifted: exp(-i gi R) = exp(-i gi Rc) exp(-i gi (R - Rc)), Rc the centroid distance,
-    // the second factor by its Taylor series (|gi (R - Rc)| <= |gi| (r_p + r_q), bounded on
-    // the host so that the series' remainder stays below 1e-17)
+    // the second factor by polynomials (|gi (R - Rc)| <= |gi| (r_p + r_q), bounded on the host)
     R cc = (R)1, sc = (R)0, rc = (R)0;
-    constexpr bool shifted = SHIFT && sizeof(R) == 8;
+    constexpr bool shifted = SHIFT > 0 && sizeof(R) == 8;
     if constexpr (shifted) {
         rc = sqrt(dc[0] * dc[0] + dc[1] * dc[1] + dc[2] * dc[2]);
         double s_, c_;
@@ -880,19 +924,9 @@ __device__ __forceinline__ void far_block(const FarArgs &A, int p, int q, cx<R> 
     auto kernel_g = [&](R dist, R idist) -> cx<R> {
         if constexpr (!shifted) return green<R>(gr, gi, dist, idist);
         const R t = gi * (dist - rc), u = t * t;
-        // cos t = sum (-1)^k u^k / (2k)!, sin t = t sum (-1)^k u^k / (2k+1)!, k <= 6
-        R pc = (R)(1.0 / 479001600.0), ps = (R)(1.0 / 6227020800.0);
-        pc = pc * u - (R)(1.0 / 3628800.0);
-        ps = ps * u - (R)(1.0 / 39916800.0);
-        pc = pc * u + (R)(1.0 / 40320.0);
-        ps = ps * u + (R)(1.0 / 362880.0);
-        pc = pc * u - (R)(1.0 / 720.0);
-        ps = ps * u - (R)(1.0 / 5040.0);
-        pc = pc * u + (R)(1.0 / 24.0);
-        ps = ps * u + (R)(1.0 / 120.0);
-        pc = pc * u - (R)0.5;
-        ps = ps * u - (R)(1.0 / 6.0);
-        const R ct = pc * u + (R)1, st = t * (ps * u + (R)1);
+        R ct, st;
+        cos_sinc<SHIFT>(u, ct, st);
+        st *= t;
         const R amp = idist * (R)kInv4Pi;
         // exp(-i gi (R - Rc)) / (4 pi R); the pair's common factor exp(-i gi Rc) = cc - i sc
         // multiplies its moments once (rot below), every quantity summed being linear in G
@@ -1156,7 +1190,7 @@ struct FarTileLds {
     static constexpr size_t kBytes = kBlk + kStageBytes > kT ? kBlk + kStageBytes : kT;
 };
 
-template <typename R, int OPK, bool ROWMAJOR, int QO, int QI, bool SHIFT = false>
+template <typename R, int OPK, bool ROWMAJOR, int QO, int QI, int SHIFT = 0>
 __device__ void far_tiles_dev(const TileArgs &A, int tr, int tc)
 {
     using L = FarTileLds<R, OPK, QO, ROWMAJOR>;
@@ -1341,7 +1375,7 @@ __global__ __launch_bounds__(kTileCells) void k_pack_rows(const int *__restrict_
 template <int OPK>
 constexpr int far_min_blocks() { return OPK == BH_OP_MW_DOUBLELAYER_ROTATED ? 2 : 1; }
 
-template <typename R, int OPK, bool ROWMAJOR, int QO, int QI, bool SHIFT = false>
+template <typename R, int OPK, bool ROWMAJOR, int QO, int QI, int SHIFT = 0>
 __global__ __launch_bounds__(256, far_min_blocks<OPK>()) void k_far_tiles(TileArgs A)
 {
     far_tiles_dev<R, OPK, ROWMAJOR, QO, QI, SHIFT>(A, blockIdx.y, blockIdx.x);
@@ -1682,12 +1716,11 @@ struct Plan {
     long long nft = 0, nfs = 0;
 };
 
-// Lossless FP64: phases relative to the centroid distance when |gi| (r_p + r_q) stays below
-// 0.369, where the degree-12/13 Taylor remainders of cos and sin are below 1e-17 (r: the
-// largest vertex-to-centroid distance of each mesh).
-bool shifted_phases(const OpParams &op, const Mesh &tm, const Mesh &sm, bool fp32)
+// Lossless FP64: phases relative to the centroid distance when |gi| (r_p + r_q) (r: the largest
+// vertex-to-centroid distance of each mesh) is within kShiftMax: the level of cos_sinc, 0 for none.
+int shifted_phases(const OpParams &op, const Mesh &tm, const Mesh &sm, bool fp32)
 {
-    if (fp32 || op.gr != 0.0) return false;
+    if (fp32 || op.gr != 0.0) return 0;
     auto radius = [](const Mesh &m) {
         double r = 0.0;
         for (int64_t c = 0; c < m.nf; ++c) {
@@ -1700,7 +1733,9 @@ bool shifted_phases(const OpParams &op, const Mesh &tm, const Mesh &sm, bool fp3
         return r;
     };
     const double th = std::fabs(op.gi) * (radius(tm) + radius(sm)) * (1.0 + 1e-12);
-    return th <= 0.369;
+    for (int l = 0; l < kShiftLevels; ++l)
+        if (th <= kShiftMax[l]) return l + 1;
+    return 0;
 }
 
 void make_plan(Ctx &ctx, const bh_operator *op, const bh_quadstrat *qs, Mesh &tm, Mesh &sm, bool fp32, Plan &P)
@@ -1722,7 +1757,7 @@ void make_plan(Ctx &ctx, const bh_operator *op, const bh_quadstrat *qs, Mesh &tm
     F.sq = quad_points(sm, P.st.far_i, &F.Qi, fp32, ctx.stream);
     F.mode = P.st.mode;
     F.k2 = P.op.gr * P.op.gr + P.op.gi * P.op.gi;
-    F.shifted = shifted_phases(P.op, tm, sm, fp32) ? 1 : 0;
+    F.shifted = shifted_phases(P.op, tm, sm, fp32);
     F.nptr = P.nd.nptr.p;
     F.nent = P.nd.entries.p;
     F.nblk = P.nd.blocks.p;
@@ -1768,11 +1803,14 @@ void launch_tiles(Ctx &ctx, const Plan &P, Space &X, Space &Y, void *Z, long lon
     // unrolled point loops
     const bool dflt = P.far.Qo == 3 && P.far.Qi == 4;
     // the centroid-shifted phases (FP64, lossless, small cells) for the default rules
-    const bool shift = sizeof(R) == 8 && dflt && P.far.shifted;
+    constexpr int kL1 = sizeof(R) == 8 ? 1 : 0, kL2 = 2 * kL1, kL3 = 3 * kL1;
+    const int shift = sizeof(R) == 8 && dflt ? P.far.shifted : 0;
     if (sl && dflt) A.rpack = pack_rows<R>(ctx.stream, X, P.far, rpack);
 #define BH_TILES(OPK, RM)                                                                    \
     do {                                                                                     \
-        if (shift) k_far_tiles<R, OPK, RM, 3, 4, true><<<grid, 256, 0, ctx.stream>>>(A);    \
+        if (shift == 1) k_far_tiles<R, OPK, RM, 3, 4, kL1><<<grid, 256, 0, ctx.stream>>>(A); \
+        else if (shift == 2) k_far_tiles<R, OPK, RM, 3, 4, kL2><<<grid, 256, 0, ctx.stream>>>(A); \
+        else if (shift == 3) k_far_tiles<R, OPK, RM, 3, 4, kL3><<<grid, 256, 0, ctx.stream>>>(A); \
         else if (dflt) k_far_tiles<R, OPK, RM, 3, 4><<<grid, 256, 0, ctx.stream>>>(A);      \
         else k_far_tiles<R, OPK, RM, 0, 0><<<grid, 256, 0, ctx.stream>>>(A);                \
     } while (0)
@@ -1782,10 +1820,12 @@ void launch_tiles(Ctx &ctx, const Plan &P, Space &X, Space &Y, void *Z, long lon
         // generic loops
         constexpr int DLR = BH_OP_MW_DOUBLELAYER_ROTATED;
         const bool r67 = P.far.Qo == 12 && P.far.Qi == 13;
-        const bool s67 = sizeof(R) == 8 && r67 && P.far.shifted;
+        const int s67 = sizeof(R) == 8 && r67 ? P.far.shifted : 0;
 #define BH_TILES_DLR(RM)                                                                     \
     do {                                                                                     \
-        if (s67) k_far_tiles<R, DLR, RM, 12, 13, true><<<grid, 256, 0, ctx.stream>>>(A);    \
+        if (s67 == 1) k_far_tiles<R, DLR, RM, 12, 13, kL1><<<grid, 256, 0, ctx.stream>>>(A); \
+        else if (s67 == 2) k_far_tiles<R, DLR, RM, 12, 13, kL2><<<grid, 256, 0, ctx.stream>>>(A); \
+        else if (s67 == 3) k_far_tiles<R, DLR, RM, 12, 13, kL3><<<grid, 256, 0, ctx.stream>>>(A); \
         else if (r67) k_far_tiles<R, DLR, RM, 12, 13><<<grid, 256, 0, ctx.stream>>>(A);     \
         else k_far_tiles<R, DLR, RM, 0, 0><<<grid, 256, 0, ctx.stream>>>(A);                \
     } while (0)
@@ -2005,7 +2045,7 @@ __global__ __launch_bounds__(256) void k_wilton_batch(const BatchNear *reqs, con
 
 // dof tiles of several requests of one kernel configuration; tile t of a request is
 // (row t / column tiles, column t mod column tiles)
-template <typename R, int OPK, bool ROWMAJOR, int QO, int QI, bool SHIFT = false>
+template <typename R, int OPK, bool ROWMAJOR, int QO, int QI, int SHIFT = 0>
 __global__ __launch_bounds__(256, far_min_blocks<OPK>()) void k_far_tiles_batch(const TileArgs *args, const int *first,
                                                                                  int n)
 {
@@ -2184,12 +2224,12 @@ void batch_far(Ctx &ctx, std::vector<BatchItem> &items)
     for (int i = 0; i < (int)items.size(); ++i) {
         BatchItem &it = items[i];
         if (it.X->ndofs == 0) continue;
-        // 0 generic rules, 1 and 2 the default far rules (3 x 4 points) without and with
-        // shifted phases, 3 and 4 the rotated double layer's default (12 x 13 points)
+        // 0 generic rules, 1 to 4 the default far rules (3 x 4 points), 5 to 8 the rotated double
+        // layer's default (12 x 13 points), each without and with shifted phases of level 1 to 3
         const bool rot = it.op.kind == BH_OP_MW_DOUBLELAYER_ROTATED;
         const bool dflt = it.far.Qo == 3 && it.far.Qi == 4 && !rot;
         const bool r67 = it.far.Qo == 12 && it.far.Qi == 13 && rot;
-        const int variant = dflt ? (it.far.shifted ? 2 : 1) : (r67 ? (it.far.shifted ? 4 : 3) : 0);
+        const int variant = dflt ? 1 + it.far.shifted : (r67 ? 5 + it.far.shifted : 0);
         Group *g = nullptr;
         for (auto &gg : groups)
             if (gg.opk == it.op.kind && gg.variant == variant) g = &gg;
@@ -2222,7 +2262,7 @@ void batch_far(Ctx &ctx, std::vector<BatchItem> &items)
             A.accumulate = 0;
             A.scale_r = 1.0;
             A.scale_i = 0.0;
-            if (g.opk == BH_OP_MW_SINGLELAYER && (g.variant == 1 || g.variant == 2)) {
+            if (g.opk == BH_OP_MW_SINGLELAYER && g.variant >= 1 && g.variant <= 4) {
                 keep.emplace_back();
                 A.rpack = pack_rows<double>(s, X, it.far, keep.back());
             }
@@ -2241,16 +2281,22 @@ void batch_far(Ctx &ctx, std::vector<BatchItem> &items)
         const unsigned grid = (unsigned)first[n];
 #define BH_BTILES(OPK)                                                                                           \
     do {                                                                                                         \
-        if (g.variant == 2) k_far_tiles_batch<double, OPK, true, 3, 4, true><<<grid, 256, 0, s>>>(da, df, n);    \
+        if (g.variant == 4) k_far_tiles_batch<double, OPK, true, 3, 4, 3><<<grid, 256, 0, s>>>(da, df, n);       \
+        else if (g.variant == 3) k_far_tiles_batch<double, OPK, true, 3, 4, 2><<<grid, 256, 0, s>>>(da, df, n);  \
+        else if (g.variant == 2) k_far_tiles_batch<double, OPK, true, 3, 4, 1><<<grid, 256, 0, s>>>(da, df, n);  \
         else if (g.variant == 1) k_far_tiles_batch<double, OPK, true, 3, 4><<<grid, 256, 0, s>>>(da, df, n);     \
         else k_far_tiles_batch<double, OPK, true, 0, 0><<<grid, 256, 0, s>>>(da, df, n);                         \
     } while (0)
         if (g.opk == BH_OP_MW_SINGLELAYER) BH_BTILES(BH_OP_MW_SINGLELAYER);
         else if (g.opk == BH_OP_MW_DOUBLELAYER) BH_BTILES(BH_OP_MW_DOUBLELAYER);
-        else if (g.variant == 4)
-            k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 12, 13, true><<<grid, 256, 0, s>>>(da, df, n);
-        else if (g.variant == 3)
-            k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 12, 13><<<grid, 256, 0, s>>>(da, df, n);
+        else if (g.variant == 8)
+            k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 12, 13, 3><<<grid, 256, 0, s>>>(da, df, n);
+        else if (g.variant == 7)
+            k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 12, 13, 2><<<grid, 256, 0, s>>>(da, df, n);
+        else if (g.variant == 6)
+            k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 12, 13, 1><<<grid, 256, 0, s>>>(da, df, n);
+        else if (g.variant == 5)
+            k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 12, 13, 0><<<grid, 256, 0, s>>>(da, df, n);
         else k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 0, 0><<<grid, 256, 0, s>>>(da, df, n);
 #undef BH_BTILES
         check_launch("k_far_tiles_batch");
@@ -2395,7 +2441,7 @@ void assemble_resident_batch(bh_ctx *ctx, int64_t count, const bh_operator *ops,
         F.sq = quad_points(m, it.st.far_i, &F.Qi, false, ctx->stream);
         F.mode = it.st.mode;
         F.k2 = it.op.gr * it.op.gr + it.op.gi * it.op.gi;
-        F.shifted = shifted_phases(it.op, m, m, false) ? 1 : 0;
+        F.shifted = shifted_phases(it.op, m, m, false);
         F.op = it.op;
         std::unique_ptr<bh_matrix> M(new bh_matrix());
         M->ctx = ctx;

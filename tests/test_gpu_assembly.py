@@ -244,3 +244,24 @@ def test_grid_classification_large_meshes(bj, orc, k):
     Ys = Y.subset(np.arange(0, Y.numfunctions(), 13))
     for op in _ops(bj, k):
         assert relfro(bj.assemble(op, Xs, Ys), _oracle_Z(orc, op, qs, Xs, Ys)) < 1e-12
+
+
+@pytest.mark.parametrize("level", [0.369, 0.785, 1.55])
+@pytest.mark.parametrize("side", [0.3, 0.999, 1.001])
+def test_shifted_phases_at_their_limits(bj, orc, golden, level, side):
+    """Lossless FP64 phases relative to the centroid distance: wavenumbers that put
+    k (r_p + r_q) within, just within and just beyond each polynomial's range, all operators,
+    host and resident matrices.  Entries of dofs more than 0.6 apart (far pairs alone): 1e-13,
+    for the rounding of up to 4 x 156 terms each."""
+    m = _mesh(bj, golden, "sphere45.in")
+    X = bj.raviartthomas(m)
+    t = m.vertices[m.cells]
+    r = np.sqrt(((t - t.mean(axis=1, keepdims=True)) ** 2).sum(-1)).max()
+    far = np.linalg.norm(X.pos[:, None] - X.pos[None], axis=-1) > 0.6
+    k = side * level / (2 * r)
+    for kind, op in [(0, bj.Maxwell3D.singlelayer(wavenumber=k)), (1, bj.Maxwell3D.doublelayer(wavenumber=k)),
+                     (3, bj.DoubleLayerRotatedMW3D(1.0, 1j * k))]:
+        qs = bj.defaultquadstrat(op, X, X)
+        Zo = orc.assemble(kind, op.gamma, op.alpha, op.beta if kind == 0 else 0.0, qs.kind, qs.params, X, X)
+        assert relfro(bj.assemble(op, X, X)[far], Zo[far]) < 1e-13
+        assert relfro(bj.DeviceMatrix.assemble(op, X).download()[far], Zo[far]) < 1e-13
