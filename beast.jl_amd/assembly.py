@@ -253,7 +253,7 @@ def assemble_rhs(field, X, quadstrat=defaultquadstrat, ctx=None):
     a = np.array([E.amplitude.real, E.amplitude.imag])
     with ctx.lock:
         nat.check(lib.bh_assemble_excitation(ctx.handle, space_handle(X, ctx), trace, nat.dptr(d), nat.dptr(pr),
-                                             nat.dptr(pi), nat.dptr(g), nat.dptr(a), int(qs.quad_rule), 1,
+                                             nat.dptr(pi), nat.dptr(g), nat.dptr(a), int(qs.quad_rule), 0,
                                              b.ctypes.data_as(nat._D)))
     return b
 

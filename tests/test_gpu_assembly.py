@@ -265,3 +265,25 @@ def test_shifted_phases_at_their_limits(bj, orc, golden, level, side):
         Zo = orc.assemble(kind, op.gamma, op.alpha, op.beta if kind == 0 else 0.0, qs.kind, qs.params, X, X)
         assert relfro(bj.assemble(op, X, X)[far], Zo[far]) < 1e-13
         assert relfro(bj.DeviceMatrix.assemble(op, X).download()[far], Zo[far]) < 1e-13
+
+
+@pytest.mark.parametrize("degree", [1, 2, 8, 10])
+@pytest.mark.parametrize("trace", ["tangential", "cross"])
+def test_excitation_rules_and_accumulation(bj, orc, golden, degree, trace):
+    """Rules of 1 to 25 points (fewer and more than a dof's 32 lanes take at once), lossy, against
+    the oracle (1e-13: up to 50 terms per entry); what the caller's vector holds is added to."""
+    X = bj.raviartthomas(_mesh(bj, golden, "sphere45.in"))
+    nat, ctx = bj._native, bj.assembly.default_context()
+    args = [np.array(x, float) for x in ([0, 0, 1], [1, 0, 0], [0, 0, 0], [0.3, 2.0], [2.0, 0])]
+
+    def run(b, accumulate):
+        nat.check(nat.load().bh_assemble_excitation(
+            ctx.handle, bj.assembly.space_handle(X, ctx), nat.TRACE_CROSS if trace == "cross" else nat.TRACE_TANGENTIAL,
+            *[nat.dptr(a) for a in args], degree, accumulate, b.ctypes.data_as(nat._D)))
+        return b
+
+    b = run(np.full(X.numfunctions(), np.nan + 0j), 0)
+    bo = orc.planewave(X, [0, 0, 1.0], [1.0, 0, 0], 0.3 + 2.0j, amplitude=2.0, degree=degree, trace=trace)
+    assert relfro(b, bo) < 1e-13
+    v = np.arange(2.0 * X.numfunctions()).view(np.complex128)
+    assert np.array_equal(run(v.copy(), 1), v + b)
