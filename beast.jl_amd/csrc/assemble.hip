@@ -324,7 +324,7 @@ __device__ __forceinline__ cx<R> green(R gr, R gi, R dist, R idist)
 // all moments folded into alpha and beta
 template <typename R>
 __device__ __forceinline__ void efie_block(const OpParams &op, R s1, const R *a, const R *b, cx<R> M0, const cx<R> *Mx,
-                                          const cx<R> *My, cx<R> Mxy, cx<R> *z, int stride, cx<R> ph = {1, 0})
+                                          const cx<R> *My, cx<R> Mxy, cx<R> *z, long long stride, cx<R> ph = {1, 0})
 {
     const cx<R> sa = cmul(ph, cx<R>{s1 * (R)op.ar, s1 * (R)op.ai});
     const cx<R> bM0 = cmul(cmul(cx<R>{(R)op.br, (R)op.bi}, M0), ph);
@@ -872,7 +872,7 @@ __device__ __forceinline__ void cos_sinc(R u, R &c, R &s)
 // maybe_near = false: the caller knows the pair is not in p's non-far list.
 // STAGED: the test cell's data come from st (LDS) instead of A's arrays.
 template <typename R, int OPK, int QO = 0, int QI = 0, int SHIFT = 0, bool STAGED = false>
-__device__ __forceinline__ void far_block(const FarArgs &A, int p, int q, cx<R> *z, int stride, bool maybe_near = true,
+__device__ __forceinline__ void far_block(const FarArgs &A, int p, int q, cx<R> *z, long long stride, bool maybe_near = true,
                                           RowStage<R> st = {})
 {
     const int Qo = QO ? QO : A.Qo, Qi = QI ? QI : A.Qi;
@@ -1154,6 +1154,12 @@ struct TileArgs {
     int accumulate;
     double scale_r, scale_i;
     const void *rpack;    // the row tiles' test cells packed field by field (single layer, default rule)
+    // tiles gathered from pair blocks (k_pair_blocks): the blocks, the place of each tile's test
+    // cells in their group, the group's padded number of test cells, its first row tile
+    const void *pblk;
+    const int *rloc;
+    long long npp;
+    int nfs, tr0;
 };
 
 // v of lane l (l wave-uniform)
@@ -1190,10 +1196,12 @@ struct FarTileLds {
     static constexpr size_t kBytes = kBlk + kStageBytes > kT ? kBlk + kStageBytes : kT;
 };
 
-template <typename R, int OPK, bool ROWMAJOR, int QO, int QI, int SHIFT = 0>
+// LOADED: the pair blocks come from A.pblk
+template <typename R, int OPK, bool ROWMAJOR, int QO, int QI, int SHIFT = 0, bool LOADED = false>
 __device__ void far_tiles_dev(const TileArgs &A, int tr, int tc)
 {
     using L = FarTileLds<R, OPK, QO, ROWMAJOR>;
+    static_assert(!LOADED || QO == 0, "loaded tiles have no rule");
     constexpr bool kStage = L::kStage;
     constexpr int kChunk = L::kChunk;
     __shared__ int s_rc[kTileCells], s_cc[kTileCells];
@@ -1211,7 +1219,7 @@ __device__ void far_tiles_dev(const TileArgs &A, int tr, int tc)
     const int c0 = A.col.ptr[tc], nc = A.col.ptr[tc + 1] - c0;
     const int mbase = tr * kTile, nbase = tc * kTile;
     for (int k = tid; k < nr; k += 256) {
-        const int p = A.row.cells[r0 + k];
+        const int p = LOADED ? A.rloc[r0 + k] : A.row.cells[r0 + k];
         s_rc[k] = p;
         if constexpr (kStage) {
             const double *tg = A.far.tgeo + (size_t)p * kGeo;
@@ -1245,7 +1253,7 @@ __device__ void far_tiles_dev(const TileArgs &A, int tr, int tc)
     // mark the tile's non-far pairs: each row cell's non-far list (ascending trial
     // cells) looked up in the sorted column cells, so that far pairs skip the
     // search of far_block
-    const bool lists = A.far.mode != kModeDoubleNum;
+    const bool lists = !LOADED && A.far.mode != kModeDoubleNum;
     if (lists) {
         for (int rc = tid; rc < nr; rc += 256) {
             const int p = s_rc[rc];
@@ -1274,6 +1282,16 @@ __device__ void far_tiles_dev(const TileArgs &A, int tr, int tc)
 #pragma unroll 1
         for (int t = tid; t < nr * cn; t += 256) {
             const int rc = t % nr, cc = t / nr;
+            if constexpr (LOADED) {
+                const cx<R> *w = (const cx<R> *)A.pblk + (size_t)s_cc[cb + cc] * A.npp + s_rc[rc];
+                const size_t plane = (size_t)A.nfs * A.npp;
+                cx<R> v[9];
+#pragma unroll
+                for (int k = 0; k < 9; ++k) v[k] = w[k * plane];
+#pragma unroll
+                for (int k = 0; k < 9; ++k) s_blk[t + k * kChunk] = v[k];
+                continue;
+            }
             const int bit = rc * kTileCells + cb + cc;
             const bool near = lists && ((s_near[bit >> 5] >> (bit & 31)) & 1u);
             if constexpr (L::kPacked) {
@@ -1371,7 +1389,7 @@ __global__ __launch_bounds__(kTileCells) void k_pack_rows(const int *__restrict_
     for (int v = 0; v < 4 * Qo; ++v) pv[(9 + v) * kTileCells + k] = tq[(size_t)p * Qo * 4 + v];
 }
 
-// workgroups per CU the compiler must fit: two for n x K (see far_block), free otherwise
+// workgroups per CU the compiler must fit: two for n x K (its rules' loops are long), free otherwise
 template <int OPK>
 constexpr int far_min_blocks() { return OPK == BH_OP_MW_DOUBLELAYER_ROTATED ? 2 : 1; }
 
@@ -1379,6 +1397,28 @@ template <typename R, int OPK, bool ROWMAJOR, int QO, int QI, int SHIFT = 0>
 __global__ __launch_bounds__(256, far_min_blocks<OPK>()) void k_far_tiles(TileArgs A)
 {
     far_tiles_dev<R, OPK, ROWMAJOR, QO, QI, SHIFT>(A, blockIdx.y, blockIdx.x);
+}
+
+// Blocks of the pairs (test cell cells[i], trial cell q), i < ncells, q < nfs, once each:
+// block entry k at blk[(k nfs + q) npp + i].  A wave takes 64 test cells and one trial cell.
+// For the rotated double layer, whose 156 point pairs cost more than 144 bytes there and back: a
+// 64 x 64 tile that forms its own blocks shares its cells with its neighbours, and every block
+// was formed 1.8 times.  Bound by FP64 VALU issue.  6002 x 6002 cells: 14.5 ms, and 2.7 ms to
+// gather them, against 28.2 ms for tiles that form their own.
+template <typename R, int OPK, int QO, int QI, int SHIFT>
+__global__ __launch_bounds__(256, 2) void k_pair_blocks(FarArgs A, const int *__restrict__ cells, int ncells, int nfs,
+                                                        cx<R> *blk, long long npp)
+{
+    const int i = blockIdx.y * 64 + (threadIdx.x & 63);
+    const int q = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (q >= nfs || i >= ncells) return;
+    far_block<R, OPK, QO, QI, SHIFT>(A, cells[i], q, blk + (size_t)q * npp + i, (long long)nfs * npp);
+}
+
+template <typename R, bool ROWMAJOR>
+__global__ __launch_bounds__(256) void k_gather_tiles(TileArgs A)
+{
+    far_tiles_dev<R, BH_OP_MW_DOUBLELAYER_ROTATED, ROWMAJOR, 0, 0, 0, true>(A, A.tr0 + blockIdx.y, blockIdx.x);
 }
 
 // Far blocks for an explicit pair list (inspection entry).
@@ -1705,6 +1745,8 @@ void build_tiles(Space &sp, hipStream_t s)
     sp.t_coef.upload(coef.data(), coef.size(), s);
     sp.ntiles = nt;
     BH_CHECK_HIP(hipStreamSynchronize(s));
+    sp.h_tptr = std::move(ptr);
+    sp.h_tcells = std::move(cells);
     sp.tiles_built = true;
 }
 
@@ -1776,6 +1818,89 @@ const void *pack_rows(hipStream_t s, const Space &X, const FarArgs &F, DevBuf<ch
     return buf.p;
 }
 
+// The rotated double layer's default-rule tiles (12 x 13 points): pair blocks of a group of row
+// tiles (k_pair_blocks), then those tiles gathered from them, group by group.  A group's blocks
+// take at most kPairBlockBytes (a quarter of that, and so on, where memory is short) or what its
+// one row tile needs.
+constexpr size_t kPairBlockBytes = size_t(2) << 30;
+
+template <typename R>
+void pair_block_tiles(Ctx &ctx, TileArgs A, const Space &X, const Space &Y)
+{
+    constexpr int DLR = BH_OP_MW_DOUBLELAYER_ROTATED;
+    hipStream_t s = ctx.stream;
+    const long long nfs = Y.mesh->nf, nt = X.ntiles;
+    const size_t per_cell = (size_t)nfs * 9 * sizeof(cx<R>);
+    struct Group {
+        long long t0, t1;
+        int c0, n;
+    };
+    std::vector<Group> groups;
+    std::vector<int> cells, rloc(X.h_tcells.size());
+    PoolBuf<char> blk;
+    long long npp = 0;
+    for (size_t budget = kPairBlockBytes;; budget /= 4) {
+        groups.clear();
+        cells.clear();
+        npp = 0;
+        std::vector<int> at(X.mesh->nf, -1);   // place in the current group, offset by its first cell
+        for (long long t = 0; t < nt;) {
+            Group g{t, t, (int)cells.size(), 0};
+            for (; t < nt; ++t) {
+                int more = 0;
+                for (int k = X.h_tptr[t]; k < X.h_tptr[t + 1]; ++k) more += at[X.h_tcells[k]] < g.c0;
+                if (t > g.t0 && (size_t)((g.n + more + 63) / 64 * 64) * per_cell > budget) break;
+                for (int k = X.h_tptr[t]; k < X.h_tptr[t + 1]; ++k) {
+                    const int c = X.h_tcells[k];
+                    if (at[c] < g.c0) {
+                        at[c] = g.c0 + g.n++;
+                        cells.push_back(c);
+                    }
+                    rloc[k] = at[c] - g.c0;
+                }
+            }
+            g.t1 = t;
+            npp = std::max(npp, (long long)(g.n + 63) / 64 * 64);
+            groups.push_back(g);
+        }
+        try {
+            blk.alloc(ctx, (size_t)npp * per_cell);
+            break;
+        } catch (const Error &e) {
+            if (e.code != BH_ERR_OOM || (long long)groups.size() == nt) throw;
+            (void)hipGetLastError();
+        }
+    }
+    DevBuf<int> dcells, drloc;
+    dcells.upload(cells.data(), cells.size(), s);
+    drloc.upload(rloc.data(), rloc.size(), s);
+    A.pblk = blk.p;
+    A.rloc = drloc.p;
+    A.npp = npp;
+    A.nfs = (int)nfs;
+    const int shift = sizeof(R) == 8 ? A.far.shifted : 0;
+    constexpr int kL1 = sizeof(R) == 8 ? 1 : 0;
+    for (const Group &g : groups) {
+        const dim3 bg((unsigned)((nfs + 3) / 4), (unsigned)((g.n + 63) / 64));
+        const int *gc = dcells.p + g.c0;
+        cx<R> *w = (cx<R> *)blk.p;
+        if (g.n == 0 || nfs == 0) {
+            // dofs without shapes: zeros
+        } else if (shift == 1) k_pair_blocks<R, DLR, 12, 13, kL1><<<bg, 256, 0, s>>>(A.far, gc, g.n, (int)nfs, w, npp);
+        else if (shift == 2) k_pair_blocks<R, DLR, 12, 13, 2 * kL1><<<bg, 256, 0, s>>>(A.far, gc, g.n, (int)nfs, w, npp);
+        else if (shift == 3) k_pair_blocks<R, DLR, 12, 13, 3 * kL1><<<bg, 256, 0, s>>>(A.far, gc, g.n, (int)nfs, w, npp);
+        else k_pair_blocks<R, DLR, 12, 13, 0><<<bg, 256, 0, s>>>(A.far, gc, g.n, (int)nfs, w, npp);
+        check_launch("k_pair_blocks");
+        A.tr0 = (int)g.t0;
+        const dim3 tg((unsigned)Y.ntiles, (unsigned)(g.t1 - g.t0));
+        if (A.rowmajor) k_gather_tiles<R, true><<<tg, 256, 0, s>>>(A);
+        else k_gather_tiles<R, false><<<tg, 256, 0, s>>>(A);
+        check_launch("k_gather_tiles");
+    }
+    BH_CHECK_HIP(hipStreamSynchronize(s));   // the lists and the blocks go out of scope
+    blk.done();
+}
+
 template <typename R>
 void launch_tiles(Ctx &ctx, const Plan &P, Space &X, Space &Y, void *Z, long long ld, bool rowmajor, bool accumulate,
                   double sr, double si, DevBuf<char> &rpack, void *Z32 = nullptr, long long ld32 = 0)
@@ -1815,23 +1940,12 @@ void launch_tiles(Ctx &ctx, const Plan &P, Space &X, Space &Y, void *Z, long lon
         else k_far_tiles<R, OPK, RM, 0, 0><<<grid, 256, 0, ctx.stream>>>(A);                \
     } while (0)
     if (P.op.kind == BH_OP_MW_DOUBLELAYER_ROTATED) {
-        // its default rules (Dunavant degrees 6 and 7: 12 x 13 points) get unrolled inner
-        // point loops, with centroid-shifted phases where they apply; other rules the
-        // generic loops
+        // its default rules (Dunavant degrees 6 and 7: 12 x 13 points) form each pair's block
+        // once, with unrolled inner point loops; other rules take the generic loops
         constexpr int DLR = BH_OP_MW_DOUBLELAYER_ROTATED;
-        const bool r67 = P.far.Qo == 12 && P.far.Qi == 13;
-        const int s67 = sizeof(R) == 8 && r67 ? P.far.shifted : 0;
-#define BH_TILES_DLR(RM)                                                                     \
-    do {                                                                                     \
-        if (s67 == 1) k_far_tiles<R, DLR, RM, 12, 13, kL1><<<grid, 256, 0, ctx.stream>>>(A); \
-        else if (s67 == 2) k_far_tiles<R, DLR, RM, 12, 13, kL2><<<grid, 256, 0, ctx.stream>>>(A); \
-        else if (s67 == 3) k_far_tiles<R, DLR, RM, 12, 13, kL3><<<grid, 256, 0, ctx.stream>>>(A); \
-        else if (r67) k_far_tiles<R, DLR, RM, 12, 13><<<grid, 256, 0, ctx.stream>>>(A);     \
-        else k_far_tiles<R, DLR, RM, 0, 0><<<grid, 256, 0, ctx.stream>>>(A);                \
-    } while (0)
-        if (rowmajor) BH_TILES_DLR(true);
-        else BH_TILES_DLR(false);
-#undef BH_TILES_DLR
+        if (P.far.Qo == 12 && P.far.Qi == 13) pair_block_tiles<R>(ctx, A, X, Y);
+        else if (rowmajor) k_far_tiles<R, DLR, true, 0, 0><<<grid, 256, 0, ctx.stream>>>(A);
+        else k_far_tiles<R, DLR, false, 0, 0><<<grid, 256, 0, ctx.stream>>>(A);
     } else if (rowmajor) {
         if (sl) BH_TILES(BH_OP_MW_SINGLELAYER, true);
         else BH_TILES(BH_OP_MW_DOUBLELAYER, true);
@@ -2224,12 +2338,12 @@ void batch_far(Ctx &ctx, std::vector<BatchItem> &items)
     for (int i = 0; i < (int)items.size(); ++i) {
         BatchItem &it = items[i];
         if (it.X->ndofs == 0) continue;
-        // 0 generic rules, 1 to 4 the default far rules (3 x 4 points), 5 to 8 the rotated double
-        // layer's default (12 x 13 points), each without and with shifted phases of level 1 to 3
+        // 0 generic rules, 1 to 4 the default far rules (3 x 4 points) without and with shifted
+        // phases of level 1 to 3, 5 the rotated double layer's default (12 x 13 points)
         const bool rot = it.op.kind == BH_OP_MW_DOUBLELAYER_ROTATED;
         const bool dflt = it.far.Qo == 3 && it.far.Qi == 4 && !rot;
         const bool r67 = it.far.Qo == 12 && it.far.Qi == 13 && rot;
-        const int variant = dflt ? 1 + it.far.shifted : (r67 ? 5 + it.far.shifted : 0);
+        const int variant = dflt ? 1 + it.far.shifted : (r67 ? 5 : 0);
         Group *g = nullptr;
         for (auto &gg : groups)
             if (gg.opk == it.op.kind && gg.variant == variant) g = &gg;
@@ -2289,14 +2403,8 @@ void batch_far(Ctx &ctx, std::vector<BatchItem> &items)
     } while (0)
         if (g.opk == BH_OP_MW_SINGLELAYER) BH_BTILES(BH_OP_MW_SINGLELAYER);
         else if (g.opk == BH_OP_MW_DOUBLELAYER) BH_BTILES(BH_OP_MW_DOUBLELAYER);
-        else if (g.variant == 8)
-            k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 12, 13, 3><<<grid, 256, 0, s>>>(da, df, n);
-        else if (g.variant == 7)
-            k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 12, 13, 2><<<grid, 256, 0, s>>>(da, df, n);
-        else if (g.variant == 6)
-            k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 12, 13, 1><<<grid, 256, 0, s>>>(da, df, n);
         else if (g.variant == 5)
-            k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 12, 13, 0><<<grid, 256, 0, s>>>(da, df, n);
+            for (int k = 0; k < n; ++k) pair_block_tiles<double>(ctx, args[k], *items[g.members[k]].X, *items[g.members[k]].X);
         else k_far_tiles_batch<double, BH_OP_MW_DOUBLELAYER_ROTATED, true, 0, 0><<<grid, 256, 0, s>>>(da, df, n);
 #undef BH_BTILES
         check_launch("k_far_tiles_batch");

@@ -303,6 +303,7 @@ struct Space {
     // dof tiles for the far-field gather kernel
     bool tiles_built = false;
     int64_t ntiles = 0;
+    std::vector<int> h_tptr, h_tcells;   // t_ptr and t_cells on the host
     DevBuf<int> t_ptr, t_cells, t_slot;
     DevBuf<double> t_coef;
 };

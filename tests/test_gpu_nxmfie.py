@@ -148,3 +148,24 @@ def test_nxmfie_resident_solve_and_mie(bj, orc):
     err = max(np.abs(fe - np.abs(S2)).max(), np.abs(fh - np.abs(S1)).max()) / np.abs(S2).max()
     print(f"nxMFIE 2396 cells, k = 1: max Mie error {err:.2e}", file=sys.stderr)
     assert err < 5e-3
+
+
+def test_pair_blocks_in_several_groups(bj):
+    """n x K of a matrix whose pair blocks take more than one group of row tiles, against the
+    same rows as small spaces: some dofs in order, some shuffled (tiles of up to 128 cells),
+    and two without shapes.  1e-14 of the largest entry: an entry sums four terms, in an order
+    that follows the tile's cells."""
+    m = bj.meshsphere(1.0, nv=2060, jitter=0.02, seed=3)   # 4116 cells: 2.4 GB of blocks
+    X = bj.raviartthomas(m)
+    n = X.numfunctions()
+    op = bj.cross(bj.n, bj.Maxwell3D.doublelayer(wavenumber=3.0))
+    Z = bj.assemble(op, X, X)
+    rng = np.random.default_rng(1)
+    for rows in (np.arange(40), np.arange(n - 70, n), rng.permutation(n)[:130]):
+        lens = np.append(np.diff(X.shape_ptr)[rows], [0, 0])
+        idx = np.concatenate([np.arange(X.shape_ptr[r], X.shape_ptr[r + 1]) for r in rows])
+        S = bj.RTBasis(m, np.append(0, np.cumsum(lens)).astype(X.shape_ptr.dtype), X.shape_cell[idx], X.shape_ref[idx],
+                       X.shape_coeff[idx])
+        Zs = bj.assemble(op, S, X)
+        assert np.abs(Zs[:-2] - Z[rows]).max() < 1e-14 * np.abs(Z).max()
+        assert not Zs[-2:].any()
