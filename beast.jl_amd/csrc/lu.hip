@@ -36,9 +36,9 @@
 //                   the FP32 updates inside a block column.
 //   k_cgemm_bf16x3  FP32 trailing update from split-bf16 planes (hi*hi + hi*lo +
 //                   lo*hi on v_mfma_f32_16x16x32_bf16, FP32 accumulation).
-// Solves: permutation gather, then for FP64 factors blocked substitution
-// (k_trsv_step); for FP32 factors one launch per triangle with the inverted
-// 128x128 diagonal blocks and their couplings (k_trinv, k_blk_coupling,
+// Solves: permutation gather, then one launch per triangle: for FP64 factors a
+// substitution in 64-row blocks (k_trsv64), for FP32 factors 128-row blocks with
+// inverted diagonal blocks and their couplings (k_trinv, k_blk_coupling,
 // k_trsv_flag).  FP32 factors precondition flexible GMRES
 // inside iterative refinement in FP64 (GMRES-IR, Carson & Higham, SIAM J. Sci.
 // Comput. 40 (2018)), whose residuals use the resident FP64 matrix.
