@@ -2578,27 +2578,10 @@ __global__ void k_axpys_cols(const double2 *__restrict__ Vb, int n, int m, int q
 }
 
 template <typename T>
-__global__ void k_gather_lo(const double2 *__restrict__ src, int n, const int *__restrict__ perm,
-                            typename CT<T>::t *dst)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        const double2 v = src[perm[i]];
-        dst[i] = {(T)v.x, (T)v.y};
-    }
-}
-
-template <typename T>
 __global__ void k_widen(const typename CT<T>::t *__restrict__ src, long long cnt, double2 *__restrict__ dst)
 {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < cnt) dst[i] = {(double)src[i].x, (double)src[i].y};
-}
-
-__global__ void k_add(double2 *x, const double2 *__restrict__ d, long long cnt)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < cnt) { x[i].x += d[i].x; x[i].y += d[i].y; }
 }
 
 // ---------------------------------------------------------------- host driver
