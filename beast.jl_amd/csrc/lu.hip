@@ -57,6 +57,7 @@
 #include "bh_device.h"
 #include "bh_internal.h"
 #include "bh_matrix.h"
+#include "lu_rules.h"
 
 namespace bh {
 
@@ -140,7 +141,6 @@ __device__ __forceinline__ unsigned wave_max_u32(unsigned v)
 // being eliminated is always the phase's first register (a full unroll does not fit the
 // instruction cache, a dynamic column index would put the row into scratch memory).
 // Finished columns meet zeros in the pivot row.
-constexpr int kPW = 32;            // panel width
 constexpr int kP64Phase = 8;
 constexpr int kP64T = 256;         // rows per workgroup beside the trailing products: the registers of half a CU,
                                    // as their workgroups, so that neither waits for a whole CU to drain
@@ -491,31 +491,9 @@ __global__ __launch_bounds__(256) void k_apply64(double2 *A, long long lda, int 
 // many more instructions per column.  Measured on the MI355X per 32-column panel, before
 // (256 rows a workgroup, the previous panel's update in front of it) -> now: tournament
 // 107 -> 75 us at 4050 unknowns, 122 -> 87 us at 9003; apply 27 -> 14 and 27 -> 17 us.
-constexpr int kTsluT = 256;                   // threads of a tournament workgroup
-constexpr int kTsluRows = 2 * kTsluT;         // its rows
-constexpr int kTsluFan = kTsluRows / kPW;     // candidate sets merged per workgroup at most
 
 // rows per workgroup of k_tslu_apply
 __host__ __device__ inline int tslu_apply_row_count(int rows) { return rows <= 8192 ? 32 : 64; }
-
-// Groups that nl sets are merged in, as even as they get: the fewest levels, and among
-// those groups of at most kTsluFan / 2 sets, whose rows take one register row per thread
-// (21 us against 28 us for 32 columns).
-__host__ __device__ inline int tslu_groups(int nl)
-{
-    const int most = nl <= kTsluFan ? kTsluFan : (nl <= kTsluFan * kTsluFan / 2 ? kTsluFan / 2 : kTsluFan);
-    return (nl + most - 1) / most;
-}
-__host__ __device__ inline int tslu_fan(int nl) { return (nl + tslu_groups(nl) - 1) / tslu_groups(nl); }
-// candidate sets of all levels, for n rows
-inline size_t tslu_sets(int n)
-{
-    size_t t = 0;
-    for (int nl = (n + kTsluRows - 1) / kTsluRows;; nl = tslu_groups(nl)) {
-        t += nl;
-        if (nl <= 1) return t;
-    }
-}
 
 // Partial pivoting over R kTsluT rows held in registers, R = 1 or 2 per thread (v: the rows'
 // kPW entries; rows with used set never pivot; slot: a row's number in the workgroup).

@@ -1,0 +1,20 @@
+"""Host-side rules of the native library, compiled without a GPU and run here: each program in
+tests/host/ includes the library's own sources and returns 0, or prints what it found."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "beast.jl_amd", "csrc")
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
+@pytest.mark.parametrize("name", ["tournament_sets"])
+def test_host_program(name, tmp_path):
+    exe = str(tmp_path / name)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-Wall", "-pthread", "-D_GLIBCXX_ASSERTIONS", "-I", CSRC,
+                    os.path.join(HERE, "host", name + ".cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
