@@ -303,7 +303,7 @@ __device__ __forceinline__ void panel64_phase(double2 (&v)[kPW], int &pos, bool 
                 if (late && lane == 0) __hip_atomic_store(w.info, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if (lane < 2 * W)
                     ((double *)S.u)[lane] = __longlong_as_double((long long)((a & 0xffffffff00000000ull) | (b >> 32)));
-                if (lane == 0) S.pos = bhi ? bp : c;
+                if (lane == 0) S.pos = panel64_pivot(late, bhi != 0, bp, c);
             }
             __syncthreads();
             u = S.u;
@@ -313,12 +313,9 @@ __device__ __forceinline__ void panel64_phase(double2 (&v)[kPW], int &pos, bool 
         const bool nz = piv.x != 0.0 || piv.y != 0.0;
         if (g == 0 && tid == 0) {
             ipiv[c] = p;
-            if (!nz && *w.info == 0) *w.info = c + 1;
+            if (!nz) atomicCAS(w.info, 0, c + 1);   // a wait that ran out keeps its mark
         }
-        if (valid && !used) {
-            if (pos == p) { used = true; pos = c; }
-            else if (pos == c) pos = p;
-        }
+        if (valid && !used) panel64_move(pos, used, c, p);
         const double den = piv.x * piv.x + piv.y * piv.y;
         const double2 inv{piv.x / den, -piv.y / den};
         const double2 v0 = v[C0];
@@ -2964,6 +2961,8 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
     W.moves.ensure(2 * kPW);
     W.plan.ensure(4 * kMaxSwaps);
     BH_CHECK_HIP(hipMemsetAsync(W.info.p, 0, sizeof(int), s));
+    // a panel whose wait ran out leaves places of moves as they were: rows of the matrix, not chance
+    BH_CHECK_HIP(hipMemsetAsync(W.moves.p, 0, 2 * kPW * sizeof(int), s));
     // block column of the right-looking LU (trailing-update depth); the FP32
     // path's deeper blocks halve the C traffic per flop of the trailing update
     auto depth = [&](int k) { return sizeof(T) == 4 ? fp32_block_depth(n, k, split) : kNBFP64; };

@@ -47,4 +47,21 @@ inline size_t tslu_sets(int n)
     return most;
 }
 
+// FP64 panels.  Row that a workgroup takes as column c's pivot: pos, the position of the best
+// candidate that it read.  Without a candidate none moves, nor after a wait that ran out (late):
+// the words read then are of an earlier column, or none, and their position may lie above the panel.
+BH_HD inline int panel64_pivot(bool late, bool found, int pos, int c) { return found && !late ? pos : c; }
+
+// The interchange of the positions c and p for a row at pos that has not been a pivot.  Workgroups
+// that disagree on p (one of them late) leave two rows in one place: void, but inside the panel.
+BH_HD inline void panel64_move(int &pos, bool &used, int c, int p)
+{
+    if (pos == p) {
+        used = true;
+        pos = c;
+    } else if (pos == c) {
+        pos = p;
+    }
+}
+
 }  // namespace bh
