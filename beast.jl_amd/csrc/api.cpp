@@ -3,7 +3,6 @@
 
 #include <cmath>
 #include <cstdarg>
-#include <atomic>
 #include <cstring>
 #include <new>
 
@@ -51,7 +50,6 @@ extern "C" int bh_ctx_create(int device, bh_ctx **out)
     c->arch = prop.gcnArchName;
     BH_CHECK_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
     *out = c.release();
-    bh::context_created();
     BH_API_END
 }
 
@@ -69,7 +67,6 @@ static void ctx_free(Ctx *c)
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete static_cast<bh_ctx *>(c);
-    context_destroyed();
 }
 
 void ctx_retain(Ctx *c) { c->refs.fetch_add(1); }
@@ -188,18 +185,6 @@ extern "C" int bh_ctx_synchronize(bh_ctx *ctx)
 }
 
 namespace bh {
-namespace {
-std::atomic<int> g_live{0};
-}
-int live_contexts() { return g_live.load(); }
-void context_created() { g_live.fetch_add(1); }
-void context_destroyed() { g_live.fetch_sub(1); }
-std::mutex &coop_mutex()
-{
-    static std::mutex m;
-    return m;
-}
-
 void resolve_stats(Ctx &ctx)
 {
     (void)hipStreamSynchronize(ctx.stream);

@@ -51,6 +51,7 @@
 #include <complex>
 #include <cstring>
 #include <limits>
+#include <map>
 #include <memory>
 #include <vector>
 
@@ -58,6 +59,7 @@
 #include "bh_internal.h"
 #include "bh_matrix.h"
 #include "lu_rules.h"
+#include "panel_gate.h"
 
 namespace bh {
 
@@ -2663,14 +2665,6 @@ void panel64(Ctx &ctx, hipStream_t s, LUWork<double> &W, double2 *A, long long l
         ProfScope prof(ctx, "k_panel", (double)rows * pw * sizeof(double2) * 2, s);
         if (G == 1) {
             k_panel64<kP64TOne><<<1, kP64TOne, 0, s>>>(A, lda, n, c, pw, ipiv, sl);
-        } else if (live_contexts() > 1) {
-            // The workgroups wait for one another, so all must be resident at once.  One panel's are
-            // (checked in lu_factor), but panels of several contexts could each hold part of the
-            // device and wait for the rest: with several live contexts they run one at a time.
-            std::lock_guard<std::mutex> lock(coop_mutex());
-            k_panel64<kP64T><<<G, kP64T, 0, s>>>(A, lda, n, c, pw, ipiv, sl);
-            check("k_panel64");
-            BH_CHECK_HIP(hipStreamSynchronize(s));
         } else {
             k_panel64<kP64T><<<G, kP64T, 0, s>>>(A, lda, n, c, pw, ipiv, sl);
         }
@@ -2932,6 +2926,15 @@ LUCache &lu_cache(Ctx &ctx)
     return *static_cast<LUCache *>(ctx.lu_cache.get());
 }
 
+// one gate per device for all contexts of the process
+PanelGate &panel_gate(int device)
+{
+    static std::mutex mu;
+    static std::map<int, PanelGate> gates;
+    std::lock_guard<std::mutex> g(mu);
+    return gates[device];
+}
+
 // dinv (FP32 only, may be NULL): the diagonal-block inverses and couplings of the
 // factors are formed on the context stream before the workspace is released, so
 // the device does not idle while the host frees it.
@@ -2954,6 +2957,7 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
         own = std::make_unique<LUBuffers<T>>();
         buf = own.get();
     }
+    PanelPlaces places;   // FP64: the panels' workgroups, until the last panel is done
     LUWork<T> &W = buf->W;
     DevBuf<__bf16> &PA = buf->PA, &PB = buf->PB;
     W.eblk_of = W.eblk_side_of = -1;
@@ -2986,6 +2990,7 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
         int per_cu = 0;
         BH_CHECK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)k_panel64<kP64T>, kP64T, 0));
         BH_REQUIRE(G <= per_cu * ctx.num_cus, "panel of %d rows: its workgroups cannot all be resident", n);
+        if (n > kP64TOne) places.take(panel_gate(ctx.device), G, (long long)per_cu * ctx.num_cus);
         const size_t words = (size_t)G * (4 + 8 * kPW);
         W.slots.ensure(words);
         BH_CHECK_HIP(hipMemsetAsync(W.slots.p, 0, words * sizeof(unsigned long long), s));
@@ -3031,6 +3036,14 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
             BH_CHECK_HIP(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
             BH_CHECK_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
         }
+        struct Drain {   // after an error too no panel runs once the places are given back
+            hipStream_t s, s2;
+            ~Drain() {
+                if (!s) return;
+                (void)hipStreamSynchronize(s);
+                (void)hipStreamSynchronize(s2);
+            }
+        } drain{s, s2};
         factor_block<T>(ctx, s, W, A, lda, n, 0, std::min(depth(0), n), ipiv);
         // block k is factored; its interchanges reach the other columns (in pieces
         // of at most kMaxSwaps interchanges, applied in order) over [c0, c1) and [c2, c3)
@@ -3075,6 +3088,7 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
             }
             BH_CHECK_HIP(hipStreamWaitEvent(s, done, 0));
         }
+        drain.s = nullptr;   // s waits for s2 and is waited for below
     }
     if constexpr (sizeof(T) == 4) {
         if (dinv) invert_diagonal_blocks(s, (const float2 *)A, lda, n, dinv);

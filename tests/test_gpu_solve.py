@@ -315,3 +315,32 @@ def test_gmres_steps_per_column(bj, cond=1e5):
         assert np.array_equal(x[:, q], M.solve(B[:, q], tol=tol, maxit=10))
         alone += M.stats["inner"]
     assert steps == alone and steps >= 3
+
+
+def test_fp64_factorisations_side_by_side(bj):
+    """FP64 panels of several factorisations at once, two contexts with two matrices each: pivots
+    and solutions are those that each matrix has alone, bit for bit."""
+    import threading
+    n = 1300
+    A = [_rand(n, 40 + i) for i in range(4)]
+    b = _rand(n, 44)[:, 0]
+    alone = [bj.DeviceMatrix.from_host(a).factor("fp64") for a in A]
+    want = [(M.pivots(), M.solve(b)) for M in alone]
+    ctxs = [bj.Context(), bj.Context()]
+    mats = [bj.DeviceMatrix.from_host(a, ctx=ctxs[i % 2]) for i, a in enumerate(A)]
+    lib, nat, codes = bj._native.load(), bj._native, [None] * 4
+
+    def factor(i):   # the library's own entry: the Python call would take the context's lock
+        codes[i] = lib.bh_matrix_factor(mats[i].h, nat.FP64)
+
+    th = [threading.Thread(target=factor, args=(i,)) for i in range(4)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert codes == [nat.BH_OK] * 4
+    for M, (p, x) in zip(mats, want):
+        assert np.array_equal(M.pivots(), p) and np.array_equal(M.solve(b), x)
+    mats.clear()
+    for c in ctxs:
+        c.close()

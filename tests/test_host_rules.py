@@ -11,7 +11,7 @@ CSRC = os.path.join(os.path.dirname(HERE), "beast.jl_amd", "csrc")
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
-@pytest.mark.parametrize("name", ["tournament_sets", "panel_positions"])
+@pytest.mark.parametrize("name", ["tournament_sets", "panel_positions", "panel_gate"])
 def test_host_program(name, tmp_path):
     exe = str(tmp_path / name)
     subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-Wall", "-pthread", "-D_GLIBCXX_ASSERTIONS", "-I", CSRC,
