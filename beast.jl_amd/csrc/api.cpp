@@ -71,76 +71,6 @@ static void ctx_free(Ctx *c)
 
 void ctx_retain(Ctx *c) { c->refs.fetch_add(1); }
 
-// ---------------------------------------------------------------- buffer pool
-namespace {
-constexpr size_t kPoolMinBytes = size_t(1) << 20;   // smaller buffers are freed at once
-}
-
-void *pool_alloc(Ctx &ctx, size_t bytes)
-{
-    {
-        std::lock_guard<std::mutex> g(ctx.pool_mu);
-        int best = -1;
-        for (int i = 0; i < (int)ctx.pool.size(); ++i) {
-            const size_t b = ctx.pool[i].second;
-            if (b >= bytes && b - bytes <= bytes / 4 && (best < 0 || b < ctx.pool[best].second)) best = i;
-        }
-        if (best >= 0) {
-            void *p = ctx.pool[best].first;
-            ctx.pool_bytes -= ctx.pool[best].second;
-            ctx.pool.erase(ctx.pool.begin() + best);
-            return p;
-        }
-    }
-    void *p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess) {   // pooled memory may be what is missing
-        (void)hipGetLastError();
-        pool_trim(ctx, 0);
-        e = hipMalloc(&p, bytes);
-    }
-    if (e != hipSuccess) {
-        set_error("hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
-        throw Error{BH_ERR_OOM};
-    }
-    return p;
-}
-
-void pool_free(Ctx &ctx, void *p, size_t bytes)
-{
-    if (!p) return;
-    std::vector<void *> drop;
-    {
-        std::lock_guard<std::mutex> g(ctx.pool_mu);
-        if (bytes < kPoolMinBytes || bytes > ctx.pool_limit) {
-            drop.push_back(p);
-        } else {
-            ctx.pool.emplace_back(p, bytes);
-            ctx.pool_bytes += bytes;
-            while (ctx.pool_bytes > ctx.pool_limit) {   // oldest first
-                drop.push_back(ctx.pool.front().first);
-                ctx.pool_bytes -= ctx.pool.front().second;
-                ctx.pool.erase(ctx.pool.begin());
-            }
-        }
-    }
-    for (void *q : drop) (void)hipFree(q);
-}
-
-void pool_trim(Ctx &ctx, size_t keep_bytes)
-{
-    std::vector<void *> drop;
-    {
-        std::lock_guard<std::mutex> g(ctx.pool_mu);
-        while (ctx.pool_bytes > keep_bytes && !ctx.pool.empty()) {
-            drop.push_back(ctx.pool.front().first);
-            ctx.pool_bytes -= ctx.pool.front().second;
-            ctx.pool.erase(ctx.pool.begin());
-        }
-    }
-    for (void *q : drop) (void)hipFree(q);
-}
-
 void ctx_release(Ctx *c)
 {
     if (c->refs.fetch_sub(1) == 1 && c->closing.load()) ctx_free(c);

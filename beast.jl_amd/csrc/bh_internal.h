@@ -66,13 +66,14 @@ template <typename T>
 struct DevBuf {
     T *p = nullptr;
     size_t n = 0;
+    size_t held = 0;   // bytes of the allocation (one from the pool can be larger than n elements)
     DevBuf() = default;
     explicit DevBuf(size_t count) { alloc(count); }
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
-    DevBuf(DevBuf &&o) noexcept : p(o.p), n(o.n) { o.p = nullptr; o.n = 0; }
+    DevBuf(DevBuf &&o) noexcept : p(o.p), n(o.n), held(o.held) { o.detach(); }
     DevBuf &operator=(DevBuf &&o) noexcept {
-        if (this != &o) { release(); p = o.p; n = o.n; o.p = nullptr; o.n = 0; }
+        if (this != &o) { release(); p = o.p; n = o.n; held = o.held; o.detach(); }
         return *this;
     }
     ~DevBuf() { release(); }
@@ -86,14 +87,14 @@ struct DevBuf {
             throw Error{BH_ERR_OOM};
         }
         n = count;
+        held = count * sizeof(T);
     }
     void ensure(size_t count) {   // at least count elements; contents unspecified
         if (n < count) alloc(count);
     }
     void release() {
         if (p) (void)hipFree(p);
-        p = nullptr;
-        n = 0;
+        detach();
     }
     void upload(const T *h, size_t count, hipStream_t s) {
         if (count > n) alloc(count);
@@ -101,8 +102,8 @@ struct DevBuf {
     }
     size_t bytes() const { return n * sizeof(T); }
     // ownership transfer to and from the context's buffer pool
-    void adopt(T *q, size_t count) { release(); p = q; n = count; }
-    T *detach() { T *q = p; p = nullptr; n = 0; return q; }
+    void adopt(T *q, size_t count, size_t bytes) { release(); p = q; n = count; held = bytes; }
+    T *detach() { T *q = p; p = nullptr; n = held = 0; return q; }
 };
 
 // ---------------------------------------------------------------- quadrature rules
@@ -137,6 +138,12 @@ struct KernelStat {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> pending;
 };
 
+// a device allocation and its whole size, whatever part of it was asked for
+struct PoolMem {
+    void *p;
+    size_t bytes;
+};
+
 struct Ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -162,7 +169,7 @@ struct Ctx {
     // a similar size (a repeated assemble-factor-solve allocates nothing); at most
     // pool_limit bytes are kept, the oldest buffers are freed first
     std::mutex pool_mu;
-    std::vector<std::pair<void *, size_t>> pool;
+    std::vector<PoolMem> pool;
     size_t pool_bytes = 0;
     size_t pool_limit = size_t(64) << 30;
 };
@@ -178,21 +185,23 @@ void scratch_register(int device);
 // buffer to the pool (or frees it when it is small or the pool is disabled).
 // The caller orders the work: a buffer goes to the pool only once the kernels
 // that use it are complete or ordered on the context stream.
-void *pool_alloc(Ctx &ctx, size_t bytes);
-void pool_free(Ctx &ctx, void *p, size_t bytes);
+PoolMem pool_alloc(Ctx &ctx, size_t bytes);
+void pool_free(Ctx &ctx, PoolMem m);
 void pool_trim(Ctx &ctx, size_t keep_bytes);
 template <typename T>
 void pool_release(Ctx &ctx, DevBuf<T> &b)
 {
-    const size_t bytes = b.n * sizeof(T);
-    if (b.p) pool_free(ctx, b.detach(), bytes);
+    const size_t bytes = b.held;
+    if (b.p) pool_free(ctx, {b.detach(), bytes});
 }
 template <typename T>
 void pool_alloc(Ctx &ctx, DevBuf<T> &b, size_t count)
 {
     if (b.n == count) return;
     pool_release(ctx, b);
-    if (count) b.adopt((T *)pool_alloc(ctx, count * sizeof(T)), count);
+    if (!count) return;
+    const PoolMem m = pool_alloc(ctx, count * sizeof(T));
+    b.adopt((T *)m.p, count, m.bytes);
 }
 
 // Copies (add = false) or adds (add = true; complex entries of 2 es-byte reals, es 4 or 8) the
@@ -206,7 +215,7 @@ template <typename T>
 struct PoolBuf {
     Ctx *ctx = nullptr;
     T *p = nullptr;
-    size_t n = 0;
+    size_t held = 0;
     PoolBuf() = default;
     PoolBuf(Ctx &c, size_t count) { alloc(c, count); }
     PoolBuf(const PoolBuf &) = delete;
@@ -216,14 +225,16 @@ struct PoolBuf {
         if (p) (void)hipFree(p);
         p = nullptr;
         ctx = &c;
-        n = count;
-        if (count) p = (T *)pool_alloc(c, count * sizeof(T));
+        if (!count) return;
+        const PoolMem m = pool_alloc(c, count * sizeof(T));
+        p = (T *)m.p;
+        held = m.bytes;
     }
     void upload(const T *h, size_t count, hipStream_t s) {
         if (count) BH_CHECK_HIP(hipMemcpyAsync(p, h, count * sizeof(T), hipMemcpyHostToDevice, s));
     }
     void done() {
-        if (p) pool_free(*ctx, p, n * sizeof(T));
+        if (p) pool_free(*ctx, {p, held});
         p = nullptr;
     }
 };
