@@ -49,6 +49,7 @@ extern "C" int bh_ctx_create(int device, bh_ctx **out)
     c->num_cus = prop.multiProcessorCount;
     c->arch = prop.gcnArchName;
     BH_CHECK_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+    bh::pool_register(c.get());
     *out = c.release();
     BH_API_END
 }
@@ -58,6 +59,7 @@ static void ctx_free(Ctx *c)
 {
     bool expected = false;
     if (!c->freed.compare_exchange_strong(expected, true)) return;   // exactly once
+    pool_unregister(c);
     (void)hipSetDevice(c->device);
     resolve_stats(*c);
     if (c->stream) (void)hipStreamSynchronize(c->stream);

@@ -62,6 +62,10 @@ struct Error {
     } while (0)
 
 // ---------------------------------------------------------------- device memory
+// hipMalloc on the current device.  What the pools of its contexts hold may be what is missing:
+// they are freed before a second attempt, whose failure is the error.
+void *device_malloc(size_t bytes);
+
 template <typename T>
 struct DevBuf {
     T *p = nullptr;
@@ -80,12 +84,7 @@ struct DevBuf {
     void alloc(size_t count) {
         release();
         if (count == 0) return;
-        hipError_t e = hipMalloc(&p, count * sizeof(T));
-        if (e != hipSuccess) {
-            p = nullptr;
-            set_error("hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
-            throw Error{BH_ERR_OOM};
-        }
+        p = (T *)device_malloc(count * sizeof(T));
         n = count;
         held = count * sizeof(T);
     }
@@ -180,14 +179,16 @@ void ctx_release(Ctx *c);
 void scratch_register(int device);
 
 // Pool of large device buffers (see Ctx::pool).  pool_alloc returns a pooled
-// buffer of at least `bytes` and at most 5/4 of it, else a fresh allocation
-// (after freeing the pool if the device is out of memory).  pool_free returns a
+// buffer of at least `bytes` and at most 5/4 of it, else a fresh one of device_malloc.  pool_free returns a
 // buffer to the pool (or frees it when it is small or the pool is disabled).
 // The caller orders the work: a buffer goes to the pool only once the kernels
 // that use it are complete or ordered on the context stream.
 PoolMem pool_alloc(Ctx &ctx, size_t bytes);
 void pool_free(Ctx &ctx, PoolMem m);
 void pool_trim(Ctx &ctx, size_t keep_bytes);
+// the contexts whose pools device_malloc may free
+void pool_register(Ctx *ctx);
+void pool_unregister(Ctx *ctx);
 template <typename T>
 void pool_release(Ctx &ctx, DevBuf<T> &b)
 {

@@ -1,10 +1,58 @@
 // Pool of large device buffers (Ctx::pool).
+#include <set>
+
 #include "bh_internal.h"
 
 namespace bh {
 
 namespace {
 constexpr size_t kPoolMinBytes = size_t(1) << 20;   // smaller buffers are freed at once
+
+// never destroyed: a context may outlive the library's static objects
+std::mutex &registry_mutex()
+{
+    static std::mutex &m = *new std::mutex;
+    return m;
+}
+std::set<Ctx *> &registry()
+{
+    static std::set<Ctx *> &s = *new std::set<Ctx *>;
+    return s;
+}
+}  // namespace
+
+void pool_register(Ctx *ctx)
+{
+    std::lock_guard<std::mutex> g(registry_mutex());
+    registry().insert(ctx);
+}
+
+void pool_unregister(Ctx *ctx)
+{
+    std::lock_guard<std::mutex> g(registry_mutex());
+    registry().erase(ctx);
+}
+
+void *device_malloc(size_t bytes)
+{
+    void *p = nullptr;
+    hipError_t e = hipMalloc(&p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        int device = -1;
+        BH_CHECK_HIP(hipGetDevice(&device));
+        {
+            std::lock_guard<std::mutex> g(registry_mutex());
+            for (Ctx *c : registry())
+                if (c->device == device) pool_trim(*c, 0);
+        }
+        e = hipMalloc(&p, bytes);
+    }
+    if (e != hipSuccess) {
+        set_error("hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
+        throw Error{BH_ERR_OOM};
+    }
+    return p;
 }
 
 PoolMem pool_alloc(Ctx &ctx, size_t bytes)
@@ -23,18 +71,7 @@ PoolMem pool_alloc(Ctx &ctx, size_t bytes)
             return m;
         }
     }
-    void *p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
-    if (e != hipSuccess) {   // pooled memory may be what is missing
-        (void)hipGetLastError();
-        pool_trim(ctx, 0);
-        e = hipMalloc(&p, bytes);
-    }
-    if (e != hipSuccess) {
-        set_error("hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
-        throw Error{BH_ERR_OOM};
-    }
-    return {p, bytes};
+    return {device_malloc(bytes), bytes};
 }
 
 void pool_free(Ctx &ctx, PoolMem m)

@@ -118,7 +118,7 @@ int bh_ctx_synchronize(bh_ctx *ctx);
  * assemble-factor-solve allocates nothing.  limit_bytes >= 0 sets the most the pool
  * keeps (default 64 GiB; 0 disables it and frees what it holds), a negative value
  * leaves it; *pooled_bytes (may be NULL) receives what the pool holds now.  A
- * device allocation that fails frees the pool and tries once more. */
+ * device allocation that fails frees the pools of the device's contexts and tries once more. */
 int bh_ctx_pool(bh_ctx *ctx, int64_t limit_bytes, int64_t *pooled_bytes);
 /* Measurement (no counterpart in the reference): while profiling is on, every
  * launch of the library's kernels is bracketed by HIP events on the context

@@ -29,6 +29,7 @@ extern "C" hipError_t hipFree(void *p)
     stub::live.erase(p);
     return hipSuccess;
 }
+extern "C" hipError_t hipGetDevice(int *device) { return *device = 0, hipSuccess; }
 extern "C" hipError_t hipGetLastError() { return hipSuccess; }
 extern "C" const char *hipGetErrorString(hipError_t) { return "stub"; }
 namespace bh {
