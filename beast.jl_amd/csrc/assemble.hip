@@ -24,13 +24,16 @@
 // moment formulas below do not cancel catastrophically (and the FP32 variant
 // keeps ~1e-7 relative accuracy).
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <map>
 
 #include "bh_device.h"
 #include "bh_internal.h"
 #include "bh_matrix.h"
+#include "tile_groups.h"
 
 namespace bh {
 
@@ -1154,12 +1157,13 @@ struct TileArgs {
     int accumulate;
     double scale_r, scale_i;
     const void *rpack;    // the row tiles' test cells packed field by field (single layer, default rule)
-    // tiles gathered from pair blocks (k_pair_blocks): the blocks, the place of each tile's test
-    // cells in their group, the group's padded number of test cells, its first row tile
+    // tiles gathered from pair blocks (k_pair_blocks): the blocks, the places of each tile's test
+    // and trial cells among the blocks', the padded number of test cells, the number of trial
+    // cells, the first row tile
     const void *pblk;
-    const int *rloc;
+    const int *rloc, *cloc;
     long long npp;
-    int nfs, tr0;
+    int ncols, tr0;
 };
 
 // v of lane l (l wave-uniform)
@@ -1233,7 +1237,7 @@ __device__ void far_tiles_dev(const TileArgs &A, int tr, int tc)
             for (int v = 0; v < 4 * QO; ++v) s_pts[v * kTileCells + k] = tq[v];
         }
     }
-    for (int k = tid; k < nc; k += 256) s_cc[k] = A.col.cells[c0 + k];
+    for (int k = tid; k < nc; k += 256) s_cc[k] = LOADED ? A.cloc[c0 + k] : A.col.cells[c0 + k];
     if (tid < 2 * kTile) {
         const int l = tid >> 1, s = tid & 1;
         const int m = mbase + l, n = nbase + l;
@@ -1284,7 +1288,7 @@ __device__ void far_tiles_dev(const TileArgs &A, int tr, int tc)
             const int rc = t % nr, cc = t / nr;
             if constexpr (LOADED) {
                 const cx<R> *w = (const cx<R> *)A.pblk + (size_t)s_cc[cb + cc] * A.npp + s_rc[rc];
-                const size_t plane = (size_t)A.nfs * A.npp;
+                const size_t plane = (size_t)A.ncols * A.npp;
                 cx<R> v[9];
 #pragma unroll
                 for (int k = 0; k < 9; ++k) v[k] = w[k * plane];
@@ -1399,20 +1403,21 @@ __global__ __launch_bounds__(256, far_min_blocks<OPK>()) void k_far_tiles(TileAr
     far_tiles_dev<R, OPK, ROWMAJOR, QO, QI, SHIFT>(A, blockIdx.y, blockIdx.x);
 }
 
-// Blocks of the pairs (test cell cells[i], trial cell q), i < ncells, q < nfs, once each:
-// block entry k at blk[(k nfs + q) npp + i].  A wave takes 64 test cells and one trial cell.
+// Blocks of the pairs (test cell cells[i], trial cell qcells[q]), i < ncells, q < ncols, once
+// each: block entry k at blk[(k ncols + q) npp + i].  A wave takes 64 test cells and one trial cell.
 // For the rotated double layer, whose 156 point pairs cost more than 144 bytes there and back: a
 // 64 x 64 tile that forms its own blocks shares its cells with its neighbours, and every block
 // was formed 1.8 times.  Bound by FP64 VALU issue.  6002 x 6002 cells: 14.5 ms, and 2.7 ms to
 // gather them, against 28.2 ms for tiles that form their own.
 template <typename R, int OPK, int QO, int QI, int SHIFT>
-__global__ __launch_bounds__(256, 2) void k_pair_blocks(FarArgs A, const int *__restrict__ cells, int ncells, int nfs,
-                                                        cx<R> *blk, long long npp)
+__global__ __launch_bounds__(256, 2) void k_pair_blocks(FarArgs A, const int *__restrict__ cells, int ncells,
+                                                        const int *__restrict__ qcells, int ncols, cx<R> *blk,
+                                                        long long npp)
 {
     const int i = blockIdx.y * 64 + (threadIdx.x & 63);
     const int q = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (q >= nfs || i >= ncells) return;
-    far_block<R, OPK, QO, QI, SHIFT>(A, cells[i], q, blk + (size_t)q * npp + i, (long long)nfs * npp);
+    if (q >= ncols || i >= ncells) return;
+    far_block<R, OPK, QO, QI, SHIFT>(A, cells[i], qcells[q], blk + (size_t)q * npp + i, (long long)ncols * npp);
 }
 
 template <typename R, bool ROWMAJOR>
@@ -1819,7 +1824,9 @@ const void *pack_rows(hipStream_t s, const Space &X, const FarArgs &F, DevBuf<ch
 }
 
 // The rotated double layer's default-rule tiles (12 x 13 points): pair blocks of a group of row
-// tiles (k_pair_blocks), then those tiles gathered from them, group by group.  A group's blocks
+// tiles with the trial cells that the columns touch (k_pair_blocks), then those tiles gathered
+// from them, group by group.  (All trial cells of the mesh cost columns of a few dofs more than
+// tiles that form their own blocks: 3000 x 60 of 3000 dofs, lossy, 2.6 -> 4.4 ms.)  A group's blocks
 // take at most kPairBlockBytes (a quarter of that, and so on, where memory is short) or what its
 // one row tile needs.
 constexpr size_t kPairBlockBytes = size_t(2) << 30;
@@ -1829,69 +1836,49 @@ void pair_block_tiles(Ctx &ctx, TileArgs A, const Space &X, const Space &Y)
 {
     constexpr int DLR = BH_OP_MW_DOUBLELAYER_ROTATED;
     hipStream_t s = ctx.stream;
-    const long long nfs = Y.mesh->nf, nt = X.ntiles;
-    const size_t per_cell = (size_t)nfs * 9 * sizeof(cx<R>);
-    struct Group {
-        long long t0, t1;
-        int c0, n;
-    };
-    std::vector<Group> groups;
-    std::vector<int> cells, rloc(X.h_tcells.size());
+    const long long nt = X.ntiles;
+    const TileGroups cols = tile_groups(Y.h_tptr, Y.h_tcells, Y.mesh->nf, 1, LLONG_MAX);   // one group
+    const size_t per_cell = (size_t)cols.most * 9 * sizeof(cx<R>);
+    TileGroups rows;
     PoolBuf<char> blk;
-    long long npp = 0;
     for (size_t budget = kPairBlockBytes;; budget /= 4) {
-        groups.clear();
-        cells.clear();
-        npp = 0;
-        std::vector<int> at(X.mesh->nf, -1);   // place in the current group, offset by its first cell
-        for (long long t = 0; t < nt;) {
-            Group g{t, t, (int)cells.size(), 0};
-            for (; t < nt; ++t) {
-                int more = 0;
-                for (int k = X.h_tptr[t]; k < X.h_tptr[t + 1]; ++k) more += at[X.h_tcells[k]] < g.c0;
-                if (t > g.t0 && (size_t)((g.n + more + 63) / 64 * 64) * per_cell > budget) break;
-                for (int k = X.h_tptr[t]; k < X.h_tptr[t + 1]; ++k) {
-                    const int c = X.h_tcells[k];
-                    if (at[c] < g.c0) {
-                        at[c] = g.c0 + g.n++;
-                        cells.push_back(c);
-                    }
-                    rloc[k] = at[c] - g.c0;
-                }
-            }
-            g.t1 = t;
-            npp = std::max(npp, (long long)(g.n + 63) / 64 * 64);
-            groups.push_back(g);
-        }
+        rows = tile_groups(X.h_tptr, X.h_tcells, X.mesh->nf, 64,
+                           per_cell ? (long long)(budget / per_cell) : LLONG_MAX);
         try {
-            blk.alloc(ctx, (size_t)npp * per_cell);
+            blk.alloc(ctx, (size_t)rows.most * per_cell);
             break;
         } catch (const Error &e) {
-            if (e.code != BH_ERR_OOM || (long long)groups.size() == nt) throw;
+            if (e.code != BH_ERR_OOM || (long long)rows.groups.size() == nt) throw;
             (void)hipGetLastError();
         }
     }
-    DevBuf<int> dcells, drloc;
-    dcells.upload(cells.data(), cells.size(), s);
-    drloc.upload(rloc.data(), rloc.size(), s);
+    std::vector<int> lists;
+    for (const std::vector<int> &v : {std::cref(rows.cells), std::cref(cols.cells), std::cref(rows.loc), std::cref(cols.loc)})
+        lists.insert(lists.end(), v.begin(), v.end());
+    DevBuf<int> dlists;
+    dlists.upload(lists.data(), lists.size(), s);
+    const int *drows = dlists.p, *dcols = drows + rows.cells.size();
+    const long long npp = rows.most;
+    const int ncols = (int)cols.most;
     A.pblk = blk.p;
-    A.rloc = drloc.p;
+    A.rloc = dcols + cols.cells.size();
+    A.cloc = A.rloc + rows.loc.size();
     A.npp = npp;
-    A.nfs = (int)nfs;
+    A.ncols = ncols;
     const int shift = sizeof(R) == 8 ? A.far.shifted : 0;
     constexpr int kL1 = sizeof(R) == 8 ? 1 : 0;
-    for (const Group &g : groups) {
-        const dim3 bg((unsigned)((nfs + 3) / 4), (unsigned)((g.n + 63) / 64));
-        const int *gc = dcells.p + g.c0;
+    for (const TileGroup &g : rows.groups) {
+        const dim3 bg((unsigned)((ncols + 3) / 4), (unsigned)((g.n + 63) / 64));
+        const int *gr = drows + g.c0, *gq = dcols;
         cx<R> *w = (cx<R> *)blk.p;
-        if (g.n == 0 || nfs == 0) {
+        if (g.n == 0 || ncols == 0) {
             // dofs without shapes: zeros
-        } else if (shift == 1) k_pair_blocks<R, DLR, 12, 13, kL1><<<bg, 256, 0, s>>>(A.far, gc, g.n, (int)nfs, w, npp);
-        else if (shift == 2) k_pair_blocks<R, DLR, 12, 13, 2 * kL1><<<bg, 256, 0, s>>>(A.far, gc, g.n, (int)nfs, w, npp);
-        else if (shift == 3) k_pair_blocks<R, DLR, 12, 13, 3 * kL1><<<bg, 256, 0, s>>>(A.far, gc, g.n, (int)nfs, w, npp);
-        else k_pair_blocks<R, DLR, 12, 13, 0><<<bg, 256, 0, s>>>(A.far, gc, g.n, (int)nfs, w, npp);
+        } else if (shift == 1) k_pair_blocks<R, DLR, 12, 13, kL1><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, ncols, w, npp);
+        else if (shift == 2) k_pair_blocks<R, DLR, 12, 13, 2 * kL1><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, ncols, w, npp);
+        else if (shift == 3) k_pair_blocks<R, DLR, 12, 13, 3 * kL1><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, ncols, w, npp);
+        else k_pair_blocks<R, DLR, 12, 13, 0><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, ncols, w, npp);
         check_launch("k_pair_blocks");
-        A.tr0 = (int)g.t0;
+        A.tr0 = g.t0;
         const dim3 tg((unsigned)Y.ntiles, (unsigned)(g.t1 - g.t0));
         if (A.rowmajor) k_gather_tiles<R, true><<<tg, 256, 0, s>>>(A);
         else k_gather_tiles<R, false><<<tg, 256, 0, s>>>(A);

@@ -169,3 +169,23 @@ def test_pair_blocks_in_several_groups(bj):
         Zs = bj.assemble(op, S, X)
         assert np.abs(Zs[:-2] - Z[rows]).max() < 1e-14 * np.abs(Z).max()
         assert not Zs[-2:].any()
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-14), ("fp32", 4e-6)])
+def test_rotated_columns_of_a_part(bj, precision, tol):
+    """n x K with columns that touch a few cells of a mesh of its own: in order, scattered, and
+    two without shapes, against the whole matrix's columns.  An entry sums four terms in an order
+    that follows the tiles' cells: 1e-14 of the largest entry (32 ulp in single precision)."""
+    X, Y = bj.raviartthomas(bj.meshsphere(1.0, nv=150)), bj.raviartthomas(bj.meshellipsoid(2.0, 1.0, 1.0, nv=400))
+    op = bj.cross(bj.n, bj.Maxwell3D.doublelayer(gamma=0.5 + 3.0j))
+    Z = bj.assemble(op, X, Y, precision=precision)
+    n = Y.numfunctions()
+    rng = np.random.default_rng(2)
+    for cols in (np.arange(30), np.arange(n - 70, n), rng.permutation(n)[:130]):
+        lens = np.append(np.diff(Y.shape_ptr)[cols], [0, 0])
+        idx = np.concatenate([np.arange(Y.shape_ptr[c], Y.shape_ptr[c + 1]) for c in cols])
+        S = bj.RTBasis(Y.geo, np.append(0, np.cumsum(lens)).astype(Y.shape_ptr.dtype), Y.shape_cell[idx], Y.shape_ref[idx],
+                       Y.shape_coeff[idx])
+        Zs = bj.assemble(op, X, S, precision=precision)
+        assert np.abs(Zs[:, :-2] - Z[:, cols]).max() < tol * np.abs(Z).max()
+        assert not Zs[:, -2:].any()
