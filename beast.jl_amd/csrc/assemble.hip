@@ -1159,11 +1159,11 @@ struct TileArgs {
     const void *rpack;    // the row tiles' test cells packed field by field (single layer, default rule)
     // tiles gathered from pair blocks (k_pair_blocks): the blocks, the places of each tile's test
     // and trial cells among the blocks', the padded number of test cells, the number of trial
-    // cells, the first row tile
+    // cells, the first row and column tile
     const void *pblk;
     const int *rloc, *cloc;
     long long npp;
-    int ncols, tr0;
+    int ncols, tr0, tc0;
 };
 
 // v of lane l (l wave-uniform)
@@ -1423,7 +1423,7 @@ __global__ __launch_bounds__(256, 2) void k_pair_blocks(FarArgs A, const int *__
 template <typename R, bool ROWMAJOR>
 __global__ __launch_bounds__(256) void k_gather_tiles(TileArgs A)
 {
-    far_tiles_dev<R, BH_OP_MW_DOUBLELAYER_ROTATED, ROWMAJOR, 0, 0, 0, true>(A, A.tr0 + blockIdx.y, blockIdx.x);
+    far_tiles_dev<R, BH_OP_MW_DOUBLELAYER_ROTATED, ROWMAJOR, 0, 0, 0, true>(A, A.tr0 + blockIdx.y, A.tc0 + blockIdx.x);
 }
 
 // Far blocks for an explicit pair list (inspection entry).
@@ -1826,9 +1826,10 @@ const void *pack_rows(hipStream_t s, const Space &X, const FarArgs &F, DevBuf<ch
 // The rotated double layer's default-rule tiles (12 x 13 points): pair blocks of a group of row
 // tiles with the trial cells that the columns touch (k_pair_blocks), then those tiles gathered
 // from them, group by group.  (All trial cells of the mesh cost columns of a few dofs more than
-// tiles that form their own blocks: 3000 x 60 of 3000 dofs, lossy, 2.6 -> 4.4 ms.)  A group's blocks
-// take at most kPairBlockBytes (a quarter of that, and so on, where memory is short) or what its
-// one row tile needs.
+// tiles that form their own blocks: 9000 x 60 of 9000 dofs 2.2 -> 12.8 ms, with the columns' cells
+// 0.70.)  The blocks take at most kPairBlockBytes, and where memory is short a quarter of that,
+// and so on down to those of one row and one column tile (2.4 MB); the columns are split into groups
+// only where one row tile with all of them is too much.  Groups change no entry's bits.
 constexpr size_t kPairBlockBytes = size_t(2) << 30;
 
 template <typename R>
@@ -1836,22 +1837,23 @@ void pair_block_tiles(Ctx &ctx, TileArgs A, const Space &X, const Space &Y)
 {
     constexpr int DLR = BH_OP_MW_DOUBLELAYER_ROTATED;
     hipStream_t s = ctx.stream;
-    const long long nt = X.ntiles;
-    const TileGroups cols = tile_groups(Y.h_tptr, Y.h_tcells, Y.mesh->nf, 1, LLONG_MAX);   // one group
-    const size_t per_cell = (size_t)cols.most * 9 * sizeof(cx<R>);
-    TileGroups rows;
+    PairGroups groups;
     PoolBuf<char> blk;
-    for (size_t budget = kPairBlockBytes;; budget /= 4) {
-        rows = tile_groups(X.h_tptr, X.h_tcells, X.mesh->nf, 64,
-                           per_cell ? (long long)(budget / per_cell) : LLONG_MAX);
+    const auto plan = [&](size_t budget) {
+        return pair_groups(X.h_tptr, X.h_tcells, X.mesh->nf, Y.h_tptr, Y.h_tcells, Y.mesh->nf, 9 * sizeof(cx<R>), budget);
+    };
+    const auto alloc = [&](size_t bytes) {
         try {
-            blk.alloc(ctx, (size_t)rows.most * per_cell);
-            break;
+            blk.alloc(ctx, bytes);
         } catch (const Error &e) {
-            if (e.code != BH_ERR_OOM || (long long)rows.groups.size() == nt) throw;
+            if (e.code != BH_ERR_OOM) throw;
             (void)hipGetLastError();
+            return false;
         }
-    }
+        return true;
+    };
+    if (!shrink_to_fit(groups, kPairBlockBytes, plan, alloc)) throw Error{BH_ERR_OOM};   // alloc's message
+    const TileGroups &rows = groups.rows, &cols = groups.cols;
     std::vector<int> lists;
     for (const std::vector<int> &v : {std::cref(rows.cells), std::cref(cols.cells), std::cref(rows.loc), std::cref(cols.loc)})
         lists.insert(lists.end(), v.begin(), v.end());
@@ -1859,31 +1861,32 @@ void pair_block_tiles(Ctx &ctx, TileArgs A, const Space &X, const Space &Y)
     dlists.upload(lists.data(), lists.size(), s);
     const int *drows = dlists.p, *dcols = drows + rows.cells.size();
     const long long npp = rows.most;
-    const int ncols = (int)cols.most;
-    A.pblk = blk.p;
+    cx<R> *w = (cx<R> *)blk.p;
+    A.pblk = w;
     A.rloc = dcols + cols.cells.size();
     A.cloc = A.rloc + rows.loc.size();
     A.npp = npp;
-    A.ncols = ncols;
     const int shift = sizeof(R) == 8 ? A.far.shifted : 0;
     constexpr int kL1 = sizeof(R) == 8 ? 1 : 0;
-    for (const TileGroup &g : rows.groups) {
-        const dim3 bg((unsigned)((ncols + 3) / 4), (unsigned)((g.n + 63) / 64));
-        const int *gr = drows + g.c0, *gq = dcols;
-        cx<R> *w = (cx<R> *)blk.p;
-        if (g.n == 0 || ncols == 0) {
-            // dofs without shapes: zeros
-        } else if (shift == 1) k_pair_blocks<R, DLR, 12, 13, kL1><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, ncols, w, npp);
-        else if (shift == 2) k_pair_blocks<R, DLR, 12, 13, 2 * kL1><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, ncols, w, npp);
-        else if (shift == 3) k_pair_blocks<R, DLR, 12, 13, 3 * kL1><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, ncols, w, npp);
-        else k_pair_blocks<R, DLR, 12, 13, 0><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, ncols, w, npp);
-        check_launch("k_pair_blocks");
-        A.tr0 = g.t0;
-        const dim3 tg((unsigned)Y.ntiles, (unsigned)(g.t1 - g.t0));
-        if (A.rowmajor) k_gather_tiles<R, true><<<tg, 256, 0, s>>>(A);
-        else k_gather_tiles<R, false><<<tg, 256, 0, s>>>(A);
-        check_launch("k_gather_tiles");
-    }
+    for (const TileGroup &g : rows.groups)
+        for (const TileGroup &h : cols.groups) {
+            const dim3 bg((unsigned)((h.n + 3) / 4), (unsigned)((g.n + 63) / 64));
+            const int *gr = drows + g.c0, *gq = dcols + h.c0;
+            if (g.n == 0 || h.n == 0) {
+                // dofs without shapes: zeros
+            } else if (shift == 1) k_pair_blocks<R, DLR, 12, 13, kL1><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, h.n, w, npp);
+            else if (shift == 2) k_pair_blocks<R, DLR, 12, 13, 2 * kL1><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, h.n, w, npp);
+            else if (shift == 3) k_pair_blocks<R, DLR, 12, 13, 3 * kL1><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, h.n, w, npp);
+            else k_pair_blocks<R, DLR, 12, 13, 0><<<bg, 256, 0, s>>>(A.far, gr, g.n, gq, h.n, w, npp);
+            check_launch("k_pair_blocks");
+            A.ncols = h.n;
+            A.tr0 = g.t0;
+            A.tc0 = h.t0;
+            const dim3 tg((unsigned)(h.t1 - h.t0), (unsigned)(g.t1 - g.t0));
+            if (A.rowmajor) k_gather_tiles<R, true><<<tg, 256, 0, s>>>(A);
+            else k_gather_tiles<R, false><<<tg, 256, 0, s>>>(A);
+            check_launch("k_gather_tiles");
+        }
     BH_CHECK_HIP(hipStreamSynchronize(s));   // the lists and the blocks go out of scope
     blk.done();
 }

@@ -2,6 +2,8 @@
 #pragma once
 
 #include <algorithm>
+#include <climits>
+#include <cstddef>
 #include <vector>
 
 namespace bh {
@@ -49,6 +51,41 @@ inline TileGroups tile_groups(const std::vector<int> &tptr, const std::vector<in
         r.groups.push_back(g);
     }
     return r;
+}
+
+// The row and column groups of a matrix formed from pair blocks of `entry` bytes: all columns
+// and as many row tiles as fit `budget` bytes of blocks; the columns are split too where one row
+// tile with all of them is too much.  bytes: the blocks of the largest pair of groups, above the
+// budget only where a row tile with a column tile is.
+struct PairGroups {
+    TileGroups rows, cols;
+    size_t bytes = 0;
+};
+
+inline PairGroups pair_groups(const std::vector<int> &rptr, const std::vector<int> &rcells, long long rnf,
+                              const std::vector<int> &cptr, const std::vector<int> &ccells, long long cnf, size_t entry,
+                              size_t budget)
+{
+    constexpr int kRowPad = 64;   // a wave's test cells
+    const long long blocks = (long long)(budget / entry);
+    PairGroups r;
+    r.cols = tile_groups(cptr, ccells, cnf, 1, LLONG_MAX);
+    r.rows = tile_groups(rptr, rcells, rnf, kRowPad, r.cols.most ? blocks / r.cols.most : LLONG_MAX);
+    if (r.rows.most * r.cols.most > blocks) r.cols = tile_groups(cptr, ccells, cnf, 1, blocks / r.rows.most);
+    r.bytes = (size_t)(r.rows.most * r.cols.most) * entry;
+    return r;
+}
+
+// The groups for the largest of budget, budget / 4, .. whose blocks alloc(bytes) has room for
+// (false: none); false if not even the smallest groups do.
+template <typename Plan, typename Alloc>
+bool shrink_to_fit(PairGroups &r, size_t budget, const Plan &plan, const Alloc &alloc)
+{
+    for (;; budget /= 4) {
+        r = plan(budget);
+        if (alloc(r.bytes)) return true;
+        if (r.bytes > budget) return false;   // no smaller groups
+    }
 }
 
 }  // namespace bh

@@ -189,3 +189,17 @@ def test_rotated_columns_of_a_part(bj, precision, tol):
         Zs = bj.assemble(op, X, S, precision=precision)
         assert np.abs(Zs[:, :-2] - Z[:, cols]).max() < tol * np.abs(Z).max()
         assert not Zs[:, -2:].any()
+
+
+def test_pair_blocks_in_column_groups(bj):
+    """n x K whose pair blocks with all columns are too many for one row tile (128 cells with more
+    than 116,508): the columns split into groups, against the same rows in two halves whose cells
+    do without.  The bound is that of the row groups: 1e-14 of the largest entry."""
+    X = bj.raviartthomas(bj.meshsphere(0.5, nv=402))
+    Y = bj.raviartthomas(bj.meshsphere(1.0, nv=58500))
+    rows = np.arange(0, 64 * 18, 18)
+    op = bj.cross(bj.n, bj.Maxwell3D.doublelayer(wavenumber=3.0))
+    Z = bj.assemble(op, X.subset(rows), Y)
+    for half in (slice(0, 32), slice(32, 64)):
+        Zh = bj.assemble(op, X.subset(rows[half]), Y)
+        assert np.abs(Zh - Z[half]).max() < 1e-14 * np.abs(Z).max()
