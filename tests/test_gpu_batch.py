@@ -41,6 +41,21 @@ def test_batch_equals_single_requests(bj):
         assert np.array_equal(xb, xs), op
 
 
+def test_batch_of_rotated_layers(bj):
+    """n x K requests that share pair-block launches: every level of shifted phases and none, a
+    lossy one, two rounds of blocks, one too large to share (4116 cells), one of two dofs."""
+    K, small = bj.Maxwell3D.doublelayer, bj.raviartthomas(bj.meshsphere(1.0, nv=102))
+    mid = [bj.raviartthomas(bj.meshsphere(1.0, nv=1300 + i)) for i in range(3)]     # 1 GB of blocks each
+    reqs = [(bj.cross(bj.n, K(wavenumber=k)), small) for k in (0.3, 1.0, 2.5, 5.0, 12.0)]
+    reqs += [(bj.cross(bj.n, K(gamma=0.5 + 2.0j)), small), (bj.cross(bj.n, K(wavenumber=1.0)), small.subset([3, 77]))]
+    reqs += [(bj.cross(bj.n, K(wavenumber=1.0)), X) for X in mid]
+    reqs += [(bj.cross(bj.n, K(wavenumber=1.0)), bj.raviartthomas(bj.meshsphere(1.0, nv=2060)))]
+    batch = bj.DeviceMatrix.assemble_batch(reqs)
+    for (op, X), M in zip(reqs, batch):
+        assert np.array_equal(M.download(), bj.DeviceMatrix.assemble(op, X).download()), (op, X.numfunctions())
+        assert np.abs(M.download() - bj.assemble(op, X, X)).max() < 1e-14 * np.abs(M.download()).max()
+
+
 def test_batch_of_one_and_errors(bj):
     X = bj.raviartthomas(bj.meshsphere(1.0, nv=200))
     t = bj.Maxwell3D.singlelayer(wavenumber=2.0)
