@@ -11,7 +11,7 @@ CSRC = os.path.join(os.path.dirname(HERE), "beast.jl_amd", "csrc")
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
-@pytest.mark.parametrize("name", ["tournament_sets", "panel_positions", "panel_gate", "pool_sizes", "pool_pressure", "tile_groups", "pair_groups"])
+@pytest.mark.parametrize("name", ["tournament_sets", "panel_positions", "panel_gate", "pool_sizes", "pool_pressure", "tile_groups", "pair_groups", "results"])
 def test_host_program(name, tmp_path):
     exe = str(tmp_path / name)
     # the platform macro: HIP's headers need it from a compiler other than hipcc
