@@ -56,7 +56,14 @@ void download_block(Ctx &ctx, const void *dev, void *host, size_t pitch, size_t 
     }
     HostStage &st = *static_cast<HostStage *>(held.get());
     std::lock_guard<std::mutex> g(st.mu);
-    if (!st.p) BH_CHECK_HIP(hipHostMalloc((void **)&st.p, HostStage::kSlots * HostStage::kPiece, hipHostMallocDefault));
+    constexpr size_t kBytes = HostStage::kSlots * HostStage::kPiece;
+    std::vector<char> pageable;   // where no memory can be pinned: slower, for this call
+    if (!st.p && hipHostMalloc((void **)&st.p, kBytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        st.p = nullptr;
+        pageable.resize(kBytes);
+    }
+    char *const slots = st.p ? st.p : pageable.data();
     for (hipEvent_t &e : st.ev)
         if (!e) BH_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     const int64_t pieces = (int64_t)((total + HostStage::kPiece - 1) / HostStage::kPiece);
@@ -64,7 +71,7 @@ void download_block(Ctx &ctx, const void *dev, void *host, size_t pitch, size_t 
     std::atomic<int> failed{(int)hipSuccess};
     auto work = [&](int slot) {
         hipError_t e = hipSetDevice(ctx.device);
-        char *buf = st.p + (size_t)slot * HostStage::kPiece;
+        char *buf = slots + (size_t)slot * HostStage::kPiece;
         while (e == hipSuccess) {
             const int64_t k = next.fetch_add(1);
             if (k >= pieces) break;

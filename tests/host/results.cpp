@@ -10,6 +10,7 @@
 namespace {
 std::atomic<int> spare{-1};   // allocations that are still granted (-1: all)
 std::atomic<int> copies_left{1 << 30};
+bool pin = true;
 }  // namespace
 
 void *operator new(size_t n)
@@ -24,7 +25,7 @@ void operator delete(void *p) noexcept { std::free(p); }
 void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 extern "C" {
-hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return (*p = std::malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return pin && (*p = std::malloc(n)) ? hipSuccess : hipErrorOutOfMemory; }
 hipError_t hipHostFree(void *p) { return std::free(p), hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return *e = (hipEvent_t)1, hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
@@ -76,6 +77,14 @@ int main()
             for (auto rc : {std::pair<int64_t, int64_t>{1, 1}, {65536, 1}, {65537, 3}, {7, 40000}, {300, 900}, {200000, 2}})
                 if (run<double>(ctx, rc.first, rc.second, pad, add) || run<float>(ctx, rc.first, rc.second, pad, add)) return 1;
         }
+    // no memory to pin, then some
+    {
+        Ctx fresh;
+        pin = false;
+        if (run<double>(fresh, 700, 1000, 5, false) || run<float>(fresh, 700, 1000, 5, true)) return 1;
+        pin = true;
+        if (run<double>(fresh, 700, 1000, 5, true)) return 1;
+    }
     // memory that runs out while the threads are made
     for (int grant = 0; grant < 12; ++grant) {
         std::vector<double> dev(2 * 700000, 2.0), host(dev.size(), 0.0);
