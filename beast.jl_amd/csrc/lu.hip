@@ -31,7 +31,6 @@
 //   update of the current one runs (look-ahead by one block).
 //   k_swap_plan, k_laswp_apply  row interchanges: the sequential swaps replayed
 //                   once on row indices, then each moved row moved once.
-//   k_trsm_unit     32-row unit-lower solve for FP32 U12, column in registers.
 //   k_cgemm         C -= A B on MFMA (v_mfma_{f32,f64}_16x16x4): FP64 updates and
 //                   the FP32 updates inside a block column.
 //   k_cgemm_bf16x3  FP32 trailing update from split-bf16 planes (hi*hi + hi*lo +
@@ -1126,129 +1125,6 @@ __global__ __launch_bounds__(256) void k_laswp_apply(typename CT<T>::t *A, long 
     laswp_apply_body<T>(A, lda, plan, len, c0, c1, c2, c3, blockIdx.x);
 }
 
-// ---------------------------------------------------------------- small triangular solve
-// B (m rows x ncols, m <= 32) := L^{-1} B with L unit lower (m x m), both inside A.
-// One wave per workgroup, lane = column: the column lives in registers (all
-// its loads in flight at once), L in LDS (every read a broadcast).
-template <typename T>
-__global__ __launch_bounds__(64) void k_trsm_unit(typename CT<T>::t *A, long long lda, int lr, int lc, int m, int br,
-                                                  int bc, int ncols)
-{
-    using V = typename CT<T>::t;
-    __shared__ V Ls[kPW][kPW + 1];
-    for (int idx = threadIdx.x; idx < m * m; idx += blockDim.x) {
-        const int i = idx / m, j = idx % m;
-        Ls[i][j] = A[(long long)(lr + i) * lda + lc + j];
-    }
-    const int lane = threadIdx.x;
-    const int col = blockIdx.x * 64 + lane;
-    const bool act = col < ncols;
-    V x[kPW];
-#pragma unroll
-    for (int i = 0; i < kPW; ++i) x[i] = (act && i < m) ? A[(long long)(br + i) * lda + bc + col] : V{0, 0};
-    __syncthreads();
-#pragma unroll
-    for (int i = 1; i < kPW; ++i) {
-        if (i < m) {   // uniform
-            V s = x[i];
-#pragma unroll
-            for (int j = 0; j < i; ++j) s = csubv(s, cmulv(Ls[i][j], x[j]));
-            x[i] = s;
-        }
-    }
-    if (act) {
-#pragma unroll
-        for (int i = 0; i < kPW; ++i)
-            if (i < m) A[(long long)(br + i) * lda + bc + col] = x[i];
-    }
-}
-
-// X := L^-1 X on the rows [k, k + kb) (kb <= kNBInner) of the columns
-// [c0, c0 + ncols), L the unit lower triangle of A[k:k+kb, k:k+kb): the FP32
-// block row in one launch.  Workgroup g keeps columns [c0 + 16 g, + 16) of the
-// rows in LDS and walks the 32-row blocks p: threads 0..15 solve block p with the
-// diagonal tile of L (their column in registers), then every thread holds
-// column c = t % 16 of the solved block in registers and updates its rows
-// below (rows 32 (p + 1) + t / 16 + 16 m), reading the rows of L from L2.
-constexpr int kStripW = 16;
-constexpr int kNBInnerMax = 512;
-constexpr int kBlockRowOneLaunch = 8192;   // widest block row solved by k_blockrow_trsm
-
-__global__ __launch_bounds__(256) void k_blockrow_trsm(float2 *A, long long lda, int k, int kb, int c0, int ncols)
-{
-    __shared__ float2 X[kNBInnerMax][kStripW];
-    __shared__ float2 Lt[kPW][kPW + 1];
-    const int tid = threadIdx.x, c = tid % kStripW, g = tid / kStripW;
-    const int col0 = c0 + (int)blockIdx.x * kStripW;
-    const int w = min(kStripW, c0 + ncols - col0);
-    for (int idx = tid; idx < kb * kStripW; idx += 256) {
-        const int r = idx / kStripW, cc = idx % kStripW;
-        X[r][cc] = cc < w ? A[(long long)(k + r) * lda + col0 + cc] : float2{0, 0};
-    }
-    const int np = (kb + kPW - 1) / kPW;
-    for (int p = 0; p < np; ++p) {
-        const int r0 = p * kPW, pr = min(kPW, kb - r0);
-        for (int idx = tid; idx < kPW * kPW; idx += 256) {
-            const int i = idx / kPW, j = idx % kPW;
-            Lt[i][j] = (i < pr && j < pr) ? A[(long long)(k + r0 + i) * lda + k + r0 + j] : float2{0, 0};
-        }
-        __syncthreads();
-        if (tid < kStripW) {
-            float2 x[kPW];
-#pragma unroll
-            for (int i = 0; i < kPW; ++i) x[i] = X[r0 + i < kb ? r0 + i : 0][tid];
-#pragma unroll
-            for (int i = 1; i < kPW; ++i) {
-                if (i < pr) {   // uniform
-                    float2 acc = x[i];
-#pragma unroll
-                    for (int j = 0; j < i; ++j) acc = csubv(acc, cmulv(Lt[i][j], x[j]));
-                    x[i] = acc;
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < kPW; ++i)
-                if (i < pr) X[r0 + i][tid] = x[i];
-        }
-        __syncthreads();
-        if (r0 + pr < kb) {
-            float2 xp[kPW];   // column c of the solved block
-#pragma unroll
-            for (int j = 0; j < kPW; ++j) xp[j] = j < pr ? X[r0 + j][c] : float2{0, 0};
-            // the rows below in tiles of 32: the tile of L through LDS (coalesced),
-            // thread (c, g) updates rows g and g + 16 of the tile
-            for (int q0 = r0 + pr; q0 < kb; q0 += kPW) {
-                const int qr = min(kPW, kb - q0);
-                __syncthreads();
-                for (int idx = tid; idx < kPW * kPW; idx += 256) {
-                    const int i = idx / kPW, j = idx % kPW;
-                    Lt[i][j] = (i < qr && j < pr) ? A[(long long)(k + q0 + i) * lda + k + r0 + j] : float2{0, 0};
-                }
-                __syncthreads();
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int i = g + 16 * h;
-                    if (i < qr) {
-                        float2 acc = X[q0 + i][c];
-#pragma unroll
-                        for (int j = 0; j < kPW; ++j) {
-                            const float2 l = Lt[i][j];
-                            acc.x = fmaf(-l.x, xp[j].x, fmaf(l.y, xp[j].y, acc.x));
-                            acc.y = fmaf(-l.x, xp[j].y, fmaf(-l.y, xp[j].x, acc.y));
-                        }
-                        X[q0 + i][c] = acc;
-                    }
-                }
-            }
-        }
-        __syncthreads();
-    }
-    for (int idx = tid; idx < kb * kStripW; idx += 256) {
-        const int r = idx / kStripW, cc = idx % kStripW;
-        if (cc < w) A[(long long)(k + r) * lda + col0 + cc] = X[r][cc];
-    }
-}
-
 // ---------------------------------------------------------------- MFMA complex GEMM
 // C[M x N] -= A[M x K] B[K x N], row-major complex, K a multiple of 16.
 // Workgroup: 4 waves in 2 x 2, wave tile (16*TM) x (16*TN) complex.
@@ -2072,48 +1948,40 @@ __device__ __forceinline__ void trinv_body(const float2 *A, long long lda, int n
     if constexpr (LOWER) {
         __shared__ float2 T[kIB / kIB32 - 1][kIB32][kIB32];
         unit_lower_inverse_blocked(S, T);
-        float2 *out = Dinv + (size_t)bid * kIB * kIB;
-        for (int idx = t; idx < kIB * kIB; idx += kIB * kTrinvParts) out[idx] = S[idx];
-        return;
-    }
-    __shared__ float2 red[kTrinvParts][kIB];
-    // part = t / kIB: the waves of a part read whole rows of S (consecutive columns,
-    // no bank conflicts); part p sums the terms k = p mod kTrinvParts of each dot product
-    for (int s = LOWER ? 1 : 0; s < kIB; ++s) {
-        const int i = LOWER ? s : kIB - 1 - s;
-        const int k0 = LOWER ? part : i + 1 + part, k1 = LOWER ? i : kIB;
-        float2 u{0, 0}, w{0, 0};   // two chains, so consecutive terms overlap
-        int k = k0;
-        for (; k + kTrinvParts < k1; k += 2 * kTrinvParts) {
-            const float2 a = S[i * kIB + k], x = S[k * kIB + col];
-            const float2 b = S[i * kIB + k + kTrinvParts], y = S[(k + kTrinvParts) * kIB + col];
-            u.x += a.x * x.x - a.y * x.y;
-            u.y += a.x * x.y + a.y * x.x;
-            w.x += b.x * y.x - b.y * y.y;
-            w.y += b.x * y.y + b.y * y.x;
-        }
-        if (k < k1) {
-            const float2 a = S[i * kIB + k], x = S[k * kIB + col];
-            u.x += a.x * x.x - a.y * x.y;
-            u.y += a.x * x.y + a.y * x.x;
-        }
-        red[part][col] = {u.x + w.x, u.y + w.y};
-        const float2 d = S[i * kIB + i];
-        __syncthreads();
-        if (part == 0) {
-            float2 acc = red[0][col];
+    } else {
+        __shared__ float2 red[kTrinvParts][kIB];
+        // part = t / kIB: the waves of a part read whole rows of S (consecutive columns,
+        // no bank conflicts); part p sums the terms k = p mod kTrinvParts of each dot product
+        for (int i = kIB - 1; i >= 0; --i) {
+            float2 u{0, 0}, w{0, 0};   // two chains, so consecutive terms overlap
+            int k = i + 1 + part;
+            for (; k + kTrinvParts < kIB; k += 2 * kTrinvParts) {
+                const float2 a = S[i * kIB + k], x = S[k * kIB + col];
+                const float2 b = S[i * kIB + k + kTrinvParts], y = S[(k + kTrinvParts) * kIB + col];
+                u.x += a.x * x.x - a.y * x.y;
+                u.y += a.x * x.y + a.y * x.x;
+                w.x += b.x * y.x - b.y * y.y;
+                w.y += b.x * y.y + b.y * y.x;
+            }
+            if (k < kIB) {
+                const float2 a = S[i * kIB + k], x = S[k * kIB + col];
+                u.x += a.x * x.x - a.y * x.y;
+                u.y += a.x * x.y + a.y * x.x;
+            }
+            red[part][col] = {u.x + w.x, u.y + w.y};
+            const float2 d = S[i * kIB + i];
+            __syncthreads();
+            if (part == 0) {
+                float2 acc = red[0][col];
 #pragma unroll
-            for (int p = 1; p < kTrinvParts; ++p) { acc.x += red[p][col].x; acc.y += red[p][col].y; }
-            if (LOWER) {
-                if (col < i) S[i * kIB + col] = {-acc.x, -acc.y};
-            } else {
+                for (int p = 1; p < kTrinvParts; ++p) { acc.x += red[p][col].x; acc.y += red[p][col].y; }
                 const float den = d.x * d.x + d.y * d.y;
                 const float2 inv{d.x / den, -d.y / den};
                 if (col > i) S[i * kIB + col] = {-(acc.x * inv.x - acc.y * inv.y), -(acc.x * inv.y + acc.y * inv.x)};
                 else if (col == i) S[i * kIB + i] = inv;
             }
+            __syncthreads();
         }
-        __syncthreads();
     }
     float2 *out = Dinv + (size_t)bid * kIB * kIB;
     for (int idx = t; idx < kIB * kIB; idx += kIB * kTrinvParts) out[idx] = S[idx];
@@ -2638,18 +2506,13 @@ void laswp(Ctx &ctx, hipStream_t s, typename CT<T>::t *A, long long lda, int k1,
     check("k_laswp_apply");
 }
 
-template <typename T>
-void trsm_unit(hipStream_t s, typename CT<T>::t *A, long long lda, int lr, int m, int br, int bc, int ncols)
+// Rows [r, r + m) (m <= 32) of the columns [bc, bc + ncols) := L^-1 times them, L the unit lower
+// triangle at (r, r).
+void trsm64(hipStream_t s, double2 *A, long long lda, int r, int m, int bc, int ncols)
 {
     if (ncols <= 0 || m <= 0) return;
-    if constexpr (sizeof(T) == 8) {
-        BH_REQUIRE(lr == br, "block row %d solved with the triangle at row %d", br, lr);
-        k_apply64<<<(ncols + 15) / 16, 256, 0, s>>>(A, lda, br, lr, m, nullptr, bc, bc, bc, bc + ncols);
-        check("k_apply64");
-    } else {
-        k_trsm_unit<T><<<(ncols + 63) / 64, 64, 0, s>>>(A, lda, lr, lr, m, br, bc, ncols);
-        check("k_trsm_unit");
-    }
+    k_apply64<<<(ncols + 15) / 16, 256, 0, s>>>(A, lda, r, r, m, nullptr, bc, bc, bc, bc + ncols);
+    check("k_apply64");
 }
 
 // FP64 panel [c, c + pw) of the block column [k, k + kb): the panel, then the row moves and the
@@ -2771,7 +2634,7 @@ void gemm_split(Ctx &ctx, hipStream_t s, float2 *A, long long lda, int ar, int a
 // split-bf16 product through PB's planes).
 template <typename T>
 void block_row_u12(Ctx &ctx, hipStream_t s, LUWork<T> &W, typename CT<T>::t *A, long long lda, int n, int k, int kb,
-                   int c0, int c1, DevBuf<__bf16> *PB = nullptr, bool one_launch = true);
+                   int c0, int c1, DevBuf<__bf16> *PB = nullptr);
 
 // Block column [k, k + kb): its 32-column panels and the updates inside the block.
 template <typename T>
@@ -2833,60 +2696,48 @@ void blockrow_apply_inverse(Ctx &ctx, hipStream_t s, const float2 *E, float2 *A,
 // U12 = L11^-1 A12 for block row [k, k + kb) over the columns [c0, n).
 template <typename T>
 void block_row_u12(Ctx &ctx, hipStream_t s, LUWork<T> &W, typename CT<T>::t *A, long long lda, int n, int k, int kb,
-                   int c0, int c1, DevBuf<__bf16> *PB, bool one_launch)
+                   int c0, int c1, DevBuf<__bf16> *PB)
 {
     if (c1 <= c0) return;
     if constexpr (sizeof(T) == 4) {
         if (kb > kNBInner && PB) {
             // top half, its update of the bottom half (split-bf16 products), bottom half
             const int h = kNBInner;
-            block_row_u12<T>(ctx, s, W, A, lda, n, k, h, c0, c1, nullptr, one_launch);
+            block_row_u12<T>(ctx, s, W, A, lda, n, k, h, c0, c1);
             gemm_split(ctx, s, A, lda, k + h, k, k, c0, k + h, c0, kb - h, c1 - c0, h, W.pa_u12, *PB);
-            block_row_u12<T>(ctx, s, W, A, lda, n, k + h, kb - h, c0, c1, nullptr, one_launch);
+            block_row_u12<T>(ctx, s, W, A, lda, n, k + h, kb - h, c0, c1);
             return;
         }
     }
     if constexpr (sizeof(T) == 4) {
         // FP32 block rows by 128-row blocks: the inverses of L11's diagonal blocks, then
-        // per block one product with I - inv(L_bb) and one K = 128 update below it
-        // (measured faster than the one-launch VALU solve at every width)
-        if (kb % kIB == 0 && kb <= kNBInnerMax) {
-            const int nb = kb / kIB;
-            const bool side = s != ctx.stream;
-            float2 *E = (side ? W.eblk_side : W.eblk).p;
-            int &of = side ? W.eblk_side_of : W.eblk_of;
-            if (of != k) {   // a block row taken in two column ranges reuses its inverses
-                ProfScope prof(ctx, "k_trinv", 4.0 * kIB * (double)kIB * kIB * nb / 3.0, s);   // kIB^3/6 complex MACs per block
-                k_trinv<true><<<nb, kIB * kTrinvParts, 0, s>>>(A + (long long)k * lda + k, lda, kb, E);
-                check("k_trinv");
-                k_inv_to_e<<<(unsigned)(((long long)nb * kIB * kIB + 255) / 256), 256, 0, s>>>(E, nb);
-                check("k_inv_to_e");
-                of = k;
-            }
-            for (int b = 0; b < nb; ++b) {
-                const int r = k + b * kIB;
-                blockrow_apply_inverse(ctx, s, E + (size_t)b * kIB * kIB, A, lda, r, c0, c1);
-                if (b + 1 < nb) gemm<T>(ctx, s, A, lda, r + kIB, r, r, c0, r + kIB, c0, k + kb - (r + kIB), c1 - c0, kIB);
-            }
-            return;
+        // per block one product with I - inv(L_bb) and one K = 128 update below it.  (A block
+        // row is only formed where columns follow the block, which is then a full one.)
+        BH_REQUIRE(kb % kIB == 0 && kb <= kNBInner, "block row of %d rows", kb);
+        const int nb = kb / kIB;
+        const bool side = s != ctx.stream;
+        float2 *E = (side ? W.eblk_side : W.eblk).p;
+        int &of = side ? W.eblk_side_of : W.eblk_of;
+        if (of != k) {   // a block row taken in two column ranges reuses its inverses
+            ProfScope prof(ctx, "k_trinv", 4.0 * kIB * (double)kIB * kIB * nb / 3.0, s);   // kIB^3/6 complex MACs per block
+            k_trinv<true><<<nb, kIB * kTrinvParts, 0, s>>>(A + (long long)k * lda + k, lda, kb, E);
+            check("k_trinv");
+            k_inv_to_e<<<(unsigned)(((long long)nb * kIB * kIB + 255) / 256), 256, 0, s>>>(E, nb);
+            check("k_inv_to_e");
+            of = k;
         }
-        // other depths: narrow block rows in one launch (latency-bound as separate
-        // 32-row steps); wide ones, and block rows that run beside the block-column
-        // chain (the one-launch kernel would take the whole device from it), keep the
-        // MFMA updates below
-        const int ncols = c1 - c0;
-        if (one_launch && kb <= kNBInnerMax && ncols <= kBlockRowOneLaunch) {
-            ProfScope prof(ctx, "k_blockrow_trsm", 4.0 * kb * (double)kb * ncols, s);   // kb^2 / 2 complex MACs per column
-            k_blockrow_trsm<<<(ncols + kStripW - 1) / kStripW, 256, 0, s>>>(A, lda, k, kb, c0, ncols);
-            check("k_blockrow_trsm");
-            return;
+        for (int b = 0; b < nb; ++b) {
+            const int r = k + b * kIB;
+            blockrow_apply_inverse(ctx, s, E + (size_t)b * kIB * kIB, A, lda, r, c0, c1);
+            if (b + 1 < nb) gemm<T>(ctx, s, A, lda, r + kIB, r, r, c0, r + kIB, c0, k + kb - (r + kIB), c1 - c0, kIB);
         }
-    }
-    for (int sp = 0; sp < kb; sp += kPW) {
-        const int pw = std::min(kPW, kb - sp);
-        trsm_unit<T>(s, A, lda, k + sp, pw, k + sp, c0, c1 - c0);
-        if (sp + pw < kb)
-            gemm<T>(ctx, s, A, lda, k + sp + pw, k + sp, k + sp, c0, k + sp + pw, c0, kb - (sp + pw), c1 - c0, pw);
+    } else {
+        for (int sp = 0; sp < kb; sp += kPW) {
+            const int pw = std::min(kPW, kb - sp);
+            trsm64(s, A, lda, k + sp, pw, c0, c1 - c0);
+            if (sp + pw < kb)
+                gemm<T>(ctx, s, A, lda, k + sp + pw, k + sp, k + sp, c0, k + sp + pw, c0, kb - (sp + pw), c1 - c0, pw);
+        }
     }
 }
 
@@ -3007,8 +2858,8 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
         W.plan_side.ensure(4 * kMaxSwaps);
         W.top.ensure((size_t)kPW * kPW);
         W.unext.ensure((size_t)kPW * kPW);
-        W.eblk.ensure((size_t)(kNBInnerMax / kIB) * kIB * kIB);
-        W.eblk_side.ensure((size_t)(kNBInnerMax / kIB) * kIB * kIB);
+        W.eblk.ensure((size_t)(kNBInner / kIB) * kIB * kIB);
+        W.eblk_side.ensure((size_t)(kNBInner / kIB) * kIB * kIB);
     }
     {
         hipStream_t s2 = nullptr;
@@ -3083,7 +2934,7 @@ void lu_factor(Ctx &ctx, typename CT<T>::t *A, long long lda, int n, long long *
             // the rest, concurrently
             if (ahead_first) {
                 swaps(k, kb, 0, k, nk + nkb, n);
-                block_row_u12<T>(ctx, s, W, A, lda, n, k, kb, nk + nkb, n, split ? &PB : nullptr, false);
+                block_row_u12<T>(ctx, s, W, A, lda, n, k, kb, nk + nkb, n, split ? &PB : nullptr);
                 trailing(s, k, kb, nk + nkb, n);
             }
             BH_CHECK_HIP(hipStreamWaitEvent(s, done, 0));
