@@ -152,8 +152,8 @@ struct Ctx {
     std::map<std::string, KernelStat> kstats;
     std::vector<hipEvent_t> event_pool;   // timing events reused across launches
     std::string profile_only;             // when set, only this kernel name is timed
-    // workspace of the FP32 factorisation kept between calls (split planes,
-    // tournament buffers, the block-column stream), so that repeated
+    // workspaces of the factorisations kept between calls (FP32: split planes, tournament
+    // buffers; FP64: candidate slots; the block-column stream), so that repeated
     // factorisations allocate and free nothing
     std::shared_ptr<void> lu_cache;
     // pinned slots that results leave the device through (download_block), allocated with the
@@ -164,9 +164,9 @@ struct Ctx {
     std::atomic<int> refs{0};
     std::atomic<bool> closing{false};
     std::atomic<bool> freed{false};
-    // device buffers of destroyed resident matrices, kept for the next matrix of
-    // a similar size (a repeated assemble-factor-solve allocates nothing); at most
-    // pool_limit bytes are kept, the oldest buffers are freed first
+    // device buffers of destroyed resident matrices and of calls' results and workspaces,
+    // kept for the next use of a similar size (a repeated assemble-factor-solve allocates
+    // nothing); at most pool_limit bytes are kept, the oldest buffers are freed first
     std::mutex pool_mu;
     std::vector<PoolMem> pool;
     size_t pool_bytes = 0;

@@ -113,8 +113,9 @@ int bh_ctx_create(int device, bh_ctx **out);
 int bh_ctx_destroy(bh_ctx *ctx);
 int bh_ctx_synchronize(bh_ctx *ctx);
 /* Buffer pool (no counterpart in the reference): the device buffers of destroyed
- * resident matrices stay with the context for the next matrix of a similar size
- * (at least the size asked for, at most 5/4 of it), so that a repeated
+ * resident matrices, and those that host results and workspaces of assembly, far
+ * fields and solves took for a call, stay with the context for the next use of a
+ * similar size (at least the size asked for, at most 5/4 of it), so that a repeated
  * assemble-factor-solve allocates nothing.  limit_bytes >= 0 sets the most the pool
  * keeps (default 64 GiB; 0 disables it and frees what it holds), a negative value
  * leaves it; *pooled_bytes (may be NULL) receives what the pool holds now.  A
@@ -251,9 +252,11 @@ int bh_matrix_download(bh_matrix *M, double *A, int64_t ld);
  * lower L).  BH_FP64 factors the FP64 matrix with LAPACK's partial pivoting (the
  * same ipiv as zgetrf).  BH_FP32 / BH_FP32_SPLIT factor a rounded FP32 copy; their
  * panels choose pivot rows by tournament pivoting, so ipiv may differ from
- * zgetrf's.  Calls on one matrix are serialised with its solves.  The FP32
- * factorisation's workspace (about 1 GB at N = 40k) stays allocated in the context
- * for the next factorisation until the context is destroyed. */
+ * zgetrf's.  Calls on one matrix are serialised with its solves.  The
+ * factorisation's workspace (FP32: about 1 GB at N = 40k) stays allocated in the context
+ * for the next factorisation until the context is destroyed.  BH_FP64 factorisations of
+ * several contexts or threads run side by side while the workgroups of their longest panels
+ * (256 rows each) fit the device together, two per compute unit; a further one waits. */
 int bh_matrix_factor(bh_matrix *M, int precision);
 /* Several resident matrices (all of ctx) factored in shared launches (no counterpart in the
  * reference, which factors one matrix per `\` or LU call, src/solvers/lusolver.jl:26-34):
