@@ -125,7 +125,7 @@ int bh_ctx_pool(bh_ctx *ctx, int64_t limit_bytes, int64_t *pooled_bytes);
  * launch of the library's kernels is bracketed by HIP events on the context
  * stream; bh_ctx_kernel_stats returns, per kernel name (e.g. "k_cgemm"), the
  * launch count, summed device seconds and the algorithmic work (flops or
- * bytes, see DESIGN) the launches were given.  Enabling clears the counters. */
+ * bytes) the launches were given.  Enabling clears the counters. */
 int bh_ctx_profile(bh_ctx *ctx, int enable);
 int bh_ctx_kernel_stats(bh_ctx *ctx, const char *kernel, int64_t *launches, double *seconds, double *work);
 /* Measurement (no counterpart in the reference): restrict profiling to the
